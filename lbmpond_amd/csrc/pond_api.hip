@@ -229,6 +229,7 @@ pond_status collect_events(pond_ctx* ctx) {
     float ms = 0;
     POND_HIP(ctx, hipEventElapsedTime(&ms, e.a, e.b));
     ms_sum += ms;
+    ctx->timed_steps += e.steps;
     ctx->ev_pool.push_back(e);
   }
   ctx->last_ms = ms_sum;
@@ -239,7 +240,6 @@ pond_status collect_events(pond_ctx* ctx) {
     ctx->last_mlp_ms = mm;
     ctx->mlp_pending = false;
   }
-  ctx->timed_steps += (int64_t)ctx->ev_pending.size();
   ctx->ev_pending.clear();
   return POND_OK;
 }
@@ -681,13 +681,22 @@ pond_status pond_step(pond_ctx* ctx, int nsteps) {
   if (nsteps < 0) return fail(ctx, POND_ERR_INVALID, "pond_step: nsteps < 0");
   pond_status s = collect_events(ctx);
   if (s != POND_OK) return s;
+  // The D1Q5 line step is one launch, so the step kernels of a call follow each other with nothing
+  // between them (without amr): one event pair around all of them instead of one around each.
+  const bool line = !ctx->split && f64_line_step(ctx->p.lattice, ctx->p.interp, ctx->g);
+  const bool one_pair = line && !ctx->p.amr;
+  EventPair e;
   for (int k = 0; k < nsteps; k++) {
-    if (ctx->ev_pool.empty()) {
-      s = collect_events(ctx);
-      if (s != POND_OK) return s;
+    const bool first = k == 0 || !one_pair, last = k == nsteps - 1 || !one_pair;
+    if (first) {
+      if (ctx->ev_pool.empty()) {
+        s = collect_events(ctx);
+        if (s != POND_OK) return s;
+      }
+      e = ctx->ev_pool.back();
+      ctx->ev_pool.pop_back();
+      e.steps = one_pair ? nsteps : 1;
     }
-    EventPair e = ctx->ev_pool.back();
-    ctx->ev_pool.pop_back();
     const int in = ctx->cur, outb = 1 - ctx->cur;
     hipError_t he = hipSuccess;
     if (ctx->split && ctx->p.lattice == POND_D3Q27) {
@@ -707,13 +716,13 @@ pond_status pond_step(pond_ctx* ctx, int nsteps) {
       POND_HIP(ctx, hipEventRecord(ctx->mlp_ev[1], ctx->stream));
       ctx->mlp_pending = true;
     }
-    if (!ctx->split) {
+    if (!ctx->split && !line) {
       he = launch_node_prep(ctx->p.lattice, ctx->f64[in].f, ctx->f64[in].m, ctx->nodeP, ctx->nodeok, ctx->g.n,
                             ctx->g.plane, ctx->stream);
       if (he != hipSuccess) return fail(ctx, POND_ERR_HIP, std::string("node prep kernel: ") + hipGetErrorString(he));
     }
     // the event pair brackets the step kernel alone
-    POND_HIP(ctx, hipEventRecord(e.a, ctx->stream));
+    if (first) POND_HIP(ctx, hipEventRecord(e.a, ctx->stream));
     if (ctx->split) {
       const SplitPtrs pin{ctx->sp[in].f, ctx->sp[in].m, ctx->sp[in].T};
       const SplitPtrs pout{ctx->sp[outb].f, ctx->sp[outb].m, ctx->sp[outb].T};
@@ -727,8 +736,10 @@ pond_status pond_step(pond_ctx* ctx, int nsteps) {
                            ctx->f64[outb].f, ctx->f64[outb].m, ctx->niter, pending_view(ctx), ctx->args, ctx->stream);
     }
     if (he != hipSuccess) return fail(ctx, POND_ERR_HIP, std::string("step kernel launch: ") + hipGetErrorString(he));
-    POND_HIP(ctx, hipEventRecord(e.b, ctx->stream));
-    ctx->ev_pending.push_back(e);
+    if (last) {
+      POND_HIP(ctx, hipEventRecord(e.b, ctx->stream));
+      ctx->ev_pending.push_back(e);
+    }
     if (ctx->p.amr) {
       he = launch_amr(ctx->f64[outb], ctx->f64[in], ctx->cell_set, ctx->cell_setnew, ctx->g, ctx->Qn, ctx->stream);
       if (he != hipSuccess) return fail(ctx, POND_ERR_HIP, std::string("amr kernels: ") + hipGetErrorString(he));

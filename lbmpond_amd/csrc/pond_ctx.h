@@ -27,6 +27,7 @@ struct SplitBuf {
 
 struct EventPair {
   hipEvent_t a = nullptr, b = nullptr;
+  int steps = 1;  // step launches between them
 };
 
 // learned gauge initializer: network, training state and dataset
@@ -61,6 +62,9 @@ hipError_t launch_node_prep(int lattice, const double* f, const double* m, doubl
 hipError_t launch_step_f64(int lattice, int interp, const double* fin, const double* min, const double* Pin,
                            const unsigned char* okin, double* fout, double* mout, int* niter, const Pending& pend,
                            const StepArgs& a, hipStream_t st);
+// whether the step of this lattice and grid is the one-launch D1Q5 line kernel, which forms its
+// node data itself (launch_node_prep is not needed)
+bool f64_line_step(int lattice, int interp, const Grid& g);
 // the cell activation passes after a D1Q5 FP64 step (amr.hip): st = the step's output buffer,
 // ld = its input buffer
 hipError_t launch_amr(const F64Buf& st, const F64Buf& ld, int* set, int* setnew, const Grid& g, int qn,

@@ -293,10 +293,11 @@ __device__ __forceinline__ Tgt5 make_tgt5(int inew, double u1x, double T1) {
   const double e1_to = kA5[1] * s1, e2_to = kA5[3] * s1;
   t.et = kA5[inew] * s1;
   const double ef = kA5[inew];
-  double wk;
-  if (ef == 0) wk = 1. / (e1_to * e1_to * e2_to * e2_to);
-  else if (fabs(ef) == kEc1) wk = 1. / (2 * e1_to * e1_to * (e1_to * e1_to - e2_to * e2_to));
-  else wk = 1. / (2 * e2_to * e2_to * (e2_to * e2_to - e1_to * e1_to));
+  // (one division of the selected denominator: the target varies across the lanes of the line step)
+  const double den = ef == 0            ? e1_to * e1_to * e2_to * e2_to
+                     : fabs(ef) == kEc1 ? 2 * e1_to * e1_to * (e1_to * e1_to - e2_to * e2_to)
+                                        : 2 * e2_to * e2_to * (e2_to * e2_to - e1_to * e1_to);
+  const double wk = 1. / den;
   t.wk = wk;
   t.fnew0 = wk * 0.0;
   t.e1sq = e1_to * e1_to;
@@ -307,21 +308,8 @@ __device__ __forceinline__ Tgt5 make_tgt5(int inew, double u1x, double T1) {
   return t;
 }
 
-// MIRX: the node's mirror image in x (Cell::mirrX, structs.cuh:552-559): u0x negated and the
-// populations +e/-e exchanged
-template <bool MIRX = false, class SRC>
-__device__ __forceinline__ double transfer5(const SRC& s, uint32_t boff, const Tgt5& t, bool mx = false) {
-  double u0x = node_m(s, 1, boff);
-  double fm[5];
-  if (MIRX) {
-    if (mx) u0x = -u0x;
-    double f0[5];
-#pragma unroll
-    for (int i = 0; i < 5; i++) f0[i] = node_f(s, i, boff);
-#pragma unroll
-    for (int i = 0; i < 5; i++) fm[i] = mx ? f0[kMir5[i]] : f0[i];
-  }
-  const double s0 = node_P(s, boff);  // sqrts(T0/1.0) = sqrt(|T0|)*sign(T0)
+// transfer of a node with axis velocity u0x, s0 = sqrts(T0/1.0) and populations f to target t
+__device__ __forceinline__ double transfer5v(double u0x, double s0, const double (&f)[5], const Tgt5& t) {
   const double et = t.et;
   const double difu = t.u1x - u0x;
   double fnew = t.fnew0;
@@ -344,10 +332,27 @@ __device__ __forceinline__ double transfer5(const SRC& s, uint32_t boff, const T
     dm4 = dm4 * dm4 * dm4 * dm4;
     dm4 *= 0;
     const double gx = K4 * difu * difu * difu * difu + K3 * difu * difu * difu + K2 * difu * difu + K1 * difu + K0 - dm4;
-    const double fadd = t.wk * gx * (MIRX ? fm[iold] : node_f(s, iold, boff));
+    const double fadd = t.wk * gx * f[iold];
     if (finite_d(fadd)) fnew += fadd;
   }
   return fnew;
+}
+
+// MIRX: the node's mirror image in x (Cell::mirrX, structs.cuh:552-559): u0x negated and the
+// populations +e/-e exchanged
+template <bool MIRX = false, class SRC>
+__device__ __forceinline__ double transfer5(const SRC& s, uint32_t boff, const Tgt5& t, bool mx = false) {
+  double u0x = node_m(s, 1, boff);
+  double f[5];
+#pragma unroll
+  for (int i = 0; i < 5; i++) f[i] = node_f(s, i, boff);
+  if (MIRX && mx) {
+    u0x = -u0x;
+    const double f1 = f[1], f3 = f[3];
+    f[1] = f[2]; f[2] = f1;
+    f[3] = f[4]; f[4] = f3;
+  }
+  return transfer5v(u0x, node_P(s, boff), f, t);  // node_P: sqrts(T0/1.0) = sqrt(|T0|)*sign(T0)
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1424,6 +1429,207 @@ __global__ __launch_bounds__(128) void k_step_q125_f64(const double* __restrict_
 }
 
 // ---------------------------------------------------------------------------------------------
+// D1Q5 lines (Ny = Nz = 1), short ones: 32 lanes per cell, one lane per (target population,
+// stencil node).
+//
+// A short line's step is one cell's serial chain: a few cells on a shock or contact run to the
+// cap of 100 gauge iterations, and with one lane per cell an iteration is ~6000 dependent FP64
+// instructions (36 us), so a step took 3.6 ms whatever the length.  Here the 25 (20 for
+// Lagrange-4) transfers of an iteration run in 25 lanes at once, the three WENO sub-stencils and
+// their weights in three of a target's lanes, and values cross lanes by shuffles; a node's
+// populations stay in registers until the lane's node changes.  Every value is the same sequence
+// of operations as f64_once gives (bit for bit).  sqrt(|T|)*sign(T) of a node is formed here, so
+// the step needs no node-preparation pass and no second pass: it is one launch.  The Sod tube at
+// 2000 cells: 3.5 -> 0.155 ms per step (1.5 us per iteration of the slowest cell, ~1000
+// instructions of a wave that runs alone on its SIMD: the chain, not the chip, bounds it).
+//
+// The y/z factors of the tensor weights: off the line's axis every stencil node is the same cell,
+// and for uy = uz = 0 the departure point lies on it, so exactly one (a, b) term of the nine
+// (sixteen) has weight 1 and the others weight zero.  Adding a zero changes no sum that starts
+// from +0, so those terms are left out where the slice terms are finite (0 * inf is not zero).
+// Above this length the Lagrange-4 line goes back to one lane per cell (below).
+constexpr int64_t kLineCellsLagr4 = 1 << 16;
+
+template <int INTERP>
+__global__ __launch_bounds__(64) void k_step_line(const double* __restrict__ fin, const double* __restrict__ min,
+                                                  double* __restrict__ fout, double* __restrict__ mout,
+                                                  int* __restrict__ niter_out, const StepArgs a) {
+  constexpr bool WENO = INTERP == 0 || INTERP == 4;
+  constexpr int NN = WENO ? 5 : 4;  // stencil nodes along x
+  constexpr int VAR = INTERP == 4 ? 2 : 0;
+  const Grid& g = a.g;
+  const int64_t P = g.plane;
+  const int lane = threadIdx.x, j = lane & 31;
+  // lanes past the last (target, node) pair repeat the last target's (they store nothing)
+  const int t = j / NN < 4 ? j / NN : 4, nd = j % NN;
+  const int base = (lane & 32) + t * NN;  // first lane of the target
+  const int64_t cell0 = (int64_t)blockIdx.x * 2 + (lane >> 5);
+  const int64_t cell = cell0 < g.n ? cell0 : g.n - 1;
+  const int x = (int)cell;
+  // a switched-off cell keeps its record (LBMpull, steps.cu:359)
+  bool active = cell0 < g.n && !(a.cell_set && a.cell_set[cell] == 0);
+  double c0[4] = {min[P + cell], min[2 * P + cell], min[3 * P + cell], min[4 * P + cell]};
+  double rho0 = min[cell];
+  const bool zero = rho0 == 0 && c0[0] == 0 && c0[1] == 0 && c0[2] == 0 && c0[3] == 0;
+  if (zero) { rho0 = 1; c0[3] = a.tlat; }  // steps.cu:360-363
+  double fo = zero ? a.w[t] * 1.0 : fin[t * P + cell];
+  const double ef = kA5[t];
+  int niter = 0;
+  int xc = -1;      // node held in (u0x, s0, f): its wrapped coordinate ...
+  bool mc = false;  // ... and whether it is held as a mirror image
+  double u0x = 0, s0 = 0, f[5] = {0, 0, 0, 0, 0};
+  while (__ballot(active) != 0) {
+    const double s = sqrt(c0[3] / a.tlat);
+    const Tgt5 tg = make_tgt5(t, c0[0], c0[3]);
+    const double cx = (double)x - (s * ef + c0[0]);
+    const int r = WENO ? floor_int(cx + 0.5) - 2 : floor_int(cx) - 4 / 2 + 1;  // first node
+    bool mx = false;
+    const int xn = INTERP == 3 ? mirror_wrap(r + nd, g.nx, (g.mirror & 1) != 0, mx) : wrapi(r + nd, g.nx);
+    if (xn != xc || mx != mc) {
+      xc = xn;
+      mc = mx;
+      u0x = min[P + xn];
+      s0 = sqrts_d(min[4 * P + xn]);
+      double v[5];
+#pragma unroll
+      for (int i = 0; i < 5; i++) v[i] = fin[i * P + xn];
+#pragma unroll
+      for (int i = 0; i < 5; i++) f[i] = INTERP == 3 && mx ? v[kMir5[i]] : v[i];
+      if (INTERP == 3 && mx) u0x = -u0x;
+    }
+    const double V = transfer5v(u0x, s0, f, tg);
+    const double cy = 0.0 - (s * 0.0 + c0[1]), cz = 0.0 - (s * 0.0 + c0[2]);
+    const bool on_line = c0[1] == 0 && c0[2] == 0;
+    double fn;
+    if constexpr (WENO) {
+      // lane q = 0, 1, 2 of the target: sub-stencil q (nodes q .. q+2), its sum and weight
+      const int q = nd < 2 ? nd : 2;
+      const double U[3] = {__shfl(V, base + q, 64), __shfl(V, base + q + 1, 64), __shfl(V, base + q + 2, 64)};
+      double Fx[3][2];
+      lag3_factors(cx - (r + q), Fx);
+      double p[3], S = 0;
+      bool plain = on_line;
+#pragma unroll
+      for (int i = 0; i < 3; i++) {
+        p[i] = 1 * Fx[i][0] * Fx[i][1];
+        const double v = p[i] * U[i];
+        plain = plain && finite_d(v);
+        S += v;
+      }
+      if (!plain) {
+        double Fy[3][2], Fz[3][2];
+        lag3_factors(cy - floor_int(cy + 0.5), Fy);
+        lag3_factors(cz - floor_int(cz + 0.5), Fz);
+        S = 0;
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+          for (int b = 0; b < 3; b++)
+#pragma unroll
+            for (int c = 0; c < 3; c++) S += p[i] * Fy[b][0] * Fy[b][1] * Fz[c][0] * Fz[c][1] * U[i];
+      }
+      // weno5_combine_f64's weight of this sub-stencil: its three indicators are one expression
+      // with other coefficients
+      const double cd = cx - (r + 2);
+      const double dl = (cd * cd - 3 * cd + 2) / 12., dr = (cd * cd + 3 * cd + 2) / 12.;
+      const double dm = VAR == 2 ? 1. - dr - dl : 1. - dl - dr;
+      const double dq = q == 0 ? dl : q == 1 ? dm : dr;
+      double beta;
+      if (VAR == 2) {
+        const double kx = q == 2 ? 10 : 4, ky = q == 2 ? 31 : q == 1 ? 13 : 19, kz = q == 1 ? 13 : 25,
+                     kw = q == 1 ? 5 : 11, ku = q == 2 ? 19 : q == 1 ? 13 : 31, kv = q == 0 ? 10 : 4;
+        beta = (kx * U[0] * U[0] - ky * U[0] * U[1] + kz * U[1] * U[1] + kw * U[0] * U[2] - ku * U[1] * U[2] +
+                kv * U[2] * U[2]) / 3.0;
+      } else {
+        const double kx = q == 0 ? 10 : 4, ky = q == 1 ? 5 : 11, kz = q == 0 ? 31 : q == 1 ? 13 : 19,
+                     kw = q == 1 ? 13 : 25, ku = q == 0 ? 19 : q == 1 ? 13 : 31, kv = q == 2 ? 10 : 4;
+        beta = (kx * U[2] * U[2] + (ky * U[0] - kz * U[1]) * U[2] + kw * U[1] * U[1] - ku * U[0] * U[1] +
+                kv * U[0] * U[0]) / 3.0;
+      }
+      const double w = dq / ((1e-6 + beta) * (1e-6 + beta));
+      const double w0 = __shfl(w, base, 64), w1 = __shfl(w, base + 1, 64), w2 = __shfl(w, base + 2, 64);
+      const double wsum = VAR == 2 ? w2 + w1 + w0 : w0 + w1 + w2;
+      const double ws = w / wsum * S;
+      const double t0 = __shfl(ws, base, 64), t1 = __shfl(ws, base + 1, 64), t2 = __shfl(ws, base + 2, 64);
+      fn = VAR == 2 ? t2 + t1 + t0 : t0 + t1 + t2;
+    } else {
+      double Fx[4][3];
+      lag4_factors(cx - r, Fx);
+      double p[4], U[4];
+      fn = 0;
+      bool plain = on_line;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        U[i] = __shfl(V, base + i, 64);
+        p[i] = 1 * Fx[i][0] * Fx[i][1] * Fx[i][2];
+        const double v = p[i] * U[i];
+        plain = plain && finite_d(v);
+        fn += v;
+      }
+      if (!plain) {
+        double Fy[4][3], Fz[4][3];
+        lag4_factors(cy - (floor_int(cy) - 4 / 2 + 1), Fy);
+        lag4_factors(cz - (floor_int(cz) - 4 / 2 + 1), Fz);
+        fn = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+          for (int b = 0; b < 4; b++)
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+              fn += p[i] * Fy[b][0] * Fy[b][1] * Fy[b][2] * Fz[c][0] * Fz[c][1] * Fz[c][2] * U[i];
+      }
+    }
+    // Cell::calcMoments in population order, in every lane
+    double rho = 0, m0 = 0, m1 = 0, m2 = 0, m3 = 0;
+    const double vy = s * 0.0 + c0[1], vz = s * 0.0 + c0[2];
+#pragma unroll
+    for (int i = 0; i < 5; i++) {
+      const double fi = __shfl(fn, (lane & 32) + i * NN, 64);
+      const double vx = s * kA5[i] + c0[0];
+      rho += fi;
+      m0 += fi * vx;
+      m1 += fi * vy;
+      m2 += fi * vz;
+      m3 += fi * (vx * vx + vy * vy + vz * vz);
+    }
+    if (rho != 0) { m0 /= rho; m1 /= rho; m2 /= rho; m3 /= rho; }
+    m3 = (m3 - m0 * m0 - m1 * m1 - m2 * m2) * a.inv_dim;
+    if (m3 < 0) m3 = c0[3];
+    const double mn[4] = {m0, m1, m2, m3};
+    bool conv = !(fabs(fn - fo) >= a.tol_abs + a.tol_rel * fabs(fn));
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      if (fabs(mn[k] - c0[k]) >= a.tol_abs + a.tol_rel * fabs(mn[k])) conv = false;
+    const uint64_t bad = __ballot(!conv);
+    if (active) {
+      niter++;
+      rho0 = rho;
+      c0[0] = m0; c0[1] = m1; c0[2] = m2; c0[3] = m3;
+      fo = fn;
+      if ((uint32_t)(bad >> (lane & 32)) == 0 || niter >= a.max_iter) {
+        // BGK towards rho*w_i (steps.cu:557-564) and the cell's outputs
+        active = false;
+        if (nd == 0 && j < 5 * NN) {
+          const double feq = rho0 * a.w[t];
+          double v = fo;
+          v += a.dtau * (feq - v);
+          fout[t * P + cell] = v;
+        }
+        if (j == 0) {
+          mout[cell] = rho0;
+          mout[P + cell] = c0[0];
+          mout[2 * P + cell] = c0[1];
+          mout[3 * P + cell] = c0[2];
+          mout[4 * P + cell] = c0[3];
+          niter_out[cell] = niter;
+        }
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
 // host-side launchers
 
 // per-step node data: sqrt(|T|)*sign(T) and the "populations finite and below 2^200" flag
@@ -1471,6 +1677,15 @@ static void launch_rest(unsigned blocks2, hipStream_t st, const NodeSrc& src, do
                        pend, a);
 }
 
+// The line kernel does 3-4 times the work per cell and iteration of the one-lane kernel (lanes of a
+// target repeat its tail), and pays where the chip is not full or the iteration counts are uneven.
+// WENO5: every line (2^20 cells, the longest: 5.3 -> 1.0 ms on the Sod tube, 3.6 -> 2.9 ms on a
+// smooth wave with 3.65 iterations everywhere).  Lagrange-4 on that wave: 32768 cells 0.120 -> 0.090
+// ms, 131072 cells 0.24 -> 0.35 ms.
+bool f64_line_step(int lattice, int interp, const Grid& g) {
+  return lattice == kD1Q5 && g.ny == 1 && g.nz == 1 && (interp != 1 || g.n <= kLineCellsLagr4);
+}
+
 hipError_t launch_step_f64(int lattice, int interp, const double* fin, const double* min, const double* Pin,
                            const unsigned char* okin, double* fout, double* mout, int* niter, const Pending& pend,
                            const StepArgs& a, hipStream_t st) {
@@ -1478,6 +1693,19 @@ hipError_t launch_step_f64(int lattice, int interp, const double* fin, const dou
     const int64_t blocks = a.g.n;
     hipLaunchKernelGGL(k_step_q125_f64, dim3((unsigned)blocks), dim3(128), 0, st, fin, min, okin, fout, mout, niter,
                        a);
+    return hipGetLastError();
+  }
+  // kernel codes: 0 WENO5 as written, 1 Lagrange-4, 2 WENO5 centred, 3 Lagrange-4 with mirror
+  // boundaries (its own instantiation, so the periodic kernels carry none of the mirror code),
+  // 4 the generic WENO5.  interp is pond_interp (POND_WENO5G = 3).
+  const int code = interp == 3 ? 4 : (interp == 1 && a.g.mirror) ? 3 : interp;
+  if (f64_line_step(lattice, interp, a.g)) {
+    // on a line the centred and as-written WENO5 coincide
+    const dim3 nb((unsigned)((a.g.n + 1) / 2)), nt(64);
+    if (code == 1) hipLaunchKernelGGL(k_step_line<1>, nb, nt, 0, st, fin, min, fout, mout, niter, a);
+    else if (code == 3) hipLaunchKernelGGL(k_step_line<3>, nb, nt, 0, st, fin, min, fout, mout, niter, a);
+    else if (code == 4) hipLaunchKernelGGL(k_step_line<4>, nb, nt, 0, st, fin, min, fout, mout, niter, a);
+    else hipLaunchKernelGGL(k_step_line<0>, nb, nt, 0, st, fin, min, fout, mout, niter, a);
     return hipGetLastError();
   }
   const unsigned blocks = (unsigned)(a.g.ntiles);
@@ -1501,10 +1729,6 @@ hipError_t launch_step_f64(int lattice, int interp, const double* fin, const dou
                        a.refill_chunk);                                                                          \
     launch_rest<L, I, true>(blocks2, st, src, fout, mout, niter, pend, a);                                       \
   } while (0)
-  // kernel codes: 0 WENO5 as written, 1 Lagrange-4, 2 WENO5 centred, 3 Lagrange-4 with mirror
-  // boundaries (its own instantiation, so the periodic kernels carry none of the mirror code),
-  // 4 the generic WENO5.  interp is pond_interp (POND_WENO5G = 3).
-  const int code = interp == 3 ? 4 : (interp == 1 && a.g.mirror) ? 3 : interp;
   if (lattice == kD3Q27 && buf && a.refill_chunk > 0) {
     if (code == 0) POND_LAUNCH_R(kD3Q27, 0);
     else if (code == 1) POND_LAUNCH_R(kD3Q27, 1);
