@@ -1431,16 +1431,28 @@ static unsigned refill_blocks(int64_t nchunks) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// D3Q125 split step: one 128-lane block per cell, lane = target population (PonDstepD3Q125,
-// steps.cu:151-250), the fixed 3x3x3 neighbourhood staged in LDS as FP32.
+// D3Q125 split step: 32 lanes per cell, lane = stencil node (PonDstepD3Q125, steps.cu:151-250: the
+// fixed 3x3x3 neighbourhood, 27 nodes), two cells per wave.
 //
 // Transfer of node n to target k (structs.cuh:396-524): per axis the target's quartic Lagrange
 // basis on the target nodes {0, +-ec1 S1, +-ec2 S1} evaluated at the five source velocities
-// (u0 - u1) + a_j S0, so f_new(k) = sum_jx Lx sum_jy Ly sum_jz Lz f(jx,jy,jz): 155 FMAs instead
-// of 125 four-factor products.  Interpolation on the fixed stencil coord-1..coord+1 with the
-// quadratic Lagrange weights, also sum-factorised.  Moments in the frame of the current gauge
-// (A = sum f, B = sum f xi, C = sum f |xi|^2) are block reductions in FP64; the moment solve,
-// the residual and the stopping rules are those of the D3Q27 split step.
+// (u0 - u1) + a_j S0, so f_new(k) = sum_jx Lx sum_jy Ly sum_jz Lz f(jx,jy,jz).  Interpolation on the
+// fixed stencil coord-1..coord+1 with the quadratic Lagrange weights, also sum-factorised.
+// Moments in the frame of the current gauge (A = sum f, B = sum f xi, C = sum f |xi|^2) are FP64
+// sums; the moment solve, the residual and the stopping rules are those of the D3Q27 split step.
+//
+// A node's transfer to all 125 targets is three contractions of 625 FMAs over its own data, so
+// one lane holds the node's 125 populations in registers and contracts them in place, one axis
+// after the other: no exchange, no barrier, no LDS operand.  Then, one ky slab of 25 targets at a
+// time, the lanes lay their transferred values down in LDS and 25 lanes of the cell sum them over
+// the 27 nodes with the interpolation weights of their target.  With a lane per target instead
+// (128 lanes per cell, the contractions through LDS, two barriers per node) the step was bound by
+// its 30 LDS reads for every 15 FMAs: 96^3 turbulence 26.0 -> 7.7 ms per step, 160^3 122 -> 36 ms.
+// Bound now by VALU issue (72 % of the cycles, 3350 instructions per iteration of a wave, 1875 of
+// them the contractions); the texture-address unit is 46 % busy.
+//
+// A wave owns `chunk` consecutive cells; a half whose cell is done takes the next one, so cells
+// that need more iterations hold up nobody but themselves.
 constexpr double kA5d[5] = {0.0, kEc1, -kEc1, kEc2, -kEc2};
 
 // target node m of one axis, {0, +e1, -e1, +e2, -e2}[m], as selects (m varies per lane)
@@ -1448,238 +1460,366 @@ __device__ __forceinline__ double node5(int m, double e1, double e2) {
   return m == 0 ? 0.0 : m == 1 ? e1 : m == 2 ? -e1 : m == 3 ? e2 : -e2;
 }
 
-__device__ __forceinline__ double block_sum128(double v, double* red, int slot) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  if ((threadIdx.x & 63) == 0) red[2 * slot + (threadIdx.x >> 6)] = v;
-  __syncthreads();
-  const double r = red[2 * slot] + red[2 * slot + 1];
-  return r;
+// orders this wave's LDS writes before its following reads and its reads before following writes
+// (a wave's LDS operations execute in order; this holds the compiler to it)
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__global__ __launch_bounds__(128) void k_step_split125(const float* __restrict__ fin, const float* __restrict__ min,
-                                                       const double* __restrict__ Tin, float* __restrict__ fout,
-                                                       float* __restrict__ mout, double* __restrict__ Tout,
-                                                       int* __restrict__ niter_out, const float* __restrict__ guess,
-                                                       const SplitArgs a) {
-  constexpr int Q = 125;
-  __shared__ float sf[27][Q];   // neighbourhood populations
-  __shared__ float su[27][3];   // neighbourhood gauge velocities
-  __shared__ float ss0[27];     // neighbourhood sqrt(|T|)*sign(T)
-  __shared__ double red[10];    // per-wave partial sums of the five moments
-  __shared__ float sL[2][3][5][5];  // a node's basis values L[d][target index][source index], by node parity
-  __shared__ float sTz[Q], sTy[Q];  // a node's z sums and y sums
+// v of the lane a DPP control takes it from (a cross-lane move in the VALU, no LDS round trip)
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xf, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// sum of v over the 32 lanes of each half of the wave, in every lane, added pairwise at distances
+// 16, 8, 4, 2, 1 (after the first two additions the values repeat with period 8, so a rotation by
+// 4 within the row pairs the lanes at distance 4)
+__device__ __forceinline__ double half_sum(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  // each row of 16 lanes and its neighbour row, side by side in both
+  const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)u, (uint32_t)u, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)(u >> 32), (uint32_t)(u >> 32), false, false);
+  v = __builtin_bit_cast(double, ((uint64_t)hi[0] << 32) | lo[0]) +
+      __builtin_bit_cast(double, ((uint64_t)hi[1] << 32) | lo[1]);
+  v += dpp_d<0x128>(v);  // row_ror:8
+  v += dpp_d<0x124>(v);  // row_ror:4
+  v += dpp_d<0x4e>(v);   // quad_perm [2, 3, 0, 1]
+  v += dpp_d<0xb1>(v);   // quad_perm [1, 0, 3, 2]
+  return v;
+}
+
+// one axis' basis values L[target class][source class] of a node: du = u0 - u1 in the axis,
+// s0 its sqrt(|T|)*sign(T), target nodes {0, +-e1, +-e2} and factors bw
+__device__ __forceinline__ void basis125(float du, float s0, float e1, float e2, const float (&bw)[5],
+                                         float (&L)[5][5]) {
+#pragma unroll
+  for (int jj = 0; jj < 5; jj++) {
+    const float bv = du + (float)kA5d[jj] * s0;
+    const float D0 = bv, D1 = bv - e1, D2 = bv + e1, D3 = bv - e2, D4 = bv + e2;
+    const float D01 = D0 * D1, D012 = D01 * D2;
+    L[0][jj] = bw[0] * (((D1 * D2) * D3) * D4);
+    L[1][jj] = bw[1] * (((D0 * D2) * D3) * D4);
+    L[2][jj] = bw[2] * ((D01 * D3) * D4);
+    L[3][jj] = bw[3] * (D012 * D4);
+    L[4][jj] = bw[4] * (D012 * D3);
+  }
+}
+
+// five values at distance `st` in f contracted with L in place (one axis of a node's populations)
+template <int ST>
+__device__ __forceinline__ void contract125(float* f, const float (&L)[5][5]) {
+  float o[5];
+#pragma unroll
+  for (int k = 0; k < 5; k++) {
+    float t = 0.f;
+#pragma unroll
+    for (int jj = 0; jj < 5; jj++) t = __builtin_fmaf(L[k][jj], f[jj * ST], t);
+    o[k] = t;
+  }
+#pragma unroll
+  for (int k = 0; k < 5; k++) f[k * ST] = o[k];
+}
+
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_step_split125(
+    const float* __restrict__ fin, const float* __restrict__ min, const double* __restrict__ Tin,
+    float* __restrict__ fout, float* __restrict__ mout, double* __restrict__ Tout, int* __restrict__ niter_out,
+    const float* __restrict__ guess, const SplitArgs a, int chunk) {
+  constexpr int Q = 125, NSTR = 28, CSTR = 27 * NSTR + 44;  // strides that spread the banks
+  __shared__ __align__(16) float st[2][CSTR];  // a ky slab: [cell half][node][5 kx + kz]
+  __shared__ __align__(16) float sfn[2][128];  // the iterate, by population
+  __shared__ __align__(16) double sxi[128][4]; // xi_x, xi_y, xi_z, |xi|^2 of each population
+  __shared__ __align__(16) float sw[128];
   const Grid& g = a.g;
   const int64_t P = g.plane;
-  const int64_t cell = xcd_block(blockIdx.x, gridDim.x);
-  const int k = threadIdx.x;
-  const bool lane_ok = k < Q;
-  const int x = (int)(cell % g.nx);
-  const int y = (int)((cell / g.nx) % g.ny);
-  const int z = (int)(cell / ((int64_t)g.nx * g.ny));
-  for (int n = 0; n < 27; n++) {
-    // mirror boundaries (steps.cu:163-190): a node beyond a mirrored face is the mirror image of
-    // the cell inside, population k read from the mirrored velocity, the axis velocity negated
-    bool rx, ry, rz;
-    const int px = mirror_wrap(x - 1 + n / 9, g.nx, (g.mirror & 1) != 0, rx);
-    const int py = mirror_wrap(y - 1 + (n / 3) % 3, g.ny, (g.mirror & 2) != 0, ry);
-    const int pz = mirror_wrap(z - 1 + n % 3, g.nz, (g.mirror & 4) != 0, rz);
-    const int64_t c = cell_index(g, px, py, pz);
-    const int kq = lane_ok ? k : 0;  // lanes 125..127 hold no population
-    const int kx = kq / 25, ky = (kq / 5) % 5, kz = kq % 5;
-    const int kl = 25 * (rx ? kMir5[kx] : kx) + 5 * (ry ? kMir5[ky] : ky) + (rz ? kMir5[kz] : kz);
-    // non-finite data as in k_node_gauge (the reference drops non-finite transfer terms,
-    // structs.cuh:516): a non-finite population stages as zero, a node with a non-finite gauge
-    // as all zeros with a zero gauge
-    const float ux = rx ? -min[P + c] : min[P + c], uy = ry ? -min[2 * P + c] : min[2 * P + c],
-                uz = rz ? -min[3 * P + c] : min[3 * P + c];
-    const double t = Tin[c];
-    const float s0 = (float)(sqrt(fabs(t)) * (double)((0.0 < t) - (t < 0.0)));
-    const bool gok = isfinite(ux) && isfinite(uy) && isfinite(uz) && isfinite(s0);
-    if (lane_ok) {
-      const float v = fin[c * kSplit125Floats + kl];
-      sf[n][k] = gok && isfinite(v) ? v : 0.0f;
-    }
-    if (k < 3) su[n][k] = gok ? (k == 0 ? ux : k == 1 ? uy : uz) : 0.0f;
-    if (k == 3) ss0[n] = gok ? s0 : 0.0f;
+  const int lane = threadIdx.x, h = lane >> 5, j = lane & 31;
+  const int n = j < 27 ? j : 26;  // lanes 27..31 repeat node 26 (they store nothing)
+  for (int k = lane; k < 128; k += 64) {
+    const double xv = k < Q ? kA5d[k / 25] : 0.0, yv = k < Q ? kA5d[(k / 5) % 5] : 0.0, zv = k < Q ? kA5d[k % 5] : 0.0;
+    sxi[k][0] = xv;
+    sxi[k][1] = yv;
+    sxi[k][2] = zv;
+    sxi[k][3] = xv * xv + yv * yv + zv * zv;
+    sw[k] = k < Q ? a.w[k] : 0.f;
+    sfn[0][k] = sfn[1][k] = 0.f;
   }
-  double rho0 = min[cell];
-  double gp[4] = {min[P + cell], min[2 * P + cell], min[3 * P + cell], Tin[cell]};
-  if (rho0 == 0 && gp[0] == 0 && gp[1] == 0 && gp[2] == 0 && gp[3] == 0) { rho0 = 1; gp[3] = a.tlat; }
-  double gc[4] = {gp[0], gp[1], gp[2], gp[3]};
-  bool learned = false;
-  if (guess) {
-    const double st = sqrt(gp[3]);
-    const double q[4] = {gp[0] + st * guess[cell], gp[1] + st * guess[P + cell], gp[2] + st * guess[2 * P + cell],
-                         gp[3] * (1.0 + (double)guess[3 * P + cell])};
-    const float pmax = fmaxf(fmaxf(fabsf(guess[cell]), fabsf(guess[P + cell])),
-                             fmaxf(fabsf(guess[2 * P + cell]), fabsf(guess[3 * P + cell])));
-    if (isfinite(q[0]) && isfinite(q[1]) && isfinite(q[2]) && isfinite(q[3]) && q[3] > 0 && pmax <= a.learned_trust &&
-        pmax > 0.0f && niter_out[cell] >= kLearnedPrevMin && niter_out[cell] <= kLearnedPrevMax) {
-      for (int d = 0; d < 4; d++) gc[d] = q[d];
-      learned = true;
-    }
-  }
-  __syncthreads();
-  const int kk = lane_ok ? k : 0;
-  const int X[3] = {kk / 25, (kk / 5) % 5, kk % 5};
-  const double xa[3] = {node5(X[0], kEc1, kEc2), node5(X[1], kEc1, kEc2), node5(X[2], kEc1, kEc2)};
-  const double xi2 = xa[0] * xa[0] + xa[1] * xa[1] + xa[2] * xa[2];
+  wave_lds_order();
+  const int64_t c_first = xcd_block(blockIdx.x, gridDim.x) * chunk;
+  const int total = (int)(g.n - c_first < chunk ? g.n - c_first : chunk);
+  int next = 0;
+  // target of this lane in a ky slab (lanes 25..31 repeat one)
+  const int kx = j < 25 ? j / 5 : 4, kz = j % 5;
+  const double xax = node5(kx, kEc1, kEc2), xaz = node5(kz, kEc1, kEc2);
+  bool active = false, dirty = false, fresh = false;
+  int64_t cell = c_first;
+  int x = 0, y = 0, z = 0;
+  bool rx = false, ry = false, rz = false;
+  int64_t rec = 0;                              // the node's populations: index of its record ...
+  float nux = 0, nuy = 0, nuz = 0, ns0 = 0;     // ... and gauge
+  bool gok = true;
+  double gc[4] = {0, 0, 0, 1}, res_prev = 0, rho = 0;
   int niter = 0, base = 0;  // base: iterations spent on an abandoned predicted start
-  bool contracted = false;   // a residual has fallen since the current start
-  double res_prev = 0, rho = rho0;
-  float fn = 0.f;
-  while (niter - base < a.max_iter) {
-    niter++;
+  bool learned = false, contracted = false;  // contracted: a residual has fallen since the current start
+  auto prev_gauge = [&](double gp[4], double& rho0) {
+    rho0 = min[cell];
+    gp[0] = min[P + cell]; gp[1] = min[2 * P + cell]; gp[2] = min[3 * P + cell]; gp[3] = Tin[cell];
+    if (rho0 == 0 && gp[0] == 0 && gp[1] == 0 && gp[2] == 0 && gp[3] == 0) { rho0 = 1; gp[3] = a.tlat; }
+  };
+  while (true) {
+    const uint64_t want = __ballot(!active);
+    if (!active) {
+      const int slot = next + (h && (want & 1) ? 1 : 0);
+      if (slot < total) {
+        active = fresh = true;
+        cell = c_first + slot;
+        x = (int)(cell % g.nx);
+        y = (int)((cell / g.nx) % g.ny);
+        z = (int)(cell / ((int64_t)g.nx * g.ny));
+        // mirror boundaries (steps.cu:163-190): a node beyond a mirrored face is the mirror image of
+        // the cell inside, population k read from the mirrored velocity, the axis velocity negated
+        const int px = mirror_wrap(x - 1 + n / 9, g.nx, (g.mirror & 1) != 0, rx);
+        const int py = mirror_wrap(y - 1 + (n / 3) % 3, g.ny, (g.mirror & 2) != 0, ry);
+        const int pz = mirror_wrap(z - 1 + n % 3, g.nz, (g.mirror & 4) != 0, rz);
+        const int64_t c = cell_index(g, px, py, pz);
+        rec = c * kSplit125Floats;
+        nux = rx ? -min[P + c] : min[P + c];
+        nuy = ry ? -min[2 * P + c] : min[2 * P + c];
+        nuz = rz ? -min[3 * P + c] : min[3 * P + c];
+        const double t = Tin[c];
+        ns0 = (float)(sqrt(fabs(t)) * (double)((0.0 < t) - (t < 0.0)));
+        // non-finite data as in k_node_gauge (the reference drops non-finite transfer terms,
+        // structs.cuh:516): a non-finite population counts as zero, a node with a non-finite gauge
+        // as all zeros with a zero gauge
+        gok = isfinite(nux) && isfinite(nuy) && isfinite(nuz) && isfinite(ns0);
+        if (!gok) nux = nuy = nuz = ns0 = 0.f;
+        double gp[4], rho0;
+        prev_gauge(gp, rho0);
+        for (int d = 0; d < 4; d++) gc[d] = gp[d];
+        learned = contracted = false;
+        niter = base = 0;
+        res_prev = 0;
+        rho = rho0;
+        if (guess) {
+          const double sq = sqrt(gp[3]);
+          const float p0 = guess[cell], p1 = guess[P + cell], p2 = guess[2 * P + cell], p3 = guess[3 * P + cell];
+          const double q[4] = {gp[0] + sq * p0, gp[1] + sq * p1, gp[2] + sq * p2, gp[3] * (1.0 + (double)p3)};
+          const float pmax = fmaxf(fmaxf(fabsf(p0), fabsf(p1)), fmaxf(fabsf(p2), fabsf(p3)));
+          if (isfinite(q[0]) && isfinite(q[1]) && isfinite(q[2]) && isfinite(q[3]) && q[3] > 0 &&
+              pmax <= a.learned_trust && pmax > 0.0f && niter_out[cell] >= kLearnedPrevMin &&
+              niter_out[cell] <= kLearnedPrevMax) {
+            for (int d = 0; d < 4; d++) gc[d] = q[d];
+            learned = true;
+          }
+        }
+      }
+    }
+    next += ((want & 1) ? 1 : 0) + ((want >> 32 & 1) ? 1 : 0);
+    if (__ballot(active) == 0) break;
+
+    // the node's populations (read again in every iteration: kept, they would take the registers of
+    // a second wave; the empty asm keeps the loads from being lifted out of the loop)
+    float f[128];
+    {
+      int64_t r = rec;
+      asm volatile("" : "+v"(r));
+#pragma unroll
+      for (int q = 0; q < 32; q++) {
+        const float4 v = reinterpret_cast<const float4*>(fin + r)[q];
+        f[4 * q] = v.x; f[4 * q + 1] = v.y; f[4 * q + 2] = v.z; f[4 * q + 3] = v.w;
+      }
+    }
     const double s = sqrt(gc[3] / a.tlat);
     // target basis constants (structs.cuh:397-416)
     const double S1 = sqrt(fabs(gc[3])) * (double)((0.0 < gc[3]) - (gc[3] < 0.0));
     const double e1 = kEc1 * S1, e2 = kEc2 * S1;
-    // departure point on the fixed stencil coord-1..coord+1 (steps.cu:163,207-208)
-    float Fx[3], Fy[3], Fz[3];
+    const float e1f = (float)e1, e2f = (float)e2;
+    float bw[5];
     {
-      const double vx = s * xa[0] + gc[0], vy = s * xa[1] + gc[1], vz = s * xa[2] + gc[2];
-      lag3f((float)(((double)x - vx) - (double)(x - 1)), Fx);
-      lag3f((float)(((double)y - vy) - (double)(y - 1)), Fy);
-      lag3f((float)(((double)z - vz) - (double)(z - 1)), Fz);
-    }
-    const float u1[3] = {(float)gc[0], (float)gc[1], (float)gc[2]};
-    const float u1l[3] = {(float)(gc[0] - (double)u1[0]), (float)(gc[1] - (double)u1[1]), (float)(gc[2] - (double)u1[2])};
-    // Transfer of each node to every target, contracted one axis at a time across the block:
-    // the basis values L[d][kd][j] of the node (75, one per lane), the z sums tz(jx, jy, kz), the
-    // y sums ty(jx, ky, kz), then each target's x sum, every value formed once and read by the
-    // targets that share it.  A target's value is the same sequence of operations as contracting
-    // its own 125 terms (z inner, then y, then x).
-    const int tb = lane_ok ? k : 0;
-    const int bd = tb / 25, bk = (tb / 5) % 5, bj = tb % 5;  // basis entry of lanes 0..74
-    float bw = 0.f, bn[4] = {0.f, 0.f, 0.f, 0.f};
-    {
-      const double xn = node5(bk, e1, e2);
+      // the factor of target class m in lane m of the half
+      const int m = j < 5 ? j : 4;
+      const double xn = node5(m, e1, e2);
       double den = 1.0;
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const double v = node5(q < bk ? q : q + 1, e1, e2);
-        den *= xn - v;
-        bn[q] = (float)v;
-      }
-      bw = (float)(1.0 / den);
+      for (int q = 0; q < 4; q++) den *= xn - node5(q < m ? q : q + 1, e1, e2);
+      const float b = (float)(1.0 / den);
+#pragma unroll
+      for (int k = 0; k < 5; k++) bw[k] = __shfl(b, (lane & 32) + k, 64);
     }
-    float acc = 0.f, accy = 0.f, accz = 0.f;
-    // basis values of node n (lanes 0..74) into sL[n & 1]
-    auto basis = [&](int n) {
-      if (k < 75) {
-        const float du = (su[n][bd] - u1[bd]) - u1l[bd];
-        const float bv = du + (float)kA5d[bj] * ss0[n];
-        sL[n & 1][bd][bk][bj] = bw * ((bv - bn[0]) * (bv - bn[1]) * (bv - bn[2]) * (bv - bn[3]));
-      }
-    };
-    // z sums of node n: tz(jx, jy, kz) at index 25 jx + 5 jy + kz
-    auto zsums = [&](int n) {
-      if (lane_ok) {
-        float tz = 0.f;
+    if (__ballot(fresh) != 0) {
+      // 0 * v is NaN for a non-finite v
+      float zz[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int jz = 0; jz < 5; jz++) tz = __builtin_fmaf(sL[n & 1][2][bj][jz], sf[n][25 * bd + 5 * bk + jz], tz);
-        sTz[k] = tz;
-      }
-    };
-    // The three phases of consecutive nodes overlap, two barriers per node: the y sums of node
-    // n with the basis values of node n + 1 (the other sL slot), then the x sums of node n with
-    // the z sums of node n + 1 (sTz, whose node-n values the y sums have read).  Each value is
-    // the same sequence of operations as with the phases of one node at a time.
-    basis(0);
-    __syncthreads();
-    zsums(0);
-    __syncthreads();
-#pragma unroll 1
-    for (int n = 0; n < 27; n++) {
-      const int pb = n & 1;
-      if (lane_ok) {  // ty(jx, ky, kz) at index 25 jx + 5 ky + kz
-        float ty = 0.f;
+      for (int q = 0; q < Q; q++) zz[q % 5] = __builtin_fmaf(f[q], 0.f, zz[q % 5]);
+      const float zs = ((zz[0] + zz[1]) + (zz[2] + zz[3])) + zz[4];
+      if (fresh) dirty = !gok || zs != zs;
+      fresh = false;
+    }
+    if (__ballot(dirty) != 0) {
 #pragma unroll
-        for (int jy = 0; jy < 5; jy++) ty = __builtin_fmaf(sL[pb][1][bk][jy], sTz[25 * bd + 5 * jy + bj], ty);
-        sTy[k] = ty;
-      }
-      if (n + 1 < 27) basis(n + 1);
-      __syncthreads();
-      float tx = 0.f;
-      if (lane_ok) {
+      for (int q = 0; q < Q; q++) f[q] = gok && isfinite(f[q]) ? f[q] : 0.0f;
+    }
+    if (g.mirror) {
+      auto swap = [](bool m, float& p, float& q) {
+        const float t = p;
+        p = m ? q : p;
+        q = m ? t : q;
+      };
+      if (__ballot(rx) != 0) {
 #pragma unroll
-        for (int jx = 0; jx < 5; jx++) tx = __builtin_fmaf(sL[pb][0][X[0]][jx], sTy[25 * jx + 5 * X[1] + X[2]], tx);
+        for (int q = 0; q < 25; q++) { swap(rx, f[25 + q], f[50 + q]); swap(rx, f[75 + q], f[100 + q]); }
       }
-      if (n + 1 < 27) zsums(n + 1);
-      // (the stencil sums of the fixed 3x3x3 neighbourhood: z inner, then y, then x)
-      const int ia = n / 9, ib = (n / 3) % 3, ic = n % 3;
-      accz = __builtin_fmaf(Fz[ic], tx, accz);
-      if (ic == 2) {
-        accy = __builtin_fmaf(Fy[ib], accz, accy);
-        accz = 0.f;
-        if (ib == 2) {
-          acc = __builtin_fmaf(Fx[ia], accy, acc);
-          accy = 0.f;
+      if (__ballot(ry) != 0) {
+#pragma unroll
+        for (int q = 0; q < 25; q++) {
+          float* p = f + 25 * (q / 5) + q % 5;
+          swap(ry, p[5], p[10]);
+          swap(ry, p[15], p[20]);
         }
       }
-      __syncthreads();
+      if (__ballot(rz) != 0) {
+#pragma unroll
+        for (int q = 0; q < 25; q++) { swap(rz, f[5 * q + 1], f[5 * q + 2]); swap(rz, f[5 * q + 3], f[5 * q + 4]); }
+      }
     }
-    fn = lane_ok ? acc : 0.f;
-    // moments in the frame of the current gauge, FP64 block sums
-    const double fd = (double)fn;
-    const double A = block_sum128(fd, red, 0);
-    const double Bx = block_sum128(fd * xa[0], red, 1);
-    const double By = block_sum128(fd * xa[1], red, 2);
-    const double Bz = block_sum128(fd * xa[2], red, 3);
-    const double C = block_sum128(fd * xi2, red, 4);
-    __syncthreads();  // red is rewritten next iteration
-    rho = A;
-    const double B[3] = {Bx, By, Bz};
-    double m[4];
-    if (rho != 0) {
-      const double ir = 1.0 / rho;
-      for (int d = 0; d < 3; d++) m[d] = gc[d] + s * (B[d] * ir);
-      m[3] = s * s * (C - (B[0] * B[0] + B[1] * B[1] + B[2] * B[2]) * ir) * ir * a.inv_dim;
-    } else {
-      for (int d = 0; d < 3; d++) m[d] = s * B[d];
-      m[3] = (2.0 * s * (gc[0] * B[0] + gc[1] * B[1] + gc[2] * B[2]) + s * s * C - (m[0] * m[0] + m[1] * m[1] + m[2] * m[2])) *
-             a.inv_dim;
+    const float u1x = (float)gc[0], u1y = (float)gc[1], u1z = (float)gc[2];
+    const float u1xl = (float)(gc[0] - (double)u1x), u1yl = (float)(gc[1] - (double)u1y),
+                u1zl = (float)(gc[2] - (double)u1z);
+    float L[5][5];
+    basis125((nuz - u1z) - u1zl, ns0, e1f, e2f, bw, L);
+#pragma unroll
+    for (int q = 0; q < 25; q++) contract125<1>(f + 5 * q, L);
+    basis125((nuy - u1y) - u1yl, ns0, e1f, e2f, bw, L);
+#pragma unroll
+    for (int q = 0; q < 25; q++) contract125<5>(f + 25 * (q / 5) + q % 5, L);
+    basis125((nux - u1x) - u1xl, ns0, e1f, e2f, bw, L);
+    // departure point on the fixed stencil coord-1..coord+1 (steps.cu:163,207-208)
+    float Fx[3], Fz[3];
+    lag3f((float)(((double)x - (s * xax + gc[0])) - (double)(x - 1)), Fx);
+    lag3f((float)(((double)z - (s * xaz + gc[2])) - (double)(z - 1)), Fz);
+#pragma unroll
+    for (int ky = 0; ky < 5; ky++) {
+#pragma unroll
+      for (int q = 0; q < 5; q++) contract125<25>(f + 5 * ky + q, L);
+      wave_lds_order();  // the previous slab's reads are done
+      if (j < 27) {
+        float* o = &st[h][n * NSTR];
+        float v[28];
+#pragma unroll
+        for (int q = 0; q < 25; q++) v[q] = f[25 * (q / 5) + 5 * ky + q % 5];
+        v[25] = v[26] = v[27] = 0.f;
+#pragma unroll
+        for (int q = 0; q < 7; q++) *reinterpret_cast<float4*>(o + 4 * q) = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+      }
+      wave_lds_order();
+      float Fy[3];
+      lag3f((float)(((double)y - (s * kA5d[ky] + gc[1])) - (double)(y - 1)), Fy);
+      // the stencil sums of the fixed 3x3x3 neighbourhood: z inner, then y, then x
+      const float* t = &st[h][5 * kx + kz];
+      float acc = 0.f;
+#pragma unroll
+      for (int ia = 0; ia < 3; ia++) {
+        float accy = 0.f;
+#pragma unroll
+        for (int ib = 0; ib < 3; ib++) {
+          float accz = 0.f;
+#pragma unroll
+          for (int ic = 0; ic < 3; ic++) accz = __builtin_fmaf(Fz[ic], t[(9 * ia + 3 * ib + ic) * NSTR], accz);
+          accy = __builtin_fmaf(Fy[ib], accz, accy);
+        }
+        acc = __builtin_fmaf(Fx[ia], accy, acc);
+      }
+      if (j < 25) sfn[h][25 * kx + 5 * ky + kz] = acc;
     }
-    if (m[3] < 0) m[3] = gc[3];
-    const double st = sqrt(fabs(m[3]));
-    double res = 0;
-    bool conv = true;
-    for (int d = 0; d < 4; d++) {
-      const double scale = d < 3 ? st : fabs(m[3]);
-      const double dd = fabs(m[d] - gc[d]);
-      if (dd > a.tol_rel * scale + a.tol_abs) conv = false;  // NaN: converged, as in the D3Q27 step
-      const double rk = dd / (scale + 1e-300);
-      if (res == res && !(rk <= res)) res = rk;  // NaN propagates (fmax would drop it)
+    wave_lds_order();
+    // moments in the frame of the current gauge, FP64 sums over the populations: pairs 32 apart, then
+    // the halves' tree, populations 0..63 and 64..127 separately
+    double mom[5];
+    {
+      double lo[5], hi[5];
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        const int k = j + 32 * b;
+        const double fd = (double)sfn[h][k];
+        const double v[5] = {fd, fd * sxi[k][0], fd * sxi[k][1], fd * sxi[k][2], fd * sxi[k][3]};
+#pragma unroll
+        for (int q = 0; q < 5; q++) {
+          if (b == 0) lo[q] = v[q];
+          if (b == 1) lo[q] += v[q];
+          if (b == 2) hi[q] = v[q];
+          if (b == 3) hi[q] += v[q];
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 5; q++) mom[q] = half_sum(lo[q]) + half_sum(hi[q]);
     }
-    if (!conv && niter - base > 1 && res <= 4.0 * a.tol_rel && res >= res_prev && (!learned || contracted)) conv = true;
-    if (niter - base > 1 && res < res_prev) contracted = true;
-    // (unlike the D3Q27 step, no fallback from a predicted start on a NaN residual: with that
-    // rule the 256^3 D3Q125 turbulence took 4.58 mean iterations instead of 2.35, although a
-    // probe counted no NaN residual there; the cause is not found)
-    if (conv) {
-      for (int d = 0; d < 4; d++) gc[d] = m[d];
-      break;
+    bool done = false;
+    if (active) {
+      niter++;
+      rho = mom[0];
+      const double B[3] = {mom[1], mom[2], mom[3]}, C = mom[4];
+      double m[4];
+      if (rho != 0) {
+        const double ir = 1.0 / rho;
+        for (int d = 0; d < 3; d++) m[d] = gc[d] + s * (B[d] * ir);
+        m[3] = s * s * (C - (B[0] * B[0] + B[1] * B[1] + B[2] * B[2]) * ir) * ir * a.inv_dim;
+      } else {
+        for (int d = 0; d < 3; d++) m[d] = s * B[d];
+        m[3] = (2.0 * s * (gc[0] * B[0] + gc[1] * B[1] + gc[2] * B[2]) + s * s * C - (m[0] * m[0] + m[1] * m[1] + m[2] * m[2])) *
+               a.inv_dim;
+      }
+      if (m[3] < 0) m[3] = gc[3];
+      const double sth = sqrt(fabs(m[3]));
+      double res = 0;
+      bool conv = true;
+      for (int d = 0; d < 4; d++) {
+        const double scale = d < 3 ? sth : fabs(m[3]);
+        const double dd = fabs(m[d] - gc[d]);
+        if (dd > a.tol_rel * scale + a.tol_abs) conv = false;  // NaN: converged, as in the D3Q27 step
+        const double rk = dd / (scale + 1e-300);
+        if (res == res && !(rk <= res)) res = rk;  // NaN propagates (fmax would drop it)
+      }
+      if (!conv && niter - base > 1 && res <= 4.0 * a.tol_rel && res >= res_prev && (!learned || contracted)) conv = true;
+      if (niter - base > 1 && res < res_prev) contracted = true;
+      // (unlike the D3Q27 step, no fallback from a predicted start on a NaN residual)
+      if (!conv && learned && ((niter > 1 && !(res < res_prev)) || niter == kLearnedBudget)) {
+        double rho0;
+        prev_gauge(gc, rho0);
+        learned = contracted = false;
+        res_prev = 0;
+        base = niter;
+      } else {
+        res_prev = res;
+        for (int d = 0; d < 4; d++) gc[d] = m[d];
+      }
+      done = conv || niter - base >= a.max_iter;
     }
-    if (learned && ((niter > 1 && !(res < res_prev)) || niter == kLearnedBudget)) {
-      for (int d = 0; d < 4; d++) gc[d] = gp[d];
-      learned = false;
-      contracted = false;
-      res_prev = 0;
-      base = niter;
-      continue;
+    if (done) {
+      // BGK on the iterate, four populations per lane: the cell's record in one store
+      active = false;
+      const float rf = (float)rho, dt = (float)a.dtau;
+      float4 o;
+      float* ov = &o.x;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const float v = sfn[h][4 * j + q];
+        ov[q] = __builtin_fmaf(dt, rf * sw[4 * j + q] - v, v);
+      }
+      reinterpret_cast<float4*>(fout + cell * kSplit125Floats)[j] = o;
+      if (j == 0) {
+        mout[cell] = rf;
+        mout[P + cell] = (float)gc[0];
+        mout[2 * P + cell] = (float)gc[1];
+        mout[3 * P + cell] = (float)gc[2];
+        Tout[cell] = gc[3];
+        niter_out[cell] = niter;
+      }
     }
-    res_prev = res;
-    for (int d = 0; d < 4; d++) gc[d] = m[d];
-  }
-  const float rf = (float)rho;
-  if (lane_ok) fout[cell * kSplit125Floats + k] = __builtin_fmaf((float)a.dtau, rf * a.w[k] - fn, fn);
-  if (k == 0) {
-    mout[cell] = rf;
-    mout[P + cell] = (float)gc[0];
-    mout[2 * P + cell] = (float)gc[1];
-    mout[3 * P + cell] = (float)gc[2];
-    Tout[cell] = gc[3];
-    niter_out[cell] = niter;
+    wave_lds_order();
   }
 }
 
@@ -1693,8 +1833,12 @@ hipError_t launch_step_split(int lattice, int interp, const SplitPtrs& in, const
                              int* niter, const float* guess, const SplitPending& pend, const SplitArgs& a,
                              hipStream_t st) {
   if (lattice == kD3Q125) {
-    hipLaunchKernelGGL(k_step_split125, dim3((unsigned)a.g.n), dim3(128), 0, st, in.f, in.m, in.T, out.f, out.m, out.T,
-                       niter, guess, a);
+    // Consecutive cells per wave: four, or two (one per half) where that would leave SIMDs without a
+    // wave.  Turbulence, ms per step with chunks of 2, 4, 8, 16, 32: 16^3 0.086, 0.104, 0.142, 0.229,
+    // 0.425; 32^3 0.359, 0.352, 0.346, 0.324, 0.484; 96^3 7.82, 7.63, 7.70, 7.72, 7.78.
+    const int chunk = a.g.n < 8192 ? 2 : 4;
+    hipLaunchKernelGGL(k_step_split125, dim3((unsigned)((a.g.n + chunk - 1) / chunk)), dim3(64), 0, st, in.f, in.m, in.T,
+                       out.f, out.m, out.T, niter, guess, a, chunk);
     return hipGetLastError();
   }
   if (lattice != kD3Q27) return hipErrorInvalidValue;
