@@ -1,6 +1,7 @@
 // pond_api.hip -- C ABI of the PonD step (include/pond.h): context lifetime, state upload and
 // download, the step driver (calcStep, update.cu:86-142, without the I/O it times), global
 // diagnostics and the .arr field dump.
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <cstdio>
@@ -84,6 +85,28 @@ __global__ void k_copy_state(StateView in, StateOut out, int64_t n, int64_t plan
     if (out.m64) out.m64[(int64_t)k * plane + c] = v;
     else if (k < 4) out.m32[(int64_t)k * plane + c] = (float)v;
     else out.T[c] = v;
+  }
+}
+
+// pond_copy_state between contexts of one precision: the buffers as they are, each read once and
+// written to both buffers of the destination, 16 bytes per lane.  blockIdx.y: the range.  (Cell by
+// cell with one lane per cell, as k_copy_state goes, a 96^3 D3Q125 split state took 6.0 ms, now 0.26;
+// a 256^3 D3Q27 one 3.2 ms.)
+struct CopyRange {
+  const uint4* in;
+  uint4 *out0, *out1;  // out1 may be null
+  int64_t n;           // 16-byte units
+};
+struct CopyRanges {
+  CopyRange r[4];
+};
+
+__global__ __launch_bounds__(256) void k_copy_same(const CopyRanges c) {
+  const CopyRange r = c.r[blockIdx.y];
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < r.n; i += (int64_t)gridDim.x * 256) {
+    const uint4 v = r.in[i];
+    r.out0[i] = v;
+    if (r.out1) r.out1[i] = v;
   }
 }
 
@@ -636,21 +659,45 @@ pond_status pond_copy_state(pond_ctx* dst, pond_ctx* src) {
   const Grid& g = dst->g;
   POND_HIP(src, hipStreamSynchronize(src->stream));
   POND_HIP(dst, hipStreamSynchronize(dst->stream));
-  StateView in{};
-  if (src->split) { in.f32 = src->sp[src->cur].f; in.m32 = src->sp[src->cur].m; in.T = src->sp[src->cur].T; }
-  else { in.f64 = src->f64[src->cur].f; in.m64 = src->f64[src->cur].m; }
-  const unsigned blocks = (unsigned)((g.n + 255) / 256);
-  // both buffers of the destination hold the state, as after pond_set_populations
-  for (int b = 0; b < 2; b++) {
-    StateOut out{};
-    if (dst->split) { out.f32 = dst->sp[b].f; out.m32 = dst->sp[b].m; out.T = dst->sp[b].T; }
-    else { out.f64 = dst->f64[b].f; out.m64 = dst->f64[b].m; }
-    hipLaunchKernelGGL(k_copy_state, dim3(blocks), dim3(256), 0, dst->stream, in, out, g.n, g.plane, dst->p.lattice,
-                       dst->Qn);
+  if (dst->split == src->split) {
+    // every buffer is a multiple of 64 elements long
+    CopyRanges c{};
+    auto range = [](const void* in, void* o0, void* o1, int64_t bytes) {
+      return CopyRange{(const uint4*)in, (uint4*)o0, (uint4*)o1, bytes / 16};
+    };
+    const int64_t f = dst->split ? split_fcount(dst->p.lattice, dst->Qn, g.plane) * (int64_t)sizeof(float)
+                                 : f64_fcount(dst->p.lattice, dst->Qn, g.plane) * (int64_t)sizeof(double);
+    if (dst->split) {
+      const SplitBuf &i = src->sp[src->cur], &o0 = dst->sp[0], &o1 = dst->sp[1];
+      c.r[0] = range(i.f, o0.f, o1.f, f);
+      c.r[1] = range(i.m, o0.m, o1.m, 4 * g.plane * (int64_t)sizeof(float));
+      c.r[2] = range(i.T, o0.T, o1.T, g.plane * (int64_t)sizeof(double));
+    } else {
+      const F64Buf &i = src->f64[src->cur], &o0 = dst->f64[0], &o1 = dst->f64[1];
+      c.r[0] = range(i.f, o0.f, o1.f, f);
+      c.r[1] = range(i.m, o0.m, o1.m, 5 * g.plane * (int64_t)sizeof(double));
+    }
+    c.r[3] = range(src->niter, dst->niter, nullptr, g.plane * (int64_t)sizeof(int));
+    const int64_t blocks = std::min<int64_t>((c.r[0].n + 255) / 256, 1 << 16);
+    hipLaunchKernelGGL(k_copy_same, dim3((unsigned)blocks, 4), dim3(256), 0, dst->stream, c);
     POND_HIP(dst, hipGetLastError());
+  } else {
+    StateView in{};
+    if (src->split) { in.f32 = src->sp[src->cur].f; in.m32 = src->sp[src->cur].m; in.T = src->sp[src->cur].T; }
+    else { in.f64 = src->f64[src->cur].f; in.m64 = src->f64[src->cur].m; }
+    const unsigned blocks = (unsigned)((g.n + 255) / 256);
+    // both buffers of the destination hold the state, as after pond_set_populations
+    for (int b = 0; b < 2; b++) {
+      StateOut out{};
+      if (dst->split) { out.f32 = dst->sp[b].f; out.m32 = dst->sp[b].m; out.T = dst->sp[b].T; }
+      else { out.f64 = dst->f64[b].f; out.m64 = dst->f64[b].m; }
+      hipLaunchKernelGGL(k_copy_state, dim3(blocks), dim3(256), 0, dst->stream, in, out, g.n, g.plane, dst->p.lattice,
+                         dst->Qn);
+      POND_HIP(dst, hipGetLastError());
+    }
+    POND_HIP(dst, hipMemcpyAsync(dst->niter, src->niter, (size_t)g.plane * sizeof(int), hipMemcpyDeviceToDevice,
+                                 dst->stream));
   }
-  POND_HIP(dst, hipMemcpyAsync(dst->niter, src->niter, (size_t)g.plane * sizeof(int), hipMemcpyDeviceToDevice,
-                               dst->stream));
   if (dst->cell_set && src->cell_set)
     POND_HIP(dst, hipMemcpyAsync(dst->cell_set, src->cell_set, (size_t)g.plane * sizeof(int),
                                  hipMemcpyDeviceToDevice, dst->stream));
