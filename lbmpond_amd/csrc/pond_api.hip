@@ -389,15 +389,11 @@ pond_status pond_create(const pond_params* p, pond_ctx** out) {
   a.inv_dim = 1. / ctx->L.Dim;
   a.g = g;
   a.global_loads = p->global_loads != 0;
-  // lane refill in the first pass of the FP64 D3Q27 step.  384^3 shock-bubble FP64 step: one
-  // tile per wave 8.07 s, chunks of 2 tiles 6.38 s, 4 tiles 7.05 s (4 tiles in a single pass
-  // 6.90 s); with 4x4 row patches 2 tiles 2.94 s, 3 3.06 s, 6 3.09 s.
-  a.refill_chunk = p->refill_chunk >= 0 ? p->refill_chunk : 2;
-  // Iterations of the first pass of the two-pass step; cells still unconverged are finished by
-  // the second pass.  Measured on the shock-bubble: FP64 D3Q27, 128^3: K=3 2.98, K=5 3.19, K=8
-  // 3.35, single pass 2.86 MLUPS; split D3Q27, 192^3: K=3 7.6, K=8 8.9, single pass 11.5 MLUPS
-  // (its second pass runs alone after the first and a few slowly converging cells make a serial
-  // tail), so the split step runs in one pass.
+  a.refill_chunk = p->refill_chunk;
+  // Iterations of the first pass of a two-pass step; cells still unconverged are finished by the
+  // second pass.  The split D3Q27 step by default runs in one pass (192^3 shock-bubble: K=3 7.6, K=8
+  // 8.9, single pass 11.5 MLUPS: its second pass runs alone after the first and a few slowly
+  // converging cells make a serial tail); the FP64 D3Q27 step always does.
   a.pass1_iters = p->pass1_iters > 0 ? p->pass1_iters : p->precision == POND_SPLIT ? (1 << 30) : 8;
   for (int i = 0; i < ctx->Qn; i++) a.w[i] = ctx->L.w[i];
 
@@ -413,10 +409,9 @@ pond_status pond_create(const pond_params* p, pond_ctx** out) {
       ctx->bytes += (int64_t)(fbytes + mbytes);
     }
     // D3Q27: 32-byte gauge records (ux, uy, uz, P); otherwise one P plane
-    if (hipMalloc(&ctx->nodeP, (size_t)(p->lattice == POND_D3Q27 ? 4 : 1) * g.plane * sizeof(double)) != hipSuccess ||
-        hipMalloc(&ctx->nodeok, (size_t)g.plane) != hipSuccess)
+    if (hipMalloc(&ctx->nodeP, (size_t)(p->lattice == POND_D3Q27 ? 4 : 1) * g.plane * sizeof(double)) != hipSuccess)
       return bail(POND_ERR_NOMEM, "pond_create: hipMalloc of the node planes failed");
-    ctx->bytes += (int64_t)g.plane * ((p->lattice == POND_D3Q27 ? 32 : 8) + 1);
+    ctx->bytes += (int64_t)g.plane * (p->lattice == POND_D3Q27 ? 32 : 8);
   } else {
     const size_t fbytes = (size_t)split_fcount(p->lattice, ctx->Qn, g.plane) * sizeof(float);
     const size_t mbytes = (size_t)4 * g.plane * sizeof(float);
@@ -512,7 +507,6 @@ void pond_destroy(pond_ctx* ctx) {
   if (ctx->cell_setnew) (void)hipFree(ctx->cell_setnew);
   if (ctx->sq) (void)hipFree(ctx->sq);
   if (ctx->nodeP) (void)hipFree(ctx->nodeP);
-  if (ctx->nodeok) (void)hipFree(ctx->nodeok);
   if (ctx->guess) (void)hipFree(ctx->guess);
   if (ctx->pend) (void)hipFree(ctx->pend);
   if (ctx->red) (void)hipFree(ctx->red);
@@ -763,9 +757,8 @@ pond_status pond_step(pond_ctx* ctx, int nsteps) {
       POND_HIP(ctx, hipEventRecord(ctx->mlp_ev[1], ctx->stream));
       ctx->mlp_pending = true;
     }
-    if (!ctx->split && !line) {
-      he = launch_node_prep(ctx->p.lattice, ctx->f64[in].f, ctx->f64[in].m, ctx->nodeP, ctx->nodeok, ctx->g.n,
-                            ctx->g.plane, ctx->stream);
+    if (!ctx->split && !line && ctx->p.lattice != POND_D3Q125) {
+      he = launch_node_prep(ctx->p.lattice, ctx->f64[in].m, ctx->nodeP, ctx->g.n, ctx->g.plane, ctx->stream);
       if (he != hipSuccess) return fail(ctx, POND_ERR_HIP, std::string("node prep kernel: ") + hipGetErrorString(he));
     }
     // the event pair brackets the step kernel alone
@@ -779,8 +772,8 @@ pond_status pond_step(pond_ctx* ctx, int nsteps) {
                              ctx->sq, ctx->niter,
                              learned ? ctx->guess : nullptr, pending_view(ctx), ctx->sargs, ctx->stream);
     } else {
-      he = launch_step_f64(ctx->p.lattice, ctx->p.interp, ctx->f64[in].f, ctx->f64[in].m, ctx->nodeP, ctx->nodeok,
-                           ctx->f64[outb].f, ctx->f64[outb].m, ctx->niter, pending_view(ctx), ctx->args, ctx->stream);
+      he = launch_step_f64(ctx->p.lattice, ctx->p.interp, ctx->f64[in].f, ctx->f64[in].m, ctx->nodeP, ctx->f64[outb].f,
+                           ctx->f64[outb].m, ctx->niter, pending_view(ctx), ctx->args, ctx->stream);
     }
     if (he != hipSuccess) return fail(ctx, POND_ERR_HIP, std::string("step kernel launch: ") + hipGetErrorString(he));
     if (last) {

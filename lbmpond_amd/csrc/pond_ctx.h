@@ -57,11 +57,10 @@ struct MlpCtx {
   int* idx = nullptr;
 };
 
-hipError_t launch_node_prep(int lattice, const double* f, const double* m, double* P, unsigned char* ok, int64_t n,
-                            int64_t plane, hipStream_t st);
+hipError_t launch_node_prep(int lattice, const double* m, double* P, int64_t n, int64_t plane, hipStream_t st);
 hipError_t launch_step_f64(int lattice, int interp, const double* fin, const double* min, const double* Pin,
-                           const unsigned char* okin, double* fout, double* mout, int* niter, const Pending& pend,
-                           const StepArgs& a, hipStream_t st);
+                           double* fout, double* mout, int* niter, const Pending& pend, const StepArgs& a,
+                           hipStream_t st);
 // whether the step of this lattice and grid is the one-launch D1Q5 line kernel, which forms its
 // node data itself (launch_node_prep is not needed)
 bool f64_line_step(int lattice, int interp, const Grid& g);
@@ -88,7 +87,6 @@ struct pond_ctx {
   pond::SplitArgs sargs{};
   double* nodeP = nullptr;  // plain path: per cell of the load buffer, D3Q27 the record (ux, uy, uz, P),
                             // else P, with P = sqrt(|T|)*sign(T)
-  unsigned char* nodeok = nullptr;  // plain path: populations finite and below 2^200
   float* sq = nullptr;      // split path: node gauge records (ux, uy, uz, sqrt(|T|)*sign(T)) of the load buffer
   float* guess = nullptr;   // split path: learned starting gauge increments (4 planes)
   // cells left unconverged by the first pass of a two-pass step: count, then per entry the

@@ -32,9 +32,9 @@ struct StepArgs {
   double sqrt_tbase;  // sqrt(TLat), evaluated once on the host (structs.cuh:530)
   double tlat;
   double inv_dim;     // 1./Dim (structs.cuh:330)
-  int pass1_iters;    // iterations of the first pass of the one-lane-per-cell step
+  int pass1_iters;    // D1Q5: iterations of the first pass of the one-lane-per-cell step
   int global_loads;   // 1: global loads even where the buffer-resource loads apply
-  int refill_chunk;   // D3Q27 first pass: 64-cell tiles per wave with lane refill (0: one tile per wave)
+  int refill_chunk;   // D3Q27: 64-cell tiles per wave (0: one; -1: the step's own choice of cells per wave)
   const int* cell_set;  // Cinfo::set per cell (0: not stepped), or null: every cell is stepped
   double w[kQmax];    // lattice weights for the collide and set_base
 };
@@ -161,6 +161,14 @@ inline int64_t f64_fcount(int lattice, int qn, int64_t plane) {
 
 __device__ __forceinline__ int64_t cell_index(const Grid& g, int x, int y, int z) {
   return (int64_t)x + (int64_t)g.nx * ((int64_t)y + (int64_t)g.ny * (int64_t)z);
+}
+
+// orders this wave's LDS writes before its following reads and its reads before following writes
+// (a wave's LDS operations execute in order; this holds the compiler to it)
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 }  // namespace pond

@@ -9,12 +9,11 @@
 //   * a node's transfer to a given target is computed once and reused where the reference
 //     recomputes it (the three overlapping WENO sub-stencils; 1D grids, where all y/z stencil
 //     nodes are the same cell);
-//   * populations of the iterate live in the output buffer instead of a register record, and
-//     the moment sums (structs.cuh:323-327) are accumulated while the populations are produced,
-//     in the same population order.
+//   * the transfer's NaN/Inf test is made on its sum (terms27);
+//   * the moment sums (structs.cuh:323-327) run over the stored iterate in the same population order.
 //
-// D1Q5/D3Q27 mapping: one lane per cell, 64 consecutive cells (x fastest) per wave, so node
-// loads of neighbouring lanes are neighbouring addresses of each population plane.
+// D3Q27 mapping: nine lanes per cell, one (ey, ez) group of three targets each.  D1Q5 lines: 32 lanes
+// per cell; other D1Q5 grids: one lane per cell, 64 consecutive cells (x fastest) per wave.
 // D3Q125 mapping: one 128-lane block per cell, lane = target population (as the reference's
 // 125-thread block), the fixed 3x3x3 neighbourhood staged in LDS.
 #include <type_traits>
@@ -30,16 +29,12 @@ struct Tgt27 {
   double W;           // (wk*wl)*wm
   double Cx, Cy, Cz;  // (e_inew*sqrt(|T1|))*sign(T1)
   bool kx, ky, kz;    // e_inew component != 0
-  bool wok;           // |W| < 2^200
 };
 
-// magnitude bound of the fast path: five factors below 2^200 multiply to below 2^1000
-constexpr double kSafe = 1.6069380442589903e60;  // 2^200
-
-__device__ __forceinline__ Tgt27 make_tgt27(int inew, double u1x, double u1y, double u1z, double T1) {
+// target population with velocity components (ex, ey, ez)
+__device__ __forceinline__ Tgt27 make_tgt27e(int ex, int ey, int ez, double u1x, double u1y, double u1z, double T1) {
   Tgt27 t;
   t.u1x = u1x; t.u1y = u1y; t.u1z = u1z; t.T1 = T1;
-  const int ex = kE27[inew][0], ey = kE27[inew][1], ez = kE27[inew][2];
   double wk = 1. / (2 * T1), wl = wk, wm = wk;
   if (ex == 0) wk = -1. / T1;
   if (ey == 0) wl = -1. / T1;
@@ -51,7 +46,6 @@ __device__ __forceinline__ Tgt27 make_tgt27(int inew, double u1x, double u1y, do
   t.Cy = (double)ey * sq1 * sg1;
   t.Cz = (double)ez * sq1 * sg1;
   t.kx = ex != 0; t.ky = ey != 0; t.kz = ez != 0;
-  t.wok = fabs(t.W) < kSafe;
   return t;
 }
 
@@ -60,7 +54,6 @@ struct NodeSrc {
   const double* __restrict__ f;          // population planes, stride g.plane
   const double* __restrict__ m;          // rho, ux, uy, uz, T planes
   const double* __restrict__ P;          // sqrt(|T|)*sign(T) per cell (params.h:110-112)
-  const unsigned char* __restrict__ ok;  // populations finite and below 2^200
   Grid g;
 };
 
@@ -69,23 +62,20 @@ __device__ __forceinline__ double ldp(const double* base, int64_t k, int64_t pla
 }
 
 __device__ __forceinline__ uint32_t node_off(const Grid& g, int x, int y, int z) {
-  return (uint32_t)cell_index(g, x, y, z) * 8u;
+  return ((uint32_t)x + (uint32_t)g.nx * ((uint32_t)y + (uint32_t)g.ny * (uint32_t)z)) * 8u;
 }
 
-// The same node data as raw buffer resources: population planes 9j .. 9j+8 in resource j, the
-// plane selected by the scalar offset, the per-lane address a single 32-bit offset (a global
-// load needs a 64-bit per-lane address: two VGPRs and a 64-bit add per load).  Resource sizes
-// are exact, so the hardware range check returns 0 rather than reading past an array.  Word 3
-// (0x00020000) is the raw-buffer configuration of the gfx9 family.  Usable while nine FP64
-// planes fit in 4 GiB (plane <= 59,652,323 cells).
-constexpr int kPlanesPerRsrc64 = 9;
+// The D3Q27 node data as raw buffer resources: pair planes 4j .. 4j+3 in resource j, the plane
+// selected by the scalar offset, the per-lane address a single 32-bit offset (a global load needs a
+// 64-bit per-lane address: two VGPRs and a 64-bit add per load).  Resource sizes are exact, so the
+// hardware range check returns 0 rather than reading past an array.  Word 3 (0x00020000) is the
+// raw-buffer configuration of the gfx9 family.  Usable while four pair planes fit in 4 GiB (plane <=
+// 67,108,800 cells).
 constexpr int kRawBufferWord3 = 0x00020000;
 
 struct NodeBuf {
-  // populations: D1Q5 planes 9j .. 9j+8 in f[j]; D3Q27 pair planes 4j .. 4j+3 in f[j]
-  __amdgpu_buffer_rsrc_t f[4], m, P, ok;
-  uint32_t pbytes;                      // bytes per FP64 plane
-  uint32_t qbytes;                      // bytes per D3Q27 pair plane
+  __amdgpu_buffer_rsrc_t f[4], P;
+  uint32_t qbytes;  // bytes per pair plane
   Grid g;
 };
 
@@ -93,47 +83,23 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc64(const void* base, uint6
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)(uint32_t)bytes, kRawBufferWord3);
 }
 
-template <int LAT>
 __device__ __forceinline__ NodeBuf make_nodebuf(const NodeSrc& s) {
   NodeBuf b;
   const uint64_t pb = (uint64_t)s.g.plane * 8u;
-  b.pbytes = (uint32_t)pb;
   b.qbytes = (uint32_t)(2 * pb);
-  if (LAT == kD3Q27) {
-    for (int j = 0; j < 4; j++) {
-      const int cnt = 14 - 4 * j < 4 ? 14 - 4 * j : 4;
-      b.f[j] = rsrc64(s.f + (int64_t)8 * j * s.g.plane, (uint64_t)cnt * 2 * pb);
-    }
-  } else {
-    for (int j = 0; j < 3; j++) b.f[j] = rsrc64(s.f + (int64_t)j * kPlanesPerRsrc64 * s.g.plane, kPlanesPerRsrc64 * pb);
-    b.f[3] = b.f[2];
+  for (int j = 0; j < 4; j++) {
+    const int cnt = 14 - 4 * j < 4 ? 14 - 4 * j : 4;
+    b.f[j] = rsrc64(s.f + (int64_t)8 * j * s.g.plane, (uint64_t)cnt * 2 * pb);
   }
-  b.m = rsrc64(s.m, 5 * pb);
-  b.P = rsrc64(s.P, LAT == kD3Q27 ? 4 * pb : pb);
-  b.ok = rsrc64(s.ok, (uint64_t)s.g.plane);
+  b.P = rsrc64(s.P, 4 * pb);
   b.g = s.g;
   return b;
 }
 
-// node accessors: population k, moment plane k, P, finite flag of the node at byte offset boff
+// node accessors: population k, moment plane k, P of the node at byte offset boff
 __device__ __forceinline__ double node_f(const NodeSrc& s, int k, uint32_t boff) { return ldp(s.f, k, s.g.plane, boff); }
 __device__ __forceinline__ double node_m(const NodeSrc& s, int k, uint32_t boff) { return ldp(s.m, k, s.g.plane, boff); }
 __device__ __forceinline__ double node_P(const NodeSrc& s, uint32_t boff) { return ldp(s.P, 0, s.g.plane, boff); }
-__device__ __forceinline__ bool node_ok(const NodeSrc& s, uint32_t boff) { return s.ok[boff >> 3] != 0; }
-
-__device__ __forceinline__ double ldb64(__amdgpu_buffer_rsrc_t r, uint32_t boff, uint32_t soff) {
-  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, (int)boff, (int)soff, 0));
-}
-__device__ __forceinline__ double node_f(const NodeBuf& s, int k, uint32_t boff) {
-  return ldb64(s.f[k / kPlanesPerRsrc64], boff, (uint32_t)(k % kPlanesPerRsrc64) * s.pbytes);
-}
-__device__ __forceinline__ double node_m(const NodeBuf& s, int k, uint32_t boff) {
-  return ldb64(s.m, boff, (uint32_t)k * s.pbytes);
-}
-__device__ __forceinline__ double node_P(const NodeBuf& s, uint32_t boff) { return ldb64(s.P, boff, 0); }
-__device__ __forceinline__ bool node_ok(const NodeBuf& s, uint32_t boff) {
-  return __builtin_amdgcn_raw_buffer_load_b8(s.ok, (int)(boff >> 3), 0, 0) != 0;
-}
 
 // D3Q27: the node's gauge record (ux, uy, uz, sqrt(|T|)*sign(T)), 32 bytes per cell, written by
 // k_node_prep into the P buffer, at byte offset boff of an FP64 plane (boff = 8 * cell)
@@ -175,55 +141,41 @@ __device__ __forceinline__ void node_f27(const NodeBuf& s, uint32_t boff, double
   }
 }
 
-// basis values of the node at byte offset boff for target t (structs.cuh:530-538).
+// basis values of a node with gauge (u0, P) for target t (structs.cuh:530-538).
 // e_iold*sqrt(|T0|)*sign(T0) for e_iold = -1, 0, +1 is exactly {-P, 0*P, P}.
-__device__ __forceinline__ bool basis27u(double u0x, double u0y, double u0z, double Pn, bool nok, const Tgt27& t,
-                                         double sqTb, double gx[3], double gy[3], double gz[3]) {
+__device__ __forceinline__ void basis27(double u0x, double u0y, double u0z, double Pn, const Tgt27& t, double sqTb,
+                                        double gx[3], double gy[3], double gz[3]) {
   const double Dx = (t.u1x - u0x) * sqTb;
   const double Dy = (t.u1y - u0y) * sqTb;
   const double Dz = (t.u1z - u0z) * sqTb;
   const double E[3] = {-Pn, 0.0 * Pn, Pn};
-  bool safe = nok && t.wok;
 #pragma unroll
   for (int j = 0; j < 3; j++) {
     const double ax = Dx - E[j], ay = Dy - E[j], az = Dz - E[j];
     gx[j] = ax * ax - (t.kx ? t.Cx * ax : t.T1);
     gy[j] = ay * ay - (t.ky ? t.Cy * ay : t.T1);
     gz[j] = az * az - (t.kz ? t.Cz * az : t.T1);
-    safe = safe && fabs(gx[j]) < kSafe && fabs(gy[j]) < kSafe && fabs(gz[j]) < kSafe;
   }
-  return safe;
 }
 
-template <class SRC>
-__device__ __forceinline__ bool basis27(const SRC& s, uint32_t boff, const Tgt27& t, double sqTb, double gx[3],
-                                        double gy[3], double gz[3]) {
-  double u0x, u0y, u0z, Pn;
-  node_g4(s, boff, u0x, u0y, u0z, Pn);
-  return basis27u(u0x, u0y, u0z, Pn, node_ok(s, boff), t, sqTb, gx, gy, gz);
-}
-
-// gauge transfer of the node at byte offset boff to target t (structs.cuh:525-548)
-template <class SRC>
-__device__ __forceinline__ double transfer27(const SRC& s, uint32_t boff, const Tgt27& t, double sqTb) {
-  double gx[3], gy[3], gz[3];
-  const bool safe = basis27(s, boff, t, sqTb, gx, gy, gz);
+// The transfer's term loop (structs.cuh:539-548) over the populations f.  The reference drops every
+// NaN or infinite term; a sum that comes out finite has dropped none (one such term leaves the plain
+// sum NaN or infinite), so the plain sum is formed and only a non-finite one is formed again with
+// the test on every term.
+__device__ __forceinline__ double terms27(double W, const double (&gx)[3], const double (&gy)[3],
+                                          const double (&gz)[3], const double (&f)[27]) {
   double p2[3][3];
 #pragma unroll
   for (int a = 0; a < 3; a++)
 #pragma unroll
-    for (int b = 0; b < 3; b++) p2[a][b] = t.W * gx[a] * gy[b];
-  double f[27];
-  node_f27(s, boff, f);
+    for (int b = 0; b < 3; b++) p2[a][b] = W * gx[a] * gy[b];
   double fnew = 0;
 #pragma unroll
   for (int iold = 0; iold < 27; iold++) {
     const int jx = kE27[iold][0] + 1, jy = kE27[iold][1] + 1, jz = kE27[iold][2] + 1;
     fnew += p2[jx][jy] * gz[jz] * f[iold];
   }
-  if (!safe) {
-    // the reference's term loop with NaN/Inf terms dropped (structs.cuh:539-542), for the
-    // nodes that fail the magnitude test; in line, so the basis values stay in registers
+  if (!finite_d(fnew)) {
     fnew = 0;
 #pragma unroll
     for (int iold = 0; iold < 27; iold++) {
@@ -233,6 +185,32 @@ __device__ __forceinline__ double transfer27(const SRC& s, uint32_t boff, const 
     }
   }
   return fnew;
+}
+
+// exchanges the populations of a D3Q27 record with their mirror images along axis AX in the lanes
+// with m set
+template <int AX>
+__device__ __forceinline__ void mirror27(bool m, double (&f)[27]) {
+#pragma unroll
+  for (int i = 0; i < 27; i++) {
+    if (kE27[i][AX] != 1) continue;
+    const int j = kIdx27.v[AX == 0 ? 0 : kE27[i][0] + 1][AX == 1 ? 0 : kE27[i][1] + 1][AX == 2 ? 0 : kE27[i][2] + 1];
+    const double a = f[i], b = f[j];
+    f[i] = m ? b : a;
+    f[j] = m ? a : b;
+  }
+}
+
+// gauge transfer of the node at byte offset boff to target t (structs.cuh:525-548)
+template <class SRC>
+__device__ __forceinline__ double transfer27(const SRC& s, uint32_t boff, const Tgt27& t, double sqTb) {
+  double u0x, u0y, u0z, Pn;
+  node_g4(s, boff, u0x, u0y, u0z, Pn);
+  double gx[3], gy[3], gz[3];
+  basis27(u0x, u0y, u0z, Pn, t, sqTb, gx, gy, gz);
+  double f[27];
+  node_f27(s, boff, f);
+  return terms27(t.W, gx, gy, gz, f);
 }
 
 // transfer27 of the node's mirror image on the axes set in mx, my, mz (Cell::mirrX/Y/Z,
@@ -247,34 +225,13 @@ __device__ double transfer27_mirrored(const SRC& s, uint32_t boff, const Tgt27& 
   if (my) u0y = -u0y;
   if (mz) u0z = -u0z;
   double gx[3], gy[3], gz[3];
-  const bool safe = basis27u(u0x, u0y, u0z, Pn, node_ok(s, boff), t, sqTb, gx, gy, gz);
-  double p2[3][3];
-#pragma unroll
-  for (int a = 0; a < 3; a++)
-#pragma unroll
-    for (int b = 0; b < 3; b++) p2[a][b] = t.W * gx[a] * gy[b];
-  double f0[27], f[27];
-  node_f27(s, boff, f0);
-#pragma unroll
-  for (int i = 0; i < 27; i++) {
-    const int jx = kE27[i][0] + 1, jy = kE27[i][1] + 1, jz = kE27[i][2] + 1;
-    // f[i] = f0 of the mirrored velocity, as selects over compile-time indices
-    const double a0 = mx ? f0[kIdx27.v[2 - jx][jy][jz]] : f0[i];
-    const double a1 = mx ? f0[kIdx27.v[2 - jx][2 - jy][jz]] : f0[kIdx27.v[jx][2 - jy][jz]];
-    const double b0 = my ? a1 : a0;
-    const double a2 = mx ? f0[kIdx27.v[2 - jx][jy][2 - jz]] : f0[kIdx27.v[jx][jy][2 - jz]];
-    const double a3 = mx ? f0[kIdx27.v[2 - jx][2 - jy][2 - jz]] : f0[kIdx27.v[jx][2 - jy][2 - jz]];
-    const double b1 = my ? a3 : a2;
-    f[i] = mz ? b1 : b0;
-  }
-  double fnew = 0;
-#pragma unroll
-  for (int iold = 0; iold < 27; iold++) {
-    const int jx = kE27[iold][0] + 1, jy = kE27[iold][1] + 1, jz = kE27[iold][2] + 1;
-    const double fadd = p2[jx][jy] * gz[jz] * f[iold];
-    if (safe || finite_d(fadd)) fnew += fadd;
-  }
-  return fnew;
+  basis27(u0x, u0y, u0z, Pn, t, sqTb, gx, gy, gz);
+  double f[27];
+  node_f27(s, boff, f);
+  mirror27<0>(mx, f);
+  mirror27<1>(my, f);
+  mirror27<2>(mz, f);
+  return terms27(t.W, gx, gy, gz, f);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -312,7 +269,7 @@ __device__ __forceinline__ Tgt5 make_tgt5(int inew, double u1x, double T1) {
 __device__ __forceinline__ double transfer5v(double u0x, double s0, const double (&f)[5], const Tgt5& t) {
   const double et = t.et;
   const double difu = t.u1x - u0x;
-  double fnew = t.fnew0;
+  double fadd[5];
 #pragma unroll
   for (int iold = 0; iold < 5; iold++) {
     const double e = kA5[iold] * s0;
@@ -332,8 +289,17 @@ __device__ __forceinline__ double transfer5v(double u0x, double s0, const double
     dm4 = dm4 * dm4 * dm4 * dm4;
     dm4 *= 0;
     const double gx = K4 * difu * difu * difu * difu + K3 * difu * difu * difu + K2 * difu * difu + K1 * difu + K0 - dm4;
-    const double fadd = t.wk * gx * f[iold];
-    if (finite_d(fadd)) fnew += fadd;
+    fadd[iold] = t.wk * gx * f[iold];
+  }
+  // non-finite terms are dropped (structs.cuh:390); a finite sum has none (as in terms27)
+  double fnew = t.fnew0;
+#pragma unroll
+  for (int iold = 0; iold < 5; iold++) fnew += fadd[iold];
+  if (!finite_d(fnew)) {
+    fnew = t.fnew0;
+#pragma unroll
+    for (int iold = 0; iold < 5; iold++)
+      if (finite_d(fadd[iold])) fnew += fadd[iold];
   }
   return fnew;
 }
@@ -366,7 +332,7 @@ struct Lat<kD3Q27> {
   static constexpr int Q = 27;
   using Tgt = Tgt27;
   __device__ static double efc(int i, int d) { return (double)kE27[i][d]; }
-  __device__ static Tgt tgt(int i, const double* g) { return make_tgt27(i, g[0], g[1], g[2], g[3]); }
+  __device__ static Tgt tgt(int i, const double* g) { return make_tgt27e(kE27[i][0], kE27[i][1], kE27[i][2], g[0], g[1], g[2], g[3]); }
   template <class SRC>
   __device__ static double xfer(const SRC& s, uint32_t boff, const Tgt& t, double sqTb) {
     return transfer27(s, boff, t, sqTb);
@@ -402,6 +368,17 @@ __device__ __forceinline__ void lag3_factors(double s, double F[3][2]) {
   F[0][0] = (s - 1) / (0 - 1); F[0][1] = (s - 2) / (0 - 2);
   F[1][0] = (s - 0) / (1 - 0); F[1][1] = (s - 2) / (1 - 2);
   F[2][0] = (s - 0) / (2 - 0); F[2][1] = (s - 1) / (2 - 1);
+}
+
+// its factors of node i alone (i the same in every lane)
+__device__ __forceinline__ void lag3_row(double s, int i, double (&f)[2]) {
+  if (i == 0) {
+    f[0] = (s - 1) / (0 - 1); f[1] = (s - 2) / (0 - 2);
+  } else if (i == 1) {
+    f[0] = (s - 0) / (1 - 0); f[1] = (s - 2) / (1 - 2);
+  } else {
+    f[0] = (s - 0) / (2 - 0); f[1] = (s - 1) / (2 - 1);
+  }
 }
 
 __device__ __forceinline__ void lag4_factors(double s, double F[4][3]) {
@@ -551,69 +528,62 @@ __device__ double interp_weno5(const SRC& src, double cx, double cy, double cz, 
 // in order inside a slice), so every value is bitwise what interp_weno5 / interp_lagr4 give.
 
 // The three targets of a group: the fields of Tgt27 they share (u1, T1 and the y, z target
-// components) once, the x ones per target.
+// components) once, the x ones per target.  An axis' term is C*a for a moving target component and
+// T1 for a resting one: with (Cy, Ty) = (C, 0) or (0, T1) it is Cy*a + Ty, the same bits for finite a
+// (the terms of a non-finite one are dropped in either form).
 struct Tgt27g3 {
-  double u1x, u1y, u1z, T1, Cy, Cz;
+  double u1x, u1y, u1z, T1, Cy, Ty, Cz, Tz;
   bool ky, kz;
-  double W[3], Cx[3];
-  bool kx[3], wok[3];
+  double W0, W1, Cx;  // W of ex = 0 and of ex = -1, +1; C of ex = +1 (its negative for ex = -1)
 };
 
-// transfer27 of one node to the targets k with use[k] (T[k]; the others untouched)
+// one stencil node's data in registers
+struct Node27 {
+  double ux, uy, uz, P, f[27];
+};
+
 template <class SRC>
-__device__ __forceinline__ void transfer27_g3(const SRC& s, uint32_t boff, const Tgt27g3& t, const bool (&use)[3],
-                                              double sqTb, double (&T)[3]) {
-  double u0x, u0y, u0z, Pn;
-  node_g4(s, boff, u0x, u0y, u0z, Pn);
-  const bool nok = node_ok(s, boff);
+__device__ __forceinline__ void load_node27(const SRC& s, uint32_t boff, Node27& n) {
+  node_g4(s, boff, n.ux, n.uy, n.uz, n.P);
+  node_f27(s, boff, n.f);
+}
+
+// transfer27 of one node to the targets k with use[k] (T[k]; the others untouched).  MIR: of its
+// mirror image on the axes set in mx, my, mz (transfer27_mirrored)
+template <bool MIR = false>
+__device__ __forceinline__ void transfer27_g3(Node27& n, const Tgt27g3& t, const bool (&use)[3], double sqTb,
+                                              double (&T)[3], bool mx = false, bool my = false, bool mz = false) {
+  double u0x = n.ux, u0y = n.uy, u0z = n.uz;
+  if (MIR) {
+    u0x = mx ? -u0x : u0x;
+    u0y = my ? -u0y : u0y;
+    u0z = mz ? -u0z : u0z;
+  }
   // basis27u, split into the x part (per target) and the shared y and z parts
   const double Dx = (t.u1x - u0x) * sqTb;
   const double Dy = (t.u1y - u0y) * sqTb;
   const double Dz = (t.u1z - u0z) * sqTb;
-  const double E[3] = {-Pn, 0.0 * Pn, Pn};
+  const double E[3] = {-n.P, 0.0 * n.P, n.P};
   double ax[3], gy[3], gz[3];
-  bool syz = true;
 #pragma unroll
   for (int j = 0; j < 3; j++) {
     ax[j] = Dx - E[j];
     const double ay = Dy - E[j], az = Dz - E[j];
-    gy[j] = ay * ay - (t.ky ? t.Cy * ay : t.T1);
-    gz[j] = az * az - (t.kz ? t.Cz * az : t.T1);
-    syz = syz && fabs(gy[j]) < kSafe && fabs(gz[j]) < kSafe;
+    gy[j] = ay * ay - (t.Cy * ay + t.Ty);
+    gz[j] = az * az - (t.Cz * az + t.Tz);
   }
-  double f[27];
-  node_f27(s, boff, f);
+  if (MIR) {
+    if (__any(mx)) mirror27<0>(mx, n.f);
+    if (__any(my)) mirror27<1>(my, n.f);
+    if (__any(mz)) mirror27<2>(mz, n.f);
+  }
 #pragma unroll
   for (int k = 0; k < 3; k++) {
     if (!use[k]) continue;
     double gx[3];
-    bool safe = nok && t.wok[k] && syz;
 #pragma unroll
-    for (int j = 0; j < 3; j++) {
-      gx[j] = ax[j] * ax[j] - (t.kx[k] ? t.Cx[k] * ax[j] : t.T1);
-      safe = safe && fabs(gx[j]) < kSafe;
-    }
-    double p2[3][3];
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-      for (int b = 0; b < 3; b++) p2[a][b] = t.W[k] * gx[a] * gy[b];
-    double fnew = 0;
-#pragma unroll
-    for (int iold = 0; iold < 27; iold++) {
-      const int jx = kE27[iold][0] + 1, jy = kE27[iold][1] + 1, jz = kE27[iold][2] + 1;
-      fnew += p2[jx][jy] * gz[jz] * f[iold];
-    }
-    if (!safe) {
-      fnew = 0;
-#pragma unroll
-      for (int iold = 0; iold < 27; iold++) {
-        const int jx = kE27[iold][0] + 1, jy = kE27[iold][1] + 1, jz = kE27[iold][2] + 1;
-        const double fadd = p2[jx][jy] * gz[jz] * f[iold];
-        if (finite_d(fadd)) fnew += fadd;
-      }
-    }
-    T[k] = fnew;
+    for (int j = 0; j < 3; j++) gx[j] = ax[j] * ax[j] - (k == 0 ? -t.Cx * ax[j] : k == 2 ? t.Cx * ax[j] : t.T1);
+    T[k] = terms27(k == 1 ? t.W0 : t.W1, gx, gy, gz, n.f);
   }
 }
 
@@ -628,39 +598,89 @@ __device__ __forceinline__ double lag3x(double cx, int r, int q, int ix) {
 __device__ __forceinline__ Tgt27 tgt27_of(const Tgt27g3& t, int k) {
   Tgt27 tk;
   tk.u1x = t.u1x; tk.u1y = t.u1y; tk.u1z = t.u1z; tk.T1 = t.T1;
-  tk.W = t.W[k]; tk.Cx = t.Cx[k]; tk.Cy = t.Cy; tk.Cz = t.Cz;
-  tk.kx = t.kx[k]; tk.ky = t.ky; tk.kz = t.kz; tk.wok = t.wok[k];
+  tk.W = k == 1 ? t.W0 : t.W1; tk.Cx = k == 0 ? -t.Cx : t.Cx; tk.Cy = t.Cy; tk.Cz = t.Cz;
+  tk.kx = k != 1; tk.ky = t.ky; tk.kz = t.kz;
   return tk;
+}
+
+// The walk over the stencil nodes of a group: slices d = dlo .. dhi relative to the cell's x, NR rows in
+// y from ry and in z from rz.  Calls slice(d) at the start of a slice, row(a) at the start of a row,
+// and node(n, d, a, b) with the node's data.  Row offsets are 32-bit (node_off, mod 2^32).
+//
+// Tried, and slower (128^3 vortex, this walk 65 ms per step): the loads of a node issued a node ahead
+// (74 ms: the populations then live through the weighting and push its values to scratch); each
+// different node of a wave's cells loaded once, 16 bytes per lane, and handed out through LDS (112
+// ms: the loaders' addresses go to scratch, and a scratch access occupies the L1 for as long as a
+// 16-byte load); held to three waves per SIMD (183 ms, scratch again).
+template <int NR, bool MIR, class SRC, class FS, class FR, class FN>
+__device__ __forceinline__ void walk27(const SRC& src, int x, int ry, int rz, int dlo, int dhi, FS&& slice, FR&& row,
+                                       FN&& node) {
+  const Grid& g = src.g;
+  bool rv;
+  uint32_t yo[NR], zo[NR];
+#pragma unroll
+  for (int q = 0; q < NR; q++) {
+    yo[q] = (uint32_t)(MIR ? mirror_wrap(ry + q, g.ny, (g.mirror & 2) != 0, rv) : wrapi(ry + q, g.ny)) * (uint32_t)g.nx;
+    zo[q] = (uint32_t)(MIR ? mirror_wrap(rz + q, g.nz, (g.mirror & 4) != 0, rv) : wrapi(rz + q, g.nz)) *
+            ((uint32_t)g.nx * (uint32_t)g.ny);
+  }
+#pragma unroll 1
+  for (int d = dlo; d <= dhi; d++) {
+    slice(d);
+    const uint32_t xw = (uint32_t)(MIR ? mirror_wrap(x + d, g.nx, (g.mirror & 1) != 0, rv) : wrapi(x + d, g.nx));
+#pragma unroll 1
+    for (int a = 0; a < NR; a++) {
+      row(a);
+      const uint32_t xy = xw + (a == 0 ? yo[0] : a == 1 ? yo[1] : a == 2 ? yo[2] : yo[NR - 1]);
+#pragma unroll 1
+      for (int b = 0; b < NR; b++) {
+        Node27 n;
+        load_node27(src, (xy + (b == 0 ? zo[0] : b == 1 ? zo[1] : b == 2 ? zo[2] : zo[NR - 1])) * 8u, n);
+        node(n, d, a, b);
+      }
+    }
+  }
 }
 
 // interp_weno5<kD3Q27, VAR> for the three targets of a group (cx[k] of target ex = k - 1; cy, cz
 // shared), on a grid that is not a line, without mirrors.  Window positions are taken relative
 // to the cell's own x, so lanes of a wave whose flow is alike visit the same positions.  Taken
-// only for s = sqrt(T1/TLat) <= 1.5 (f64_once): the windows of ex = -1 and +1 are 2s apart, so
+// only for s = sqrt(T1/TLat) <= 1.5 (f64_group): the windows of ex = -1 and +1 are 2s apart, so
 // the union spans at most 9 slices.
+//
+// Registers are what this is short of: the departure points and windows in x are formed again at
+// every slice and the y and z Lagrange factors at every row and node instead of being kept.
 template <int VAR, class SRC>
-__device__ void interp_weno5_g3(const SRC& src, int x, const double (&cx)[3], double cy, double cz,
-                                const Tgt27g3& t, double sqTb, double (&fn)[3]) {
+__device__ __forceinline__ void interp_weno5_g3(const SRC& src, int x, double s, double cy, double cz,
+                                                const Tgt27g3& t, double sqTb, double (&fn)[3]) {
   constexpr bool CENTRED = VAR == 1;
   const Grid& g = src.g;
   const int ry = floor_int(cy + 0.5) - (CENTRED ? 1 : 0), rz = floor_int(cz + 0.5) - (CENTRED ? 1 : 0);
   const double sy = cy - ry, sz = cz - rz;
-  double Fy[3][2], Fz[3][2];
-  lag3_factors(sy, Fy);
-  lag3_factors(sz, Fz);
-  int r[3], w0[3];  // window start relative to x
+  auto target_x = [&](int k, double& cx, int& r) {  // departure point and window middle of ex = k - 1
+    cx = (double)x - (s * (double)(k - 1) + t.u1x);
+    r = floor_int(cx + 0.5);
+  };
+  int wlo = 0, whi = 0;  // lowest and highest window start relative to x
 #pragma unroll
   for (int k = 0; k < 3; k++) {
-    r[k] = floor_int(cx[k] + 0.5);
-    w0[k] = (r[k] - 2) - x;
+    double cx;
+    int r;
+    target_x(k, cx, r);
+    const int w = (r - 2) - x;
+    wlo = k == 0 ? w : min(wlo, w);
+    whi = k == 0 ? w : max(whi, w);
   }
-  const int dlo = min(w0[0], min(w0[1], w0[2]));
+  const int dlo = wlo;
   // (at most dlo + 8 for s <= 1.5; the bound keeps the loop finite whatever the caller passes)
-  const int dhi = min(max(w0[0], max(w0[1], w0[2])) + 4, dlo + 8);
-  // the smoothness samples of the three targets wait in LDS (one wave per block), which keeps
-  // the sub-stencil sums and a node's populations in registers
+  const int dhi = min(whi + 4, dlo + 8);
+  // The smoothness samples of the three targets wait in LDS (one wave per block), which keeps the
+  // sub-stencil sums and a node's populations in registers; so do the slice's x weights (the same
+  // for a cell's lanes), which a row takes up with its own y factors: the products' left prefixes,
+  // shared by the row's nodes.
   __shared__ double s_ub[3][5][64];
-  const int lane = threadIdx.x & 63;
+  __shared__ double s_pw[3][3][8];
+  const int lane = threadIdx.x & 63, slot = lane / 9;
   double S[3][3];
 #pragma unroll
   for (int k = 0; k < 3; k++) {
@@ -669,57 +689,76 @@ __device__ void interp_weno5_g3(const SRC& src, int x, const double (&cx)[3], do
 #pragma unroll
     for (int j = 0; j < 5; j++) s_ub[k][j][lane] = 0;
   }
-  for (int d = dlo; d <= dhi; d++) {
-    const int xw = wrapi(x + d, g.nx);
-    int xs[3];
-    bool use[3];
-    double pw[3][3];  // per target, the x weight of this slice in sub-stencils 0, 1, 2
+  const bool finite_w = finite_d(cy) && finite_d(cz);
+  int xs[3] = {0, 0, 0};
+  bool use[3] = {false, false, false};
+  double pf[3][3];  // per target, the left prefix of the row's weights in sub-stencils 0, 1, 2
+  auto slice = [&](int d) {
+    wave_lds_order();
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-      xs[k] = d - w0[k];
-      use[k] = xs[k] >= 0 && xs[k] <= 4;
-      const int j = xs[k];
+      double cx;
+      int r;
+      target_x(k, cx, r);
+      const int j = d - ((r - 2) - x);
+      xs[k] = j;
+      use[k] = j >= 0 && j <= 4;
 #pragma unroll
-      for (int q = 0; q < 3; q++) pw[k][q] = (j - q >= 0 && j - q <= 2) ? lag3x(cx[k], r[k], q, j - q) : 0.0;
+      for (int q = 0; q < 3; q++) s_pw[k][q][slot] = (j - q >= 0 && j - q <= 2) ? lag3x(cx, r, q, j - q) : 0.0;
     }
-#pragma unroll 1
-    for (int a = 0; a < 3; a++) {
-      const int ya = wrapi(ry + a, g.ny);
-#pragma unroll 1
-      for (int b = 0; b < 3; b++) {
-        double T[3] = {0, 0, 0};
-        transfer27_g3(src, node_off(g, xw, ya, wrapi(rz + b, g.nz)), t, use, sqTb, T);
-        const double fy0 = a == 0 ? Fy[0][0] : a == 1 ? Fy[1][0] : Fy[2][0];
-        const double fy1 = a == 0 ? Fy[0][1] : a == 1 ? Fy[1][1] : Fy[2][1];
-        const double fz0 = b == 0 ? Fz[0][0] : b == 1 ? Fz[1][0] : Fz[2][0];
-        const double fz1 = b == 0 ? Fz[0][1] : b == 1 ? Fz[1][1] : Fz[2][1];
+    wave_lds_order();
+  };
+  auto row = [&](int a) {
+    double fy[2];
+    lag3_row(sy, a, fy);
 #pragma unroll
-        for (int k = 0; k < 3; k++) {
-          if (!use[k]) continue;
-          const int j = xs[k];
+    for (int k = 0; k < 3; k++)
 #pragma unroll
-          for (int q = 0; q < 3; q++)
-            if (j - q >= 0 && j - q <= 2) S[k][q] += pw[k][q] * fy0 * fy1 * fz0 * fz1 * T[k];
-          if (CENTRED && a == 1 && b == 1) s_ub[k][j][lane] = T[k];
-        }
+      for (int q = 0; q < 3; q++) pf[k][q] = s_pw[k][q][slot] * fy[0] * fy[1];
+  };
+  auto node = [&](Node27& n, int d, int a, int b) {
+    double T[3] = {0, 0, 0};
+    transfer27_g3(n, t, use, sqTb, T);
+    double fz[2];
+    lag3_row(sz, b, fz);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      if (__ballot(use[k]) == 0) continue;
+      // a sub-stencil that does not hold the slice has weight zero, and adding a zero changes no sum
+      // that started from +0; only with a value or weight that is not finite it is left out
+      if (__ballot(!(finite_w && finite_d(T[k]))) == 0) {
+#pragma unroll
+        for (int q = 0; q < 3; q++) S[k][q] += pf[k][q] * fz[0] * fz[1] * T[k];
+      } else {
+        const int j = xs[k];
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+          if (use[k] && j - q >= 0 && j - q <= 2) S[k][q] += pf[k][q] * fz[0] * fz[1] * T[k];
       }
+      if (CENTRED && a == 1 && b == 1 && use[k]) s_ub[k][xs[k]][lane] = T[k];
     }
-    if (!CENTRED) {
+    if (!CENTRED && a == 2 && b == 2) {
       // smoothness samples on the row (r mod Ny, r mod Nz) of each target
 #pragma unroll
       for (int k = 0; k < 3; k++) {
         if (!use[k]) continue;
+        double cx;
+        int r;
+        target_x(k, cx, r);
         s_ub[k][xs[k]][lane] =
-            transfer27(src, node_off(g, xw, wrapi(r[k], g.ny), wrapi(r[k], g.nz)), tgt27_of(t, k), sqTb);
+            transfer27(src, node_off(g, wrapi(x + d, g.nx), wrapi(r, g.ny), wrapi(r, g.nz)), tgt27_of(t, k), sqTb);
       }
     }
-  }
+  };
+  walk27<3, false>(src, x, ry, rz, dlo, dhi, slice, row, node);
 #pragma unroll
   for (int k = 0; k < 3; k++) {
-    double ub[5];
+    double ub[5], cx;
+    int r;
+    target_x(k, cx, r);
 #pragma unroll
     for (int j = 0; j < 5; j++) ub[j] = s_ub[k][j][lane];
-    fn[k] = weno5_combine_f64<VAR>(cx[k] - r[k], ub, S[k][0], S[k][1], S[k][2]);
+    fn[k] = weno5_combine_f64<VAR>(cx - r, ub, S[k][0], S[k][1], S[k][2]);
   }
 }
 
@@ -734,57 +773,77 @@ __device__ __forceinline__ double lag4x(double cx, int lx, int ix) {
                    : 1 * Fx[3][0] * Fx[3][1] * Fx[3][2];
 }
 
-// interp_lagr4<kD3Q27, false> for the three targets of a group, as interp_weno5_g3 does for
+// interp_lagr4<kD3Q27, MIR> for the three targets of a group, as interp_weno5_g3 does for
 // WENO5: each node of the union of their windows (at most 8 slices for s <= 1.5) loaded once,
 // each target's sum in its own node order.
-template <class SRC>
-__device__ void interp_lagr4_g3(const SRC& src, int x, const double (&cx)[3], double cy, double cz,
-                                const Tgt27g3& t, double sqTb, double (&fn)[3]) {
+template <bool MIR, class SRC>
+__device__ __forceinline__ void interp_lagr4_g3(const SRC& src, int x, double s, double cy, double cz,
+                                                const Tgt27g3& t, double sqTb, double (&fn)[3]) {
   const Grid& g = src.g;
   const int ly = floor_int(cy) - 4 / 2 + 1;
   const int lz = floor_int(cz) - 4 / 2 + 1;
-  double Fy[4][3], Fz[4][3];
-  lag4_factors(cy - ly, Fy);
-  lag4_factors(cz - lz, Fz);
-  int lx[3], w0[3];
+  // the y and z Lagrange factors wait in LDS
+  __shared__ double s_fy[12][64], s_fz[12][64];
+  const int lane = threadIdx.x & 63;
+  {
+    double F[4][3];
+    lag4_factors(cy - ly, F);
+#pragma unroll
+    for (int q = 0; q < 12; q++) s_fy[q][lane] = F[q / 3][q % 3];
+    lag4_factors(cz - lz, F);
+#pragma unroll
+    for (int q = 0; q < 12; q++) s_fz[q][lane] = F[q / 3][q % 3];
+  }
+  auto target_x = [&](int k, double& cx, int& lx) {  // departure point and window start of ex = k - 1
+    cx = (double)x - (s * (double)(k - 1) + t.u1x);
+    lx = floor_int(cx) - 4 / 2 + 1;
+  };
+  int wlo = 0, whi = 0;  // lowest and highest window start relative to x
 #pragma unroll
   for (int k = 0; k < 3; k++) {
-    lx[k] = floor_int(cx[k]) - 4 / 2 + 1;
-    w0[k] = lx[k] - x;
+    double cx;
+    int lx;
+    target_x(k, cx, lx);
+    wlo = k == 0 ? lx - x : min(wlo, lx - x);
+    whi = k == 0 ? lx - x : max(whi, lx - x);
     fn[k] = 0;
   }
-  const int dlo = min(w0[0], min(w0[1], w0[2]));
+  const int dlo = wlo;
   // (at most dlo + 7 for s <= 1.5; the bound keeps the loop finite whatever the caller passes)
-  const int dhi = min(max(w0[0], max(w0[1], w0[2])) + 3, dlo + 7);
-  for (int d = dlo; d <= dhi; d++) {
-    const int xw = wrapi(x + d, g.nx);
-    bool use[3];
-    double p[3];
+  const int dhi = min(whi + 3, dlo + 7);
+  bool use[3] = {false, false, false};
+  double p[3] = {0, 0, 0}, pf[3] = {0, 0, 0};
+  auto slice = [&](int d) {
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-      const int ix = d - w0[k];
+      double cx;
+      int lx;
+      target_x(k, cx, lx);
+      const int ix = d - (lx - x);
       use[k] = ix >= 0 && ix <= 3;
-      p[k] = use[k] ? lag4x(cx[k], lx[k], ix) : 0.0;
+      p[k] = use[k] ? lag4x(cx, lx, ix) : 0.0;
     }
-#pragma unroll 1
-    for (int a = 0; a < 4; a++) {
-      const int ya = wrapi(ly + a, g.ny);
-      const double fy0 = a == 0 ? Fy[0][0] : a == 1 ? Fy[1][0] : a == 2 ? Fy[2][0] : Fy[3][0];
-      const double fy1 = a == 0 ? Fy[0][1] : a == 1 ? Fy[1][1] : a == 2 ? Fy[2][1] : Fy[3][1];
-      const double fy2 = a == 0 ? Fy[0][2] : a == 1 ? Fy[1][2] : a == 2 ? Fy[2][2] : Fy[3][2];
-#pragma unroll 1
-      for (int b = 0; b < 4; b++) {
-        double T[3] = {0, 0, 0};
-        transfer27_g3(src, node_off(g, xw, ya, wrapi(lz + b, g.nz)), t, use, sqTb, T);
-        const double fz0 = b == 0 ? Fz[0][0] : b == 1 ? Fz[1][0] : b == 2 ? Fz[2][0] : Fz[3][0];
-        const double fz1 = b == 0 ? Fz[0][1] : b == 1 ? Fz[1][1] : b == 2 ? Fz[2][1] : Fz[3][1];
-        const double fz2 = b == 0 ? Fz[0][2] : b == 1 ? Fz[1][2] : b == 2 ? Fz[2][2] : Fz[3][2];
+  };
+  auto row = [&](int a) {
+    const double fy0 = s_fy[3 * a][lane], fy1 = s_fy[3 * a + 1][lane], fy2 = s_fy[3 * a + 2][lane];
 #pragma unroll
-        for (int k = 0; k < 3; k++)
-          if (use[k]) fn[k] += p[k] * fy0 * fy1 * fy2 * fz0 * fz1 * fz2 * T[k];
-      }
+    for (int k = 0; k < 3; k++) pf[k] = p[k] * fy0 * fy1 * fy2;
+  };
+  auto node = [&](Node27& n, int d, int a, int b) {
+    bool mx = false, my = false, mz = false;
+    if (MIR) {
+      mirror_wrap(x + d, g.nx, (g.mirror & 1) != 0, mx);
+      mirror_wrap(ly + a, g.ny, (g.mirror & 2) != 0, my);
+      mirror_wrap(lz + b, g.nz, (g.mirror & 4) != 0, mz);
     }
-  }
+    double T[3] = {0, 0, 0};
+    transfer27_g3<MIR>(n, t, use, sqTb, T, mx, my, mz);
+    const double fz0 = s_fz[3 * b][lane], fz1 = s_fz[3 * b + 1][lane], fz2 = s_fz[3 * b + 2][lane];
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+      if (use[k]) fn[k] += pf[k] * fz0 * fz1 * fz2 * T[k];
+  };
+  walk27<4, MIR>(src, x, ly, lz, dlo, dhi, slice, row, node);
 }
 
 // propagate<4> (steps.cu:986-1036): tricubic Lagrange on floor(x)-1 .. floor(x)+2.
@@ -852,88 +911,10 @@ struct F64Iter {
   int niter;
 };
 
-// f64_once for D3Q27 WENO5 (INTERP 0, 2, 4) and Lagrange-4 (1) off a line, without mirrors: the
-// targets in (ey, ez) groups of three (interp_weno5_g3, interp_lagr4_g3), each value stored as it
-// is found; then the moments summed over the stored values in population order, as calcMoments
-// does.
-template <int INTERP, class SRC>
-__device__ __forceinline__ bool f64_once_g3(const SRC& src, const NodeSrc& gsrc, double* __restrict__ fout,
-                                            int64_t cell, int x, int y, int z, bool zero, F64Iter& st,
-                                            const StepArgs& a) {
-  constexpr int VAR = INTERP == 2 ? 1 : INTERP == 4 ? 2 : 0;
-  const int64_t P = a.g.plane;
-  double* c0 = st.c0;
-  st.niter++;
-  const int niter = st.niter;
-  const double uT[4] = {c0[0], c0[1], c0[2], c0[3]};
-  const double s = sqrt(uT[3] / a.tlat);
-  bool conv = true;
-#pragma unroll 1
-  for (int gi = 0; gi < 9; gi++) {
-    const int jy = gi / 3, jz = gi % 3;
-    int idx[3];
-    Tgt27g3 t;
-    double cx[3];
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-      idx[k] = kIdx27.v[k][jy][jz];
-      const double vx = s * Lat<kD3Q27>::efc(idx[k], 0) + uT[0];
-      const Tgt27 tk = Lat<kD3Q27>::tgt(idx[k], uT);
-      t.W[k] = tk.W; t.Cx[k] = tk.Cx; t.kx[k] = tk.kx; t.wok[k] = tk.wok;
-      if (k == 0) {
-        t.u1x = tk.u1x; t.u1y = tk.u1y; t.u1z = tk.u1z; t.T1 = tk.T1;
-        t.Cy = tk.Cy; t.Cz = tk.Cz; t.ky = tk.ky; t.kz = tk.kz;
-      }
-      cx[k] = (double)x - vx;
-    }
-    const double vy = s * Lat<kD3Q27>::efc(idx[0], 1) + uT[1];
-    const double vz = s * Lat<kD3Q27>::efc(idx[0], 2) + uT[2];
-    const double cy = (double)y - vy, cz = (double)z - vz;
-    double fn[3];
-    if constexpr (INTERP == 1) interp_lagr4_g3(src, x, cx, cy, cz, t, a.sqrt_tbase, fn);
-    else interp_weno5_g3<VAR>(src, x, cx, cy, cz, t, a.sqrt_tbase, fn);
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-      const int64_t o = f64_fidx(kD3Q27, idx[k], cell, P);
-      const double fo = niter > 1 ? fout[o] : (zero ? a.w[idx[k]] * 1.0 : gsrc.f[o]);
-      if (fabs(fn[k] - fo) >= a.tol_abs + a.tol_rel * fabs(fn[k])) conv = false;
-      fout[o] = fn[k];
-    }
-  }
-  double rho = 0, m0 = 0, m1 = 0, m2 = 0, m3 = 0;
-  for (int i = 0; i < 27; i++) {
-    const double vx = s * Lat<kD3Q27>::efc(i, 0) + uT[0];
-    const double vy = s * Lat<kD3Q27>::efc(i, 1) + uT[1];
-    const double vz = s * Lat<kD3Q27>::efc(i, 2) + uT[2];
-    const double fn = fout[f64_fidx(kD3Q27, i, cell, P)];
-    rho += fn;
-    m0 += fn * vx;
-    m1 += fn * vy;
-    m2 += fn * vz;
-    m3 += fn * (vx * vx + vy * vy + vz * vz);
-  }
-  if (rho != 0) { m0 /= rho; m1 /= rho; m2 /= rho; m3 /= rho; }
-  m3 = (m3 - m0 * m0 - m1 * m1 - m2 * m2) * a.inv_dim;
-  if (m3 < 0) m3 = c0[3];
-  const double mn[4] = {m0, m1, m2, m3};
-#pragma unroll
-  for (int k = 0; k < 4; k++)
-    if (fabs(mn[k] - c0[k]) >= a.tol_abs + a.tol_rel * fabs(mn[k])) conv = false;
-  st.rho0 = rho;
-  c0[0] = m0; c0[1] = m1; c0[2] = m2; c0[3] = m3;
-  return conv;
-}
-
 // One fixed-point iteration (LBMpull, steps.cu:421-512) of one cell: true when it has converged.
 template <int LAT, int INTERP, class SRC>
 __device__ __forceinline__ bool f64_once(const SRC& src, const NodeSrc& gsrc, double* __restrict__ fout, int64_t cell,
                                          int x, int y, int z, bool zero, F64Iter& st, const StepArgs& a) {
-  if constexpr (LAT == kD3Q27 && (INTERP == 0 || INTERP == 1 || INTERP == 2 || INTERP == 4)) {
-    // the grouped path off a line, for gauges whose targets' windows lie close (s <= 1.5, not
-    // NaN); hotter or non-finite ones, one target at a time below
-    if ((a.g.ny > 1 || a.g.nz > 1) && sqrt(st.c0[3] / a.tlat) <= 1.5)
-      return f64_once_g3<INTERP>(src, gsrc, fout, cell, x, y, z, zero, st, a);
-  }
   constexpr int Q = Lat<LAT>::Q;
   const int64_t P = a.g.plane;
   double* c0 = st.c0;
@@ -1034,14 +1015,11 @@ __device__ __forceinline__ void f64_finish(double* __restrict__ fout, double* __
 // shock-bubble FP64 step, A/B on one GPU: the grouped WENO5C kernel 2.70 s at one wave per SIMD
 // (its registers spilled to AGPRs), 2.58 s at two; Lagrange-4 5.34 s -> 4.99 s.  The D1Q5 kernel
 // keeps its registers (held to two waves it would spill 1.7 KB per lane).
-template <int LAT, int INTERP, bool BUF>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LAT == kD3Q27 ? 2 : 1))) void k_step_f64(const NodeSrc gsrc, double* __restrict__ fout,
+template <int LAT, int INTERP>
+__global__ __launch_bounds__(64) void k_step_f64(const NodeSrc gsrc, double* __restrict__ fout,
                                                  double* __restrict__ mout, int* __restrict__ niter_out, Pending pend,
                                                  const StepArgs a) {
-  using Src = typename std::conditional<BUF, NodeBuf, NodeSrc>::type;
-  Src src;
-  if constexpr (BUF) src = make_nodebuf<LAT>(gsrc);
-  else src = gsrc;
+  const NodeSrc& src = gsrc;
   const Grid& g = a.g;
   int x, y, z;
   bool active = tile_cell(g, xcd_block(blockIdx.x, gridDim.x), threadIdx.x, x, y, z);
@@ -1068,76 +1046,178 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LAT == kD3Q2
   }
 }
 
-// First pass with lane refill: a wave owns `chunk` consecutive 64-cell tiles and its lanes take
-// the next unstarted cell of them whenever theirs converges or is set aside (after
-// a.pass1_iters iterations, to the pending list), instead of idling until the slowest cell of
-// their tile is done.  Each cell's arithmetic is that of k_step_f64.
-template <int LAT, int INTERP, bool BUF>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LAT == kD3Q27 ? 2 : 1))) void k_step_f64_refill(const NodeSrc gsrc, double* __restrict__ fout,
-                                                        double* __restrict__ mout, int* __restrict__ niter_out,
-                                                        Pending pend, const StepArgs a, int chunk) {
+// ---------------------------------------------------------------------------------------------
+// D3Q27 step: nine lanes per cell, lane = (ey, ez) group of three targets, seven cells per wave.
+//
+// One lane per cell (all 27 targets one after the other) left two thirds of the lanes idle behind
+// the slowest cell of their tile (the mean count is 1.3 to 5 iterations, the slowest of 64 cells
+// several times that), gave a small grid a fraction of the chip (8316 cells: 130 waves for 1024
+// SIMDs, 10 ms per step), sent the populations through global memory between iterations and needed a
+// second pass for the slow cells.  Here a cell's groups run side by side, a slot whose cell has
+// converged takes the next one, the iterate stays in LDS and the previous one in registers; the
+// lanes of a cell mostly want the same nodes, so a load touches a few cache lines.  Each value is the
+// same sequence of operations (bit for bit).
+// Per step, before and after: 33x18x14 vortex 10.0 -> 0.85 ms; 128^3 vortex 86 -> 65 ms; 256x128x128
+// shock-bubble 289 -> 181 ms; Lagrange-4 128^3 255 -> 124 ms, 100x52x46 with walls 109 -> 16.5 ms.
+// Bound by the L1: at 128^3 the VALU is busy 60-65 % of the time, the texture-address unit 56 %, with
+// the L1 stalled on pending misses for half of it; the minimum of FP64 operations (no contraction,
+// every rounding of the reference) is half of what the waves issue.
+template <int INTERP, class SRC>
+__device__ __forceinline__ void f64_group(const SRC& src, int x, int y, int z, int ey, int ez, const double (&uT)[4],
+                                          double s, const StepArgs& a, double (&fn)[3]) {
+  constexpr int VAR = INTERP == 2 ? 1 : INTERP == 4 ? 2 : 0;
+  const double cy = (double)y - (s * (double)ey + uT[1]), cz = (double)z - (s * (double)ez + uT[2]);
+  // the three together off a line, for gauges whose targets' windows lie close (s <= 1.5, not
+  // NaN); hotter or non-finite ones, one target at a time
+  if ((a.g.ny > 1 || a.g.nz > 1) && s <= 1.5) {
+    // (W and C of ex = -1 and +1 are the same up to C's sign)
+    const Tgt27 t0 = make_tgt27e(0, ey, ez, uT[0], uT[1], uT[2], uT[3]);
+    const Tgt27 t1 = make_tgt27e(1, ey, ez, uT[0], uT[1], uT[2], uT[3]);
+    Tgt27g3 t;
+    t.u1x = uT[0]; t.u1y = uT[1]; t.u1z = uT[2]; t.T1 = uT[3];
+    t.W0 = t0.W; t.W1 = t1.W; t.Cx = t1.Cx;
+    t.Cy = t0.ky ? t0.Cy : 0.0; t.Ty = t0.ky ? 0.0 : uT[3];
+    t.Cz = t0.kz ? t0.Cz : 0.0; t.Tz = t0.kz ? 0.0 : uT[3];
+    t.ky = t0.ky; t.kz = t0.kz;
+    if constexpr (INTERP == 1 || INTERP == 3) interp_lagr4_g3<INTERP == 3>(src, x, s, cy, cz, t, a.sqrt_tbase, fn);
+    else interp_weno5_g3<VAR>(src, x, s, cy, cz, t, a.sqrt_tbase, fn);
+  } else {
+#pragma unroll 1
+    for (int k = 0; k < 3; k++) {
+      const Tgt27 tk = make_tgt27e(k - 1, ey, ez, uT[0], uT[1], uT[2], uT[3]);
+      const double c = (double)x - (s * (double)(k - 1) + uT[0]);
+      double v;
+      if constexpr (INTERP == 1 || INTERP == 3) v = interp_lagr4<kD3Q27, INTERP == 3>(src, c, cy, cz, tk, a.sqrt_tbase);
+      else v = interp_weno5<kD3Q27, VAR>(src, c, cy, cz, tk, a.sqrt_tbase);
+      fn[0] = k == 0 ? v : fn[0];
+      fn[1] = k == 1 ? v : fn[1];
+      fn[2] = k == 2 ? v : fn[2];
+    }
+  }
+}
+
+template <int INTERP, bool BUF>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_step_f64_27(
+    const NodeSrc gsrc, double* __restrict__ fout, double* __restrict__ mout, int* __restrict__ niter_out,
+    const StepArgs a, int cells) {
   using Src = typename std::conditional<BUF, NodeBuf, NodeSrc>::type;
   Src src;
-  if constexpr (BUF) src = make_nodebuf<LAT>(gsrc);
+  if constexpr (BUF) src = make_nodebuf(gsrc);
   else src = gsrc;
+  __shared__ __align__(16) double s_fn[8][28];  // the iterate's populations, per cell
+  __shared__ double s_w[28];
   const Grid& g = a.g;
+  const int64_t P = g.plane;
   const int lane = threadIdx.x;
-  const int64_t ntiles = g.ntiles;
-  const int64_t t0 = xcd_block(blockIdx.x, gridDim.x) * chunk;
-  const int64_t total = (ntiles - t0 < chunk ? ntiles - t0 : chunk) * 64;  // cell slots of the chunk
-  const int stop = a.pass1_iters < a.max_iter ? a.pass1_iters : a.max_iter;
+  const int slot = lane / 9, gi = lane - 9 * slot;  // lane 63 has no cell
+  const int ey = gi / 3 - 1, ez = gi % 3 - 1;
+  constexpr uint64_t kHeads = 0x0040201008040201ull;  // lanes 0, 9, .., 54
+  if (lane < 28) s_w[lane] = lane < 27 ? a.w[lane] : 0.0;
+  const int64_t q0 = xcd_block(blockIdx.x, gridDim.x) * cells;
+  const int64_t total = g.ntiles * 64 - q0 < cells ? g.ntiles * 64 - q0 : cells;  // cell slots of the wave
   int64_t next = 0;  // first unstarted slot (the same in every lane)
-  bool active = false, zero = false;
+  bool active = false;
   int64_t cell = 0;
-  int x = 0, y = 0, z = 0;
-  F64Iter st;
+  int x = 0, y = 0, z = 0, niter = 0;
+  double c0[4] = {0, 0, 0, 1}, fo[3] = {0, 0, 0};
+  int idx[3];
+#pragma unroll
+  for (int k = 0; k < 3; k++) idx[k] = kIdx27.v[k][ey + 1][ez + 1];
   while (true) {
-    const uint64_t want = __ballot(!active);
-    const int rank = __popcll(want & ((1ull << lane) - 1ull));
-    if (!active) {
-      const int64_t slot = next + rank;
-      if (slot < total && tile_cell(g, t0 + slot / 64, (int)(slot % 64), x, y, z)) {
+    const uint64_t want = __ballot(!active) & kHeads;
+    if (!active && slot < 7) {
+      const int64_t q = next + __popcll(want & ((1ull << (9 * slot)) - 1ull));
+      if (q < total && tile_cell(g, (q0 + q) / 64, (int)((q0 + q) % 64), x, y, z)) {
         cell = cell_index(g, x, y, z);
-        zero = f64_start(gsrc, cell, a, st);
+        F64Iter st;
+        const bool zero = f64_start(gsrc, cell, a, st);
+#pragma unroll
+        for (int k = 0; k < 4; k++) c0[k] = st.c0[k];
+#pragma unroll
+        for (int k = 0; k < 3; k++) fo[k] = zero ? a.w[idx[k]] * 1.0 : gsrc.f[f64_fidx(kD3Q27, idx[k], cell, P)];
+        niter = 0;
         active = true;
       }
     }
     next += __popcll(want);
     if (__ballot(active) == 0 && next >= total) break;
-    bool pending = false;
+    const double uT[4] = {c0[0], c0[1], c0[2], c0[3]};
+    const double s = sqrt(uT[3] / a.tlat);
+    bool conv = true;
     if (active) {
-      // the loop condition of f64_iterate, one iteration per trip
-      bool done = st.niter >= stop, conv = false;
-      if (!done) {
-        conv = f64_once<LAT, INTERP>(src, gsrc, fout, cell, x, y, z, zero, st, a);
-        done = conv || st.niter >= stop;
+      double fn[3] = {0, 0, 0};
+      f64_group<INTERP>(src, x, y, z, ey, ez, uT, s, a, fn);
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        if (fabs(fn[k] - fo[k]) >= a.tol_abs + a.tol_rel * fabs(fn[k])) conv = false;
+        fo[k] = fn[k];
+        s_fn[slot][idx[k]] = fn[k];
       }
-      if (done) {
-        pending = !conv && st.niter < a.max_iter;
-        if (!pending) f64_finish<Lat<LAT>::Q>(fout, mout, niter_out, cell, st, a);
+    }
+    wave_lds_order();
+    // Cell::calcMoments: lane gi of the cell sums moment gi % 5 over the populations in order.  Its
+    // factor of population (ex, ey, ez) is wx[ex] + wy[ey] + wz[ez] with the two tables it does not
+    // need at zero (adding zero changes neither a factor nor a sum that starts from +0).
+    const int mq = gi < 5 ? gi : gi - 5;
+    double wx[3], wy[3], wz[3];
+#pragma unroll
+    for (int e = 0; e < 3; e++) {
+      const double vx = s * (double)(e - 1) + uT[0], vy = s * (double)(e - 1) + uT[1], vz = s * (double)(e - 1) + uT[2];
+      wx[e] = mq == 0 ? 1.0 : mq == 1 ? vx : mq == 4 ? vx * vx : 0.0;
+      wy[e] = mq == 2 ? vy : mq == 4 ? vy * vy : 0.0;
+      wz[e] = mq == 3 ? vz : mq == 4 ? vz * vz : 0.0;
+    }
+    double acc = 0;
+#pragma unroll
+    for (int i = 0; i < 27; i++) acc += s_fn[slot][i] * (wx[kE27[i][0] + 1] + wy[kE27[i][1] + 1] + wz[kE27[i][2] + 1]);
+    const int head = 9 * slot;
+    const double rho = __shfl(acc, head, 64);
+    if (rho != 0) acc /= rho;
+    const double m0 = __shfl(acc, head + 1, 64), m1 = __shfl(acc, head + 2, 64), m2 = __shfl(acc, head + 3, 64);
+    double m3 = __shfl(acc, head + 4, 64);
+    m3 = (m3 - m0 * m0 - m1 * m1 - m2 * m2) * a.inv_dim;
+    if (m3 < 0) m3 = uT[3];  // steps.cu:475-478
+    const double mn[4] = {m0, m1, m2, m3};
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      if (fabs(mn[k] - uT[k]) >= a.tol_abs + a.tol_rel * fabs(mn[k])) conv = false;
+    const uint64_t bad = __ballot(!conv) >> head;
+    if (active) {
+      niter++;
+#pragma unroll
+      for (int k = 0; k < 4; k++) c0[k] = mn[k];
+      if ((bad & 0x1ff) == 0 || niter >= a.max_iter) {
+        // BGK towards rho*w_i (steps.cu:557-564), two populations per lane and store
         active = false;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          const int p = gi + 9 * h;
+          if (p < 14) {
+            double f[2];
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+              f[k] = s_fn[slot][2 * p + k];
+              const double feq = rho * s_w[2 * p + k];
+              f[k] += a.dtau * (feq - f[k]);
+            }
+            if (p < 13) reinterpret_cast<double2*>(fout)[p * P + cell] = make_double2(f[0], f[1]);
+            else fout[(p * P + cell) * 2] = f[0];
+          }
+        }
+        if (gi < 5) mout[gi * P + cell] = gi == 0 ? rho : gi == 1 ? m0 : gi == 2 ? m1 : gi == 3 ? m2 : m3;
+        if (gi == 5) niter_out[cell] = niter;
       }
     }
-    bool any;
-    const int64_t e = pending_slot(pend, pending, any);
-    if (pending) {
-      pend.cell[e] = (int)cell;
-      for (int k = 0; k < 4; k++) pend.g[k * pend.cap + e] = st.c0[k];
-      pend.res[e] = st.rho0;
-      pend.meta[e] = st.niter;
-    }
+    wave_lds_order();
   }
 }
 
 // Second pass: a fixed grid of waves walks the pending list, every cell resumes its iteration
-template <int LAT, int INTERP, bool BUF>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LAT == kD3Q27 ? 2 : 1))) void k_step_f64_rest(const NodeSrc gsrc, double* __restrict__ fout,
+template <int LAT, int INTERP>
+__global__ __launch_bounds__(64) void k_step_f64_rest(const NodeSrc gsrc, double* __restrict__ fout,
                                                       double* __restrict__ mout, int* __restrict__ niter_out,
                                                       Pending pend, const StepArgs a) {
-  using Src = typename std::conditional<BUF, NodeBuf, NodeSrc>::type;
-  Src src;
-  if constexpr (BUF) src = make_nodebuf<LAT>(gsrc);
-  else src = gsrc;
+  const NodeSrc& src = gsrc;
   const Grid& g = a.g;
   const int count = *pend.count;
   for (int64_t e = (int64_t)blockIdx.x * 64 + threadIdx.x; e - threadIdx.x < count; e += (int64_t)gridDim.x * 64) {
@@ -1156,116 +1236,31 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LAT == kD3Q2
   }
 }
 
-// Second pass, one wave per unconverged cell and one lane per target population: each lane
-// interpolates its own population with the one-target code, the wave then sums the moments over
-// the populations in order from LDS (every lane the same sums), so every value is the one
-// f64_once gives, while an iteration of a slow cell costs one population's interpolation instead
-// of all of them in one lane.  The waves walk the pending list.  Used for the D3Q27 WENO5 steps
-// (384^3 shock-bubble FP64 WENO5C step 2079 -> 1948 ms); the Lagrange-4 step keeps the one-lane
-// pass, whose cells take the grouped path (2587 ms against 2712 wide).
-template <int LAT, int INTERP, bool BUF>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LAT == kD3Q27 ? 2 : 1))) void k_step_f64_rest_wide(const NodeSrc gsrc, double* __restrict__ fout,
-                                                           double* __restrict__ mout, int* __restrict__ niter_out,
-                                                           Pending pend, const StepArgs a) {
-  using Src = typename std::conditional<BUF, NodeBuf, NodeSrc>::type;
-  Src src;
-  if constexpr (BUF) src = make_nodebuf<LAT>(gsrc);
-  else src = gsrc;
-  constexpr int Q = Lat<LAT>::Q;
-  constexpr int VAR = INTERP == 2 ? 1 : INTERP == 4 ? 2 : 0;
-  __shared__ double sfn[Q];
-  const Grid& g = a.g;
-  const int64_t P = g.plane;
-  const int i = threadIdx.x;
-  const bool lane_ok = i < Q;
-  const int count = *pend.count;
-  for (int64_t e = blockIdx.x; e < count; e += gridDim.x) {
-    const int64_t cell = pend.cell[e];
-    const int x = (int)(cell % g.nx);
-    const int y = (int)((cell / g.nx) % g.ny);
-    const int z = (int)(cell / ((int64_t)g.nx * g.ny));
-    double c0[4];
-    for (int k = 0; k < 4; k++) c0[k] = pend.g[k * pend.cap + e];
-    double rho0 = pend.res[e];
-    int niter = pend.meta[e];
-    const int64_t o = lane_ok ? f64_fidx(LAT, i, cell, P) : 0;
-    while (niter < a.max_iter) {
-      niter++;
-      const double uT[4] = {c0[0], c0[1], c0[2], c0[3]};
-      const double s = sqrt(uT[3] / a.tlat);
-      bool conv_i = true;
-      if (lane_ok) {
-        const double vx = s * Lat<LAT>::efc(i, 0) + uT[0];
-        const double vy = s * Lat<LAT>::efc(i, 1) + uT[1];
-        const double vz = s * Lat<LAT>::efc(i, 2) + uT[2];
-        const typename Lat<LAT>::Tgt t = Lat<LAT>::tgt(i, uT);
-        const double cx = (double)x - vx, cy = (double)y - vy, cz = (double)z - vz;
-        const double fn = INTERP == 1   ? interp_lagr4<LAT, false>(src, cx, cy, cz, t, a.sqrt_tbase)
-                          : INTERP == 3 ? interp_lagr4<LAT, true>(src, cx, cy, cz, t, a.sqrt_tbase)
-                                        : interp_weno5<LAT, VAR>(src, cx, cy, cz, t, a.sqrt_tbase);
-        const double fo = fout[o];  // the previous iterate (the first pass ran at least one)
-        if (fabs(fn - fo) >= a.tol_abs + a.tol_rel * fabs(fn)) conv_i = false;
-        fout[o] = fn;
-        sfn[i] = fn;
-      }
-      __syncthreads();
-      // Cell::calcMoments (structs.cuh:329-330), population order, in every lane
-      double rho = 0, m0 = 0, m1 = 0, m2 = 0, m3 = 0;
-      for (int j = 0; j < Q; j++) {
-        const double vx = s * Lat<LAT>::efc(j, 0) + uT[0];
-        const double vy = s * Lat<LAT>::efc(j, 1) + uT[1];
-        const double vz = s * Lat<LAT>::efc(j, 2) + uT[2];
-        const double fn = sfn[j];
-        rho += fn;
-        m0 += fn * vx;
-        m1 += fn * vy;
-        m2 += fn * vz;
-        m3 += fn * (vx * vx + vy * vy + vz * vz);
-      }
-      __syncthreads();  // sfn is rewritten next iteration
-      if (rho != 0) { m0 /= rho; m1 /= rho; m2 /= rho; m3 /= rho; }
-      m3 = (m3 - m0 * m0 - m1 * m1 - m2 * m2) * a.inv_dim;
-      if (m3 < 0) m3 = c0[3];
-      const double mn[4] = {m0, m1, m2, m3};
-      bool conv = __ballot(!conv_i) == 0;
-#pragma unroll
-      for (int k = 0; k < 4; k++)
-        if (fabs(mn[k] - c0[k]) >= a.tol_abs + a.tol_rel * fabs(mn[k])) conv = false;
-      rho0 = rho;
-      c0[0] = m0; c0[1] = m1; c0[2] = m2; c0[3] = m3;
-      if (conv) break;
-    }
-    // f64_finish, one population per lane
-    if (lane_ok) {
-      double f = fout[o];
-      const double feq = rho0 * a.w[i];
-      f += a.dtau * (feq - f);
-      fout[o] = f;
-    }
-    if (i == 0) {
-      mout[cell] = rho0;
-      mout[P + cell] = c0[0];
-      mout[2 * P + cell] = c0[1];
-      mout[3 * P + cell] = c0[2];
-      mout[4 * P + cell] = c0[3];
-      niter_out[cell] = niter;
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------------------------
 // D3Q125: one block per cell, lane = target population (PonDstepD3Q125, steps.cu:151-250)
-
+//
+// A transfer term is W*(gx*gy*gz)*f, four FP64 operations that no two targets share: 125 x 125 x 27 of
+// them per cell and iteration are what this step is made of.  Everything else is kept off the lanes:
+//   * the basis values of a node depend on (axis, target class, source class) alone: 75 per node, 2025
+//     per cell, each formed once by one lane and read by the others from LDS (every lane used to form
+//     15 per node);
+//   * a node's populations are the same for the whole block: scalar loads put them in SGPRs, which the
+//     multiplications read directly (from LDS, 125 broadcast reads per node and wave took as long as
+//     the arithmetic).  A node beyond a mirror wall (MIR) is read permuted, through LDS;
+//   * lane q of a wave sums moment q % 5 over the populations in order (every lane used to sum all five).
+// 40^3 turbulence 20.1 -> 12.4 ms per step, 64^3 82 -> 51 ms; the VALU is busy 94 % of the time, 83 % of
+// its instructions being the terms.
+template <bool MIR>
 __global__ __launch_bounds__(128) void k_step_q125_f64(const double* __restrict__ fin, const double* __restrict__ min,
-                                                       const unsigned char* __restrict__ okin,
                                                        double* __restrict__ fout, double* __restrict__ mout,
                                                        int* __restrict__ niter_out, const StepArgs a) {
   constexpr int Q = 125;
-  __shared__ double sf[27][Q];   // fixed neighbourhood populations (cfix, steps.cu:150)
-  __shared__ double sg[27][4];   // their gauges
-  __shared__ double snew[Q];     // cnew.f
+  typedef const __attribute__((address_space(4))) double ConstD;
+  __shared__ double sf[MIR ? Q : 1];      // MIR: populations of a mirrored node
+  __shared__ double sg[27][4];            // the nodes' gauges, the temperature as sqrts(T/1.0)
+  __shared__ double sb[27][76];           // basis values g[axis][target class][source class]
+  __shared__ double snew[Q];              // cnew.f
   __shared__ int sflag[2];
-  __shared__ int sok[27];        // node populations finite and below 2^200
   const Grid& g = a.g;
   const int64_t P = g.plane;
   const int64_t cell = xcd_block(blockIdx.x, gridDim.x);
@@ -1274,23 +1269,19 @@ __global__ __launch_bounds__(128) void k_step_q125_f64(const double* __restrict_
   const int x = (int)(cell % g.nx);
   const int y = (int)((cell / g.nx) % g.ny);
   const int z = (int)(cell / ((int64_t)g.nx * g.ny));
-  for (int n = 0; n < 27; n++) {
-    // mirror boundaries (steps.cu:163-190): a node beyond a mirrored face is the mirror image of
-    // the cell inside, population k read from the mirrored velocity, the axis velocity negated
+  // mirror boundaries (steps.cu:163-190): a node beyond a mirrored face is the mirror image of
+  // the cell inside, population k read from the mirrored velocity, the axis velocity negated
+  auto node_cell = [&](int n, bool& rx, bool& ry, bool& rz) {
+    const int px = mirror_wrap(x - 1 + n / 9, g.nx, MIR && (g.mirror & 1) != 0, rx);
+    const int py = mirror_wrap(y - 1 + (n / 3) % 3, g.ny, MIR && (g.mirror & 2) != 0, ry);
+    const int pz = mirror_wrap(z - 1 + n % 3, g.nz, MIR && (g.mirror & 4) != 0, rz);
+    return cell_index(g, px, py, pz);
+  };
+  if (k < 108) {
+    const int n = k >> 2, d = k & 3;
     bool rx, ry, rz;
-    const int px = mirror_wrap(x - 1 + n / 9, g.nx, (g.mirror & 1) != 0, rx);
-    const int py = mirror_wrap(y - 1 + (n / 3) % 3, g.ny, (g.mirror & 2) != 0, ry);
-    const int pz = mirror_wrap(z - 1 + n % 3, g.nz, (g.mirror & 4) != 0, rz);
-    const int64_t c = cell_index(g, px, py, pz);
-    const int kq = lane_ok ? k : 0;  // lanes 125..127 hold no population
-    const int kx = kq / 25, ky = (kq / 5) % 5, kz = kq % 5;
-    const int kl = 25 * (rx ? kMir5[kx] : kx) + 5 * (ry ? kMir5[ky] : ky) + (rz ? kMir5[kz] : kz);
-    if (lane_ok) sf[n][k] = fin[f64_fidx(kD3Q125, kl, c, P)];
-    if (k < 4) {
-      const double v = min[(int64_t)(k + 1) * P + c];
-      sg[n][k] = (k == 0 && rx) || (k == 1 && ry) || (k == 2 && rz) ? -v : v;
-    }
-    if (k == 4) sok[n] = okin[c];
+    const double v = min[(int64_t)(d + 1) * P + node_cell(n, rx, ry, rz)];
+    sg[n][d] = d == 3 ? sqrts_d(v / 1.0) : (d == 0 && rx) || (d == 1 && ry) || (d == 2 && rz) ? -v : v;
   }
   double rho0 = min[cell], c0[4] = {min[P + cell], min[2 * P + cell], min[3 * P + cell], min[4 * P + cell]};
   const bool zero = rho0 == 0 && c0[0] == 0 && c0[1] == 0 && c0[2] == 0 && c0[3] == 0;
@@ -1309,92 +1300,107 @@ __global__ __launch_bounds__(128) void k_step_q125_f64(const double* __restrict_
     // target constants (structs.cuh:397-416)
     const double S1 = sqrts_d(uT[3] / 1.0);
     const double e1_to = kEc1 * S1, e2_to = kEc2 * S1;
+    // basis values of every node: entry (d, X, j) is the product of the four factors b - c over the
+    // target nodes c other than X's, in the cyclic order (X+1..X+4)%5 of structs.cuh:432-434, with
+    // b - c as b + {-0.0, -e1_to, +e1_to, -e2_to, +e2_to}[c] (b + (-0.0) == b exactly)
+    for (int i = k; i < 27 * 75; i += 128) {
+      const int n = i / 75, r = i - 75 * n, d = r / 25, Xi = (r / 5) % 5, j = r % 5;
+      const double e = j == 0 ? 0.0 : j == 1 ? kEc1 : j == 2 ? -kEc1 : j == 3 ? kEc2 : -kEc2;
+      const double u = d == 0 ? uT[0] : d == 1 ? uT[1] : uT[2];
+      const double b = (sg[n][d] - u) + e * sg[n][3];
+      double f[4];
+#pragma unroll
+      for (int mm = 1; mm <= 4; mm++) {
+        const int c = (Xi + mm) % 5;
+        f[mm - 1] = b + (c == 0 ? -0.0 : c == 1 ? -e1_to : c == 2 ? e1_to : c == 3 ? -e2_to : e2_to);
+      }
+      sb[n][r] = f[0] * f[1] * f[2] * f[3];
+    }
     double wv[3];
 #pragma unroll
     for (int d = 0; d < 3; d++) {
       const double en = kA5[X[d]];
-      if (en == 0) wv[d] = 1. / (e1_to * e1_to * e2_to * e2_to);
-      else if (fabs(en) == kEc1) wv[d] = 1. / (2 * e1_to * e1_to * (e1_to * e1_to - e2_to * e2_to));
-      else wv[d] = 1. / (2 * e2_to * e2_to * (e2_to * e2_to - e1_to * e1_to));
+      const double den = en == 0           ? e1_to * e1_to * e2_to * e2_to
+                         : fabs(en) == kEc1 ? 2 * e1_to * e1_to * (e1_to * e1_to - e2_to * e2_to)
+                                            : 2 * e2_to * e2_to * (e2_to * e2_to - e1_to * e1_to);
+      wv[d] = 1. / den;
     }
     const double W = wv[0] * wv[1] * wv[2];
-    const bool wok = fabs(W) < kSafe;
     const double vk[3] = {s * kA5[X[0]] + uT[0], s * kA5[X[1]] + uT[1], s * kA5[X[2]] + uT[2]};
     const double sh[3] = {((double)x - vk[0]) - (double)(x - 1), ((double)y - vk[1]) - (double)(y - 1),
                           ((double)z - vk[2]) - (double)(z - 1)};
-    double Fx[3][2], Fy[3][2], Fz[3][2];
-    lag3_factors(sh[0], Fx);
-    lag3_factors(sh[1], Fy);
-    lag3_factors(sh[2], Fz);
-    // per-lane offsets of the four factors of the target's basis polynomial, in the cyclic
-    // order (X+1..X+4)%5 of structs.cuh:432-434: factor m is b + off[(X+m)%5] with
-    // off = {-0.0, -e1_to, +e1_to, -e2_to, +e2_to} (b - c == b + (-c) and b + (-0.0) == b exactly)
-    double off[3][4];
-#pragma unroll
-    for (int d = 0; d < 3; d++)
-#pragma unroll
-      for (int mm = 1; mm <= 4; mm++) {
-        const int c = (X[d] + mm) % 5;
-        off[d][mm - 1] = c == 0 ? -0.0 : c == 1 ? -e1_to : c == 2 ? e1_to : c == 3 ? -e2_to : e2_to;
-      }
+    __syncthreads();
     double fpr = 0;
+#pragma unroll 1
     for (int n = 0; n < 27; n++) {
-      const double S0 = sqrts_d(sg[n][3] / 1.0);
-      double gb[3][5];
-      bool safe = wok && sok[n] != 0;
+      bool rx, ry, rz;
+      const int64_t c = node_cell(n, rx, ry, rz);
+      ConstD* rec = (ConstD*)(uintptr_t)(fin + c * kF64Q125Doubles);
+      const double *bx = &sb[n][5 * X[0]], *by = &sb[n][25 + 5 * X[1]], *bz = &sb[n][50 + 5 * X[2]];
+      double gy[5], gz[5];
 #pragma unroll
-      for (int d = 0; d < 3; d++) {
-        const double du = sg[n][d] - uT[d];
+      for (int j = 0; j < 5; j++) { gy[j] = by[j]; gz[j] = bz[j]; }
+      auto terms = [&](auto f) {
+        double fnew = 0;
 #pragma unroll
-        for (int j = 0; j < 5; j++) {
-          const double b = du + kA5[j] * S0;
-          gb[d][j] = (b + off[d][0]) * (b + off[d][1]) * (b + off[d][2]) * (b + off[d][3]);
-          safe = safe && fabs(gb[d][j]) < kSafe;
+        for (int jx = 0; jx < 5; jx++) {
+          const double gx = bx[jx];
+#pragma unroll
+          for (int jy = 0; jy < 5; jy++) {
+            const double gxy = gx * gy[jy];
+#pragma unroll
+            for (int jz = 0; jz < 5; jz++) fnew += W * (gxy * gz[jz]) * f[25 * jx + 5 * jy + jz];
+          }
         }
-      }
-      double fnew = 0;
-      if (safe) {
-        // every term is finite: |W|,|gx|,|gy|,|gz|,|f| < 2^200
-#pragma unroll
-        for (int jx = 0; jx < 5; jx++)
-#pragma unroll
-          for (int jy = 0; jy < 5; jy++) {
-            const double gxy = gb[0][jx] * gb[1][jy];
-#pragma unroll
-            for (int jz = 0; jz < 5; jz++) fnew += W * (gxy * gb[2][jz]) * sf[n][25 * jx + 5 * jy + jz];
+        if (!finite_d(fnew)) {
+          // a non-finite term: the loop again with such terms dropped (as in terms27)
+          fnew = 0;
+#pragma unroll 1
+          for (int i = 0; i < Q; i++) {
+            const double gxy = bx[i / 25] * by[(i / 5) % 5];
+            const double fadd = W * (gxy * bz[i % 5]) * f[i];
+            if (finite_d(fadd)) fnew += fadd;
           }
+        }
+        return fnew;
+      };
+      double fnew;
+      if (MIR && (rx || ry || rz)) {  // (the same in the whole block)
+        const int kl = 25 * (rx ? kMir5[X[0]] : X[0]) + 5 * (ry ? kMir5[X[1]] : X[1]) + (rz ? kMir5[X[2]] : X[2]);
+        __syncthreads();
+        if (lane_ok) sf[MIR ? k : 0] = fin[c * kF64Q125Doubles + kl];
+        __syncthreads();
+        fnew = terms((const double*)sf);
       } else {
-#pragma unroll
-        for (int jx = 0; jx < 5; jx++)
-#pragma unroll
-          for (int jy = 0; jy < 5; jy++) {
-            const double gxy = gb[0][jx] * gb[1][jy];
-#pragma unroll
-            for (int jz = 0; jz < 5; jz++) {
-              const double fadd = W * (gxy * gb[2][jz]) * sf[n][25 * jx + 5 * jy + jz];
-              if (finite_d(fadd)) fnew += fadd;
-            }
-          }
+        fnew = terms(rec);
       }
-      const int ia = n / 9, ib = (n / 3) % 3, ic = n % 3;
-      fpr += 1 * Fx[ia][0] * Fx[ia][1] * Fy[ib][0] * Fy[ib][1] * Fz[ic][0] * Fz[ic][1] * fnew;
+      double Fx[2], Fy[2], Fz[2];
+      lag3_row(sh[0], n / 9, Fx);
+      lag3_row(sh[1], (n / 3) % 3, Fy);
+      lag3_row(sh[2], n % 3, Fz);
+      fpr += 1 * Fx[0] * Fx[1] * Fy[0] * Fy[1] * Fz[0] * Fz[1] * fnew;
     }
     if (lane_ok) snew[k] = fpr;
     __syncthreads();
-    // Cell::calcMoments on the shared cnew, serial in population order (every lane, same result)
-    double rho = 0, m0 = 0, m1 = 0, m2 = 0, m3 = 0;
-    for (int i = 0; i < Q; i++) {
-      const double fi = snew[i];
-      const double vx = s * kA5[i / 25] + uT[0];
-      const double vy = s * kA5[(i / 5) % 5] + uT[1];
-      const double vz = s * kA5[i % 5] + uT[2];
-      rho += fi;
-      m0 += fi * vx;
-      m1 += fi * vy;
-      m2 += fi * vz;
-      m3 += fi * (vx * vx + vy * vy + vz * vz);
+    // Cell::calcMoments on the shared cnew in population order, one moment per lane: the factor of
+    // population (ix, iy, iz) is wx[ix] + wy[iy] + wz[iz], the tables a lane does not need at zero
+    // (as in k_step_f64_27)
+    const int mq = (k & 63) % 5;
+    double wx[5], wy[5], wz[5];
+#pragma unroll
+    for (int e = 0; e < 5; e++) {
+      const double vx = s * kA5[e] + uT[0], vy = s * kA5[e] + uT[1], vz = s * kA5[e] + uT[2];
+      wx[e] = mq == 0 ? 1.0 : mq == 1 ? vx : mq == 4 ? vx * vx : 0.0;
+      wy[e] = mq == 2 ? vy : mq == 4 ? vy * vy : 0.0;
+      wz[e] = mq == 3 ? vz : mq == 4 ? vz * vz : 0.0;
     }
-    if (rho != 0) { m0 /= rho; m1 /= rho; m2 /= rho; m3 /= rho; }
+    double acc = 0;
+#pragma unroll
+    for (int i = 0; i < Q; i++) acc += snew[i] * (wx[i / 25] + wy[(i / 5) % 5] + wz[i % 5]);
+    const double rho = __shfl(acc, 0, 64);
+    if (rho != 0) acc /= rho;
+    const double m0 = __shfl(acc, 1, 64), m1 = __shfl(acc, 2, 64), m2 = __shfl(acc, 3, 64);
+    double m3 = __shfl(acc, 4, 64);
     m3 = (m3 - m0 * m0 - m1 * m1 - m2 * m2) * a.inv_dim;
     if (m3 < 0) m3 = c0[3];
     const double mn[4] = {m0, m1, m2, m3};
@@ -1410,7 +1416,7 @@ __global__ __launch_bounds__(128) void k_step_q125_f64(const double* __restrict_
     rho0 = rho;
     c0[0] = m0; c0[1] = m1; c0[2] = m2; c0[3] = m3;
     f0 = fpr;
-    __syncthreads();  // sflag and snew are rewritten next iteration
+    __syncthreads();  // sflag, snew and sb are rewritten next iteration
     if (all_conv) break;
   }
   if (lane_ok) {
@@ -1632,49 +1638,25 @@ __global__ __launch_bounds__(64) void k_step_line(const double* __restrict__ fin
 // ---------------------------------------------------------------------------------------------
 // host-side launchers
 
-// per-step node data: sqrt(|T|)*sign(T) and the "populations finite and below 2^200" flag
-template <int Q>
-__global__ void k_node_prep(const double* __restrict__ f, const double* __restrict__ m, double* __restrict__ P,
-                            unsigned char* __restrict__ ok, int64_t n, int64_t plane) {
+// per-step node data of the load state: D3Q27 the gauge record (ux, uy, uz, P) of every cell, 32
+// bytes, D1Q5 the plane of P, with P = sqrt(|T|)*sign(T)
+__global__ void k_node_prep(const double* __restrict__ m, double* __restrict__ P, int64_t n, int64_t plane,
+                            bool record) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= n) return;
-  const double T = m[4 * plane + c];
-  const double Pc = sqrt(fabs(T)) * (double)isign_d(T);
-  if (Q == 27) {
-    // gauge record (ux, uy, uz, P) of the cell, 32 bytes
+  const double Pc = sqrts_d(m[4 * plane + c]);
+  if (record) {
     reinterpret_cast<double2*>(P)[2 * c] = make_double2(m[plane + c], m[2 * plane + c]);
     reinterpret_cast<double2*>(P)[2 * c + 1] = make_double2(m[3 * plane + c], Pc);
   } else {
     P[c] = Pc;
   }
-  bool good = true;
-  for (int i = 0; i < Q; i++)
-    good = good && fabs(f[f64_fidx(Q == 27 ? kD3Q27 : Q == 5 ? kD1Q5 : kD3Q125, i, c, plane)]) < kSafe;
-  ok[c] = good ? 1 : 0;
 }
 
-hipError_t launch_node_prep(int lattice, const double* f, const double* m, double* P, unsigned char* ok, int64_t n,
-                            int64_t plane, hipStream_t st) {
-  const unsigned blocks = (unsigned)((n + 255) / 256);
-  if (lattice == kD3Q27)
-    hipLaunchKernelGGL(k_node_prep<27>, dim3(blocks), dim3(256), 0, st, f, m, P, ok, n, plane);
-  else if (lattice == kD1Q5)
-    hipLaunchKernelGGL(k_node_prep<5>, dim3(blocks), dim3(256), 0, st, f, m, P, ok, n, plane);
-  else
-    hipLaunchKernelGGL(k_node_prep<125>, dim3(blocks), dim3(256), 0, st, f, m, P, ok, n, plane);
+hipError_t launch_node_prep(int lattice, const double* m, double* P, int64_t n, int64_t plane, hipStream_t st) {
+  hipLaunchKernelGGL(k_node_prep, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, m, P, n, plane,
+                     lattice == kD3Q27);
   return hipGetLastError();
-}
-
-// the second pass: wide for the D3Q27 WENO5 steps, one lane per cell otherwise
-template <int LAT, int INTERP, bool BUF>
-static void launch_rest(unsigned blocks2, hipStream_t st, const NodeSrc& src, double* fout, double* mout, int* niter,
-                        const Pending& pend, const StepArgs& a) {
-  if constexpr (LAT == kD3Q27 && (INTERP == 0 || INTERP == 2 || INTERP == 4))
-    hipLaunchKernelGGL((k_step_f64_rest_wide<LAT, INTERP, BUF>), dim3(blocks2), dim3(64), 0, st, src, fout, mout, niter,
-                       pend, a);
-  else
-    hipLaunchKernelGGL((k_step_f64_rest<LAT, INTERP, BUF>), dim3(blocks2), dim3(64), 0, st, src, fout, mout, niter,
-                       pend, a);
 }
 
 // The line kernel does 3-4 times the work per cell and iteration of the one-lane kernel (lanes of a
@@ -1687,77 +1669,66 @@ bool f64_line_step(int lattice, int interp, const Grid& g) {
 }
 
 hipError_t launch_step_f64(int lattice, int interp, const double* fin, const double* min, const double* Pin,
-                           const unsigned char* okin, double* fout, double* mout, int* niter, const Pending& pend,
-                           const StepArgs& a, hipStream_t st) {
+                           double* fout, double* mout, int* niter, const Pending& pend, const StepArgs& a,
+                           hipStream_t st) {
   if (lattice == kD3Q125) {
-    const int64_t blocks = a.g.n;
-    hipLaunchKernelGGL(k_step_q125_f64, dim3((unsigned)blocks), dim3(128), 0, st, fin, min, okin, fout, mout, niter,
-                       a);
+    const dim3 nb((unsigned)a.g.n), nt(128);
+    if (a.g.mirror) hipLaunchKernelGGL(k_step_q125_f64<true>, nb, nt, 0, st, fin, min, fout, mout, niter, a);
+    else hipLaunchKernelGGL(k_step_q125_f64<false>, nb, nt, 0, st, fin, min, fout, mout, niter, a);
     return hipGetLastError();
   }
   // kernel codes: 0 WENO5 as written, 1 Lagrange-4, 2 WENO5 centred, 3 Lagrange-4 with mirror
   // boundaries (its own instantiation, so the periodic kernels carry none of the mirror code),
   // 4 the generic WENO5.  interp is pond_interp (POND_WENO5G = 3).
   const int code = interp == 3 ? 4 : (interp == 1 && a.g.mirror) ? 3 : interp;
+  const dim3 nt(64);
   if (f64_line_step(lattice, interp, a.g)) {
     // on a line the centred and as-written WENO5 coincide
-    const dim3 nb((unsigned)((a.g.n + 1) / 2)), nt(64);
+    const dim3 nb((unsigned)((a.g.n + 1) / 2));
     if (code == 1) hipLaunchKernelGGL(k_step_line<1>, nb, nt, 0, st, fin, min, fout, mout, niter, a);
     else if (code == 3) hipLaunchKernelGGL(k_step_line<3>, nb, nt, 0, st, fin, min, fout, mout, niter, a);
     else if (code == 4) hipLaunchKernelGGL(k_step_line<4>, nb, nt, 0, st, fin, min, fout, mout, niter, a);
     else hipLaunchKernelGGL(k_step_line<0>, nb, nt, 0, st, fin, min, fout, mout, niter, a);
     return hipGetLastError();
   }
-  const unsigned blocks = (unsigned)(a.g.ntiles);
-  const NodeSrc src{fin, min, Pin, okin, a.g};
-  // buffer-resource loads while nine FP64 planes (D1Q5) or four pair planes (D3Q27) fit a 32-bit
-  // offset
-  const bool buf = (uint64_t)a.g.plane * 8u * (lattice == kD3Q27 ? 8u : (uint64_t)kPlanesPerRsrc64) <= 0xffffffffull &&
-                   !a.global_loads;
-  hipLaunchKernelGGL(k_zero_count, dim3(1), dim3(64), 0, st, pend.count);
-  const int64_t w2 = (a.g.n + 63) / 64;
-  const unsigned blocks2 = (unsigned)(w2 < 16384 ? w2 : 16384);
-#define POND_LAUNCH(L, I, B)                                                                                     \
+  const NodeSrc src{fin, min, Pin, a.g};
+  if (lattice == kD3Q27) {
+    // buffer-resource loads while four pair planes fit a 32-bit offset
+    const bool buf = (uint64_t)a.g.plane * 8u * 8u <= 0xffffffffull && !a.global_loads;
+    // Cells per wave: one per slot, or two where that still leaves several waves for every SIMD (a slot
+    // then fills the tail of a slow neighbour).  ms per step with 7, 14, 28 cells: 33x18x14 0.85,
+    // 1.09, 1.7; 128^3 vortex 64.9, 65.8, 68; 256x128x128 shock-bubble 183.7, 180.7, 182.
+    const int64_t slots = a.g.ntiles * 64;
+    int64_t cells = a.refill_chunk > 0 ? 64ll * a.refill_chunk : a.refill_chunk == 0 ? 64 : a.g.n < (1 << 20) ? 7 : 14;
+    if (cells > slots) cells = slots;
+    const dim3 nb((unsigned)((slots + cells - 1) / cells));
+#define POND_LAUNCH(I)                                                                                           \
   do {                                                                                                           \
-    hipLaunchKernelGGL((k_step_f64<L, I, B>), dim3(blocks), dim3(64), 0, st, src, fout, mout, niter, pend, a);   \
-    launch_rest<L, I, B>(blocks2, st, src, fout, mout, niter, pend, a);                                          \
+    if (buf) hipLaunchKernelGGL((k_step_f64_27<I, true>), nb, nt, 0, st, src, fout, mout, niter, a, (int)cells);   \
+    else hipLaunchKernelGGL((k_step_f64_27<I, false>), nb, nt, 0, st, src, fout, mout, niter, a, (int)cells);      \
   } while (0)
-#define POND_LAUNCH_R(L, I)                                                                                      \
-  do {                                                                                                           \
-    const unsigned w = (unsigned)(((int64_t)blocks + a.refill_chunk - 1) / a.refill_chunk);                       \
-    hipLaunchKernelGGL((k_step_f64_refill<L, I, true>), dim3(w), dim3(64), 0, st, src, fout, mout, niter, pend, a, \
-                       a.refill_chunk);                                                                          \
-    launch_rest<L, I, true>(blocks2, st, src, fout, mout, niter, pend, a);                                       \
-  } while (0)
-  if (lattice == kD3Q27 && buf && a.refill_chunk > 0) {
-    if (code == 0) POND_LAUNCH_R(kD3Q27, 0);
-    else if (code == 1) POND_LAUNCH_R(kD3Q27, 1);
-    else if (code == 3) POND_LAUNCH_R(kD3Q27, 3);
-    else if (code == 4) POND_LAUNCH_R(kD3Q27, 4);
-    else POND_LAUNCH_R(kD3Q27, 2);
-  } else if (lattice == kD3Q27) {
-    if (buf) {
-      if (code == 0) POND_LAUNCH(kD3Q27, 0, true);
-      else if (code == 1) POND_LAUNCH(kD3Q27, 1, true);
-      else if (code == 3) POND_LAUNCH(kD3Q27, 3, true);
-      else if (code == 4) POND_LAUNCH(kD3Q27, 4, true);
-      else POND_LAUNCH(kD3Q27, 2, true);
-    } else {
-      if (code == 0) POND_LAUNCH(kD3Q27, 0, false);
-      else if (code == 1) POND_LAUNCH(kD3Q27, 1, false);
-      else if (code == 3) POND_LAUNCH(kD3Q27, 3, false);
-      else if (code == 4) POND_LAUNCH(kD3Q27, 4, false);
-      else POND_LAUNCH(kD3Q27, 2, false);
-    }
-  } else {
-    // on a line (Ny = Nz = 1) the centred and as-written WENO5 coincide
-    if (code == 1) POND_LAUNCH(kD1Q5, 1, false);
-    else if (code == 3) POND_LAUNCH(kD1Q5, 3, false);
-    else if (code == 4) POND_LAUNCH(kD1Q5, 4, false);
-    else POND_LAUNCH(kD1Q5, 0, false);
-  }
+    if (code == 0) POND_LAUNCH(0);
+    else if (code == 1) POND_LAUNCH(1);
+    else if (code == 3) POND_LAUNCH(3);
+    else if (code == 4) POND_LAUNCH(4);
+    else POND_LAUNCH(2);
 #undef POND_LAUNCH
-#undef POND_LAUNCH_R
+    return hipGetLastError();
+  }
+  // D1Q5 off a line and long Lagrange-4 lines: one lane per cell, two passes
+  hipLaunchKernelGGL(k_zero_count, dim3(1), nt, 0, st, pend.count);
+  const int64_t w2 = (a.g.n + 63) / 64;
+  const dim3 nb1((unsigned)a.g.ntiles), nb2((unsigned)(w2 < 16384 ? w2 : 16384));
+#define POND_LAUNCH(I)                                                                                           \
+  do {                                                                                                           \
+    hipLaunchKernelGGL((k_step_f64<kD1Q5, I>), nb1, nt, 0, st, src, fout, mout, niter, pend, a);                  \
+    hipLaunchKernelGGL((k_step_f64_rest<kD1Q5, I>), nb2, nt, 0, st, src, fout, mout, niter, pend, a);             \
+  } while (0)
+  if (code == 1) POND_LAUNCH(1);
+  else if (code == 3) POND_LAUNCH(3);
+  else if (code == 4) POND_LAUNCH(4);
+  else POND_LAUNCH(0);
+#undef POND_LAUNCH
   return hipGetLastError();
 }
 

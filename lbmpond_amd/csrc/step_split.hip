@@ -1460,14 +1460,6 @@ __device__ __forceinline__ double node5(int m, double e1, double e2) {
   return m == 0 ? 0.0 : m == 1 ? e1 : m == 2 ? -e1 : m == 3 ? e2 : -e2;
 }
 
-// orders this wave's LDS writes before its following reads and its reads before following writes
-// (a wave's LDS operations execute in order; this holds the compiler to it)
-__device__ __forceinline__ void wave_lds_order() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // v of the lane a DPP control takes it from (a cross-lane move in the VALU, no LDS round trip)
 template <int CTRL>
 __device__ __forceinline__ double dpp_d(double v) {
