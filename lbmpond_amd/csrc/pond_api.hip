@@ -286,11 +286,10 @@ void pond_params_default(pond_params* p, int lattice) {
   // residual; 1e-7 converges reliably above it
   p->split_tol_rel = 1e-7;
   p->split_tol_abs = 1e-12;
-  // Row patches (-1: chosen in pond_create).  384^3 shock-bubble D3Q27: the FP64 step (pair
-  // planes, lane refill) 4.10 s in row order, 3.13 s with 4x4 patches, 3.14 s with 8x8; the split
-  // step with its node loads one step ahead, WENO5C 261 ms in row order, 161.4 ms with 4x4
-  // patches, 157.0 with 8x8, 157.8 with 6x6, 157.2 with 12x12, 158.2 with 16x16; Lagrange-4
-  // 422, 225.2, 226.2 and 232.2 ms (row order, 4, 8, 16).
+  // Row patches (-1: chosen in pond_create).  Split step, 256^3: WENO5C vortex 39.5, 39.5, 39.7 ms with
+  // 4x4, 8x8, 16x16 patches, shock-bubble 71.9, 69.4, 69.8; Lagrange-4 shock-bubble 106.8, 102.5,
+  // 101.9.  (384^3 shock-bubble with one lane per cell: in row order 261 ms, with 8x8 patches 157;
+  // the FP64 step 4.10 s and 3.13 s.)
   p->tile_patch = -1;
   p->refill_chunk = -1;
   p->pass1_iters = -1;
@@ -434,22 +433,7 @@ pond_status pond_create(const pond_params* p, pond_ctx** out) {
     }
     SplitArgs& sa = ctx->sargs;
     sa.pass1_iters = a.pass1_iters;
-    // lane refill over chunks of 64-cell tiles.  Measured on the 384^3 shock-bubble, split step
-    // ms, with paired x-slice loads: one tile 1065, chunks of 2 tiles 805, 3 976, 4 775-778, 6
-    // 763, 8 840, 12 910 (one slice per load and one tile per wave: 1025).  Larger chunks keep
-    // more lanes busy but spread the active cells of a wave over more rows, so its loads touch
-    // more cache lines.  With the current node loop (gather-bound): 3 319, 4 293, 5 305, 6 279,
-    // 7 321, 8 317, 9 328, 12 321.  Six tiles are one whole x row at 384^3: with row patches the
-    // tiles are 64-cell row segments, nx/64 per row, so chunks of whole rows let the waves
-    // resident on an XCD cover a compact patch of rows (traffic from beyond L2 per launch:
-    // 1.23 TB with chunks of 4 tiles, 0.50 TB with 6; at 256^3, 4 tiles per row: chunks of 4
-    // 113 ms, 3 128, 6 127, 8 124).  Default: whole rows, at least 4 tiles.
-    sa.refill_chunk = 4;
-    if (g.rp > 0) {
-      const int wpr = g.nx / 64;
-      sa.refill_chunk = wpr * ((4 + wpr - 1) / wpr);
-    }
-    if (p->refill_chunk >= 0) sa.refill_chunk = p->refill_chunk;
+    sa.refill_chunk = p->refill_chunk;
     sa.learned_trust = (float)p->learned_trust;
     sa.g = g;
     sa.dtau = p->dtau;

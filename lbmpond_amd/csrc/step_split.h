@@ -13,9 +13,9 @@ struct SplitArgs {
   double sqrt_tbase;
   double tlat;
   double inv_dim;
-  int pass1_iters;  // iterations of the first pass of the D3Q27 step (the rest go to the second)
+  int pass1_iters;  // D3Q27 WENO5 as written: iterations of the first pass (the rest go to the second)
   float learned_trust;  // largest predicted change (thermal units) taken as a start
-  int refill_chunk;     // D3Q27 WENO5C single pass: 64-cell tiles per wave with lane refill (0: one tile per wave)
+  int refill_chunk;     // D3Q27: 64-cell tiles per wave (0: one; -1: the step's own choice of cells per wave)
   float w[kQmax];
 };
 

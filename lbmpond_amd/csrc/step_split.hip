@@ -531,8 +531,8 @@ __device__ void interp_group_weno5c(const NodeSrcF& src, int x, int y, int z, do
 // of a window are kept.  Each target's value is stored to fout (its population slot of this
 // cell).  Windows or rows far apart (absurd gauges) fall back to
 // interp_group_weno5c per group, which bounds the loops whatever the gauge.
-__device__ void interp_pass_weno5c(const NodeSrcF& src, int x, int y, int z, double s, const double gc[4], int ez,
-                                   float sqTb, float* __restrict__ fout, int64_t cell, int64_t P) {
+__device__ __forceinline__ void interp_pass_weno5c(const NodeSrcF& src, int x, int y, int z, double s,
+                                                   const double gc[4], int ez, float sqTb, float* o) {
   const Grid& g = src.g;
   const float u1x = (float)gc[0], u1y = (float)gc[1], u1z = (float)gc[2];
   const float u1xl = (float)(gc[0] - (double)u1x), u1yl = (float)(gc[1] - (double)u1y),
@@ -575,7 +575,7 @@ __device__ void interp_pass_weno5c(const NodeSrcF& src, int x, int y, int z, dou
       float f3[3];
       interp_group_weno5c(src, x, y, z, s, gc, e - 1, ez, sqTb, f3);
 #pragma unroll
-      for (int t = 0; t < 3; t++) fout[split27_fidx(kIdx27.v[t][e][ez + 1], cell, P)] = f3[t];
+      for (int t = 0; t < 3; t++) o[3 * e + t] = f3[t];
     }
     return;
   }
@@ -736,7 +736,7 @@ __device__ void interp_pass_weno5c(const NodeSrcF& src, int x, int y, int z, dou
       for (int j = 0; j < 5; j++) ubt[j] = s_ub[(e * 3 + t) * 5 + j][lane] * wt;
 #pragma unroll
       for (int k = 0; k < 3; k++) S[k] = Sk[e][t][k] * wt;
-      fout[split27_fidx(kIdx27.v[t][e][ez + 1], cell, P)] = weno5_combine(c[t], ubt, S);
+      o[3 * e + t] = weno5_combine(c[t], ubt, S);
     }
   }
 }
@@ -811,8 +811,8 @@ constexpr int kLearnedBudget = 12;
 // a mirrored face is the mirror image of the cell inside).  Windows or rows far apart (absurd
 // gauges) fall back to interp_lagr4f per target.  Each target's value is stored to fout.
 template <bool MIR>
-__device__ void interp_pass_lagr4(const NodeSrcF& src, int x, int y, int z, double s, const double gc[4], int ez,
-                                  float sqTb, float* __restrict__ fout, int64_t cell, int64_t P) {
+__device__ __forceinline__ void interp_pass_lagr4(const NodeSrcF& src, int x, int y, int z, double s,
+                                                  const double gc[4], int ez, float sqTb, float* o) {
   const Grid& g = src.g;
   const float u1x = (float)gc[0], u1y = (float)gc[1], u1z = (float)gc[2];
   const float u1xl = (float)(gc[0] - (double)u1x), u1yl = (float)(gc[1] - (double)u1y),
@@ -845,7 +845,7 @@ __device__ void interp_pass_lagr4(const NodeSrcF& src, int x, int y, int z, doub
     for (int q = 0; q < 9; q++) {
       const int e = q / 3, t = q % 3;
       const int i = kIdx27.v[t][e][ez + 1];
-      fout[split27_fidx(i, cell, P)] = interp_lagr4f<MIR>(src, cxv[t], cyv[e], cz, make_tgtf(i, gc), sqTb);
+      o[q] = interp_lagr4f<MIR>(src, cxv[t], cyv[e], cz, make_tgtf(i, gc), sqTb);
     }
     return;
   }
@@ -977,7 +977,7 @@ __device__ void interp_pass_lagr4(const NodeSrcF& src, int x, int y, int z, doub
     const float wyz = ((e != 1) ? h : mm) * wz;
 #pragma unroll
     for (int t = 0; t < 3; t++)
-      fout[split27_fidx(kIdx27.v[t][e][ez + 1], cell, P)] = acc[e][t] * ((t != 1 ? h : mm) * wyz);
+      o[3 * e + t] = acc[e][t] * ((t != 1 ? h : mm) * wyz);
   }
 }
 
@@ -1000,65 +1000,38 @@ __device__ __forceinline__ void split_prev_gauge(const float* __restrict__ min, 
   if (rho0 == 0 && gp[0] == 0 && gp[1] == 0 && gp[2] == 0 && gp[3] == 0) { rho0 = 1; gp[3] = tlat; }
 }
 
-// One fixed-point iteration of one cell: true when it has converged.
-template <int INTERP>
-__device__ __forceinline__ bool split27_once(const NodeSrcF& src, float* __restrict__ fout, int64_t cell, int x,
-                                             int y, int z, const float* __restrict__ min,
-                                             const double* __restrict__ Tin, SplitIter& st, const SplitArgs& a) {
+// moments in the frame of the current gauge: A = sum f, B = sum f xi (compensated, FP32) and
+// C = sum f |xi|^2 (FP64)
+struct SplitSums {
+  float as = 0.f, ac = 0.f, bxs = 0.f, bxc = 0.f, bys = 0.f, byc = 0.f, bzs = 0.f, bzc = 0.f;
+  double cs = 0.0;
+  __device__ __forceinline__ void add(int ex, int ey, int ez, float fn) {
+    kahan_add(as, ac, fn);
+    kahan_add(bxs, bxc, (float)ex * fn);
+    kahan_add(bys, byc, (float)ey * fn);
+    kahan_add(bzs, bzc, (float)ez * fn);
+    cs += (double)fn * (double)(ex * ex + ey * ey + ez * ez);
+  }
+};
+
+// The end of one fixed-point iteration of one cell, from the sums over its new populations (s: the
+// lattice scale of the gauge they were formed in): true when it has converged.
+__device__ __forceinline__ bool split27_update(const SplitSums& q, double s, int64_t cell,
+                                               const float* __restrict__ min, const double* __restrict__ Tin,
+                                               SplitIter& st, const SplitArgs& a) {
   const int64_t P = a.g.plane;
-  const float sqTb = (float)a.sqrt_tbase;
   double* gc = st.gc;
+  st.niter++;
   {
-    st.niter++;
-    const double s = sqrt(gc[3] / a.tlat);
-    // moments in the frame of the current gauge: A = sum f, B = sum f xi, C = sum f |xi|^2
-    float as = 0.f, ac = 0.f, bxs = 0.f, bxc = 0.f, bys = 0.f, byc = 0.f, bzs = 0.f, bzc = 0.f;
-    double cs = 0.0;
-    auto add = [&](int ex, int ey, int ez, float fn) {
-      fout[split27_fidx(kIdx27.v[ex + 1][ey + 1][ez + 1], cell, P)] = fn;
-      kahan_add(as, ac, fn);
-      kahan_add(bxs, bxc, (float)ex * fn);
-      kahan_add(bys, byc, (float)ey * fn);
-      kahan_add(bzs, bzc, (float)ez * fn);
-      cs += (double)fn * (double)(ex * ex + ey * ey + ez * ez);
-    };
-    if constexpr (INTERP == 1 || INTERP == 2 || INTERP == 3) {
-      // WENO5C and Lagrange-4: the nine targets of each ez share their node loads and their z
-      // contraction (the pass stores the values to fout); the moments are then summed in the
-      // order (ey, ez, ex)
-#pragma unroll 1
-      for (int pz = 0; pz < 3; pz++) {
-        if constexpr (INTERP == 2) interp_pass_weno5c(src, x, y, z, s, gc, pz - 1, sqTb, fout, cell, P);
-        else interp_pass_lagr4<INTERP == 3>(src, x, y, z, s, gc, pz - 1, sqTb, fout, cell, P);
-      }
-      for (int gi = 0; gi < 9; gi++) {
-        const int ey = gi / 3 - 1, ez = gi % 3 - 1;
-#pragma unroll
-        for (int ex = -1; ex <= 1; ex++) add(ex, ey, ez, fout[split27_fidx(kIdx27.v[ex + 1][ey + 1][ez + 1], cell, P)]);
-      }
-    } else {
-      for (int i = 0; i < 27; i++) {
-        const int ex = kE27[i][0], ey = kE27[i][1], ez = kE27[i][2];
-        const double vx = s * (double)ex + gc[0];
-        const double vy = s * (double)ey + gc[1];
-        const double vz = s * (double)ez + gc[2];
-        const TgtF t = make_tgtf(i, gc);
-        const double cx = (double)x - vx, cy = (double)y - vy, cz = (double)z - vz;
-        // INTERP 3: Lagrange-4 with mirror boundaries
-        const float fn = INTERP == 1   ? interp_lagr4f<false>(src, cx, cy, cz, t, sqTb)
-                         : INTERP == 3 ? interp_lagr4f<true>(src, cx, cy, cz, t, sqTb)
-                                       : interp_weno5f<false>(src, cx, cy, cz, t, sqTb);
-        add(ex, ey, ez, fn);
-      }
-    }
     // FP64 moment solve (Cell::calcMoments, structs.cuh:315-342) restated in the gauge frame:
     // with v = u_g + s xi, sum f v / rho = u_g + s B/rho and
     // (sum f |v|^2/rho - |u|^2)/Dim = s^2 (C - |B|^2/rho) / (rho Dim).  This is the same
     // algebra without the cancellation of |u|^2 against sum f |v|^2 / rho, which at Mach 1
     // and above would amplify the FP32 rounding of the populations several times.
-    const double rho = (double)as - (double)ac;
+    const double rho = (double)q.as - (double)q.ac;
+    const double cs = q.cs;
     st.rho = rho;
-    const double B[3] = {(double)bxs - (double)bxc, (double)bys - (double)byc, (double)bzs - (double)bzc};
+    const double B[3] = {(double)q.bxs - (double)q.bxc, (double)q.bys - (double)q.byc, (double)q.bzs - (double)q.bzc};
     double m[4];
     if (rho != 0) {
       const double ir = 1.0 / rho;
@@ -1117,17 +1090,39 @@ __device__ __forceinline__ bool split27_once(const NodeSrcF& src, float* __restr
   return false;
 }
 
+// One iteration of one cell with the WENO5 as written, target by target; the iterate's populations are
+// left in fout.
+__device__ __forceinline__ bool split27_once(const NodeSrcF& src, float* __restrict__ fout, int64_t cell, int x,
+                                             int y, int z, const float* __restrict__ min,
+                                             const double* __restrict__ Tin, SplitIter& st, const SplitArgs& a) {
+  const float sqTb = (float)a.sqrt_tbase;
+  const double* gc = st.gc;
+  const double s = sqrt(gc[3] / a.tlat);
+  SplitSums sums;
+  for (int i = 0; i < 27; i++) {
+    const int ex = kE27[i][0], ey = kE27[i][1], ez = kE27[i][2];
+    const double vx = s * (double)ex + gc[0];
+    const double vy = s * (double)ey + gc[1];
+    const double vz = s * (double)ez + gc[2];
+    const TgtF t = make_tgtf(i, gc);
+    const double cx = (double)x - vx, cy = (double)y - vy, cz = (double)z - vz;
+    const float fn = interp_weno5f<false>(src, cx, cy, cz, t, sqTb);
+    fout[split27_fidx(i, cell, a.g.plane)] = fn;
+    sums.add(ex, ey, ez, fn);
+  }
+  return split27_update(sums, s, cell, min, Tin, st, a);
+}
+
 // Fixed-point iterations of one cell from state st until it converges (true), its count
 // reaches stop_at, or its count since its current start reaches the cap (false).  A cell that
 // abandons a predicted start gets the full cap from its previous gauge, so a cell that does
 // not converge ends on the same iterate as without the prediction.  The iterate's populations
 // are left in fout.
-template <int INTERP>
 __device__ bool split27_iterate(const NodeSrcF& src, float* __restrict__ fout, int64_t cell, int x, int y, int z,
                                 const float* __restrict__ min, const double* __restrict__ Tin, SplitIter& st,
                                 int stop_at, const SplitArgs& a) {
   while (st.niter < stop_at && st.niter - st.base < a.max_iter)
-    if (split27_once<INTERP>(src, fout, cell, x, y, z, min, Tin, st, a)) return true;
+    if (split27_once(src, fout, cell, x, y, z, min, Tin, st, a)) return true;
   return false;
 }
 
@@ -1197,20 +1192,16 @@ __device__ __forceinline__ void split27_start(const float* __restrict__ min, con
   }
 }
 
-// First pass: every cell iterates up to a.pass1_iters times.  A wave runs as long as its
-// slowest cell, and on contact discontinuities and shocks a thin layer of cells needs several
-// times the mean, so cells still unconverged after the first pass are appended to a list
-// (wave-aggregated: one atomic per wave) and finished by k_step_split27_rest, whose waves
-// hold only such cells.  Each cell's arithmetic is the same as in a single pass.
-// INTERP: 0 WENO5 as written, 1 Lagrange-4, 2 WENO5C with the targets of an (ey, ez) group
-// sharing their node work.
-template <int INTERP>
-__device__ __forceinline__ void split27_pass1(const float* __restrict__ fin, const float* __restrict__ min,
-                                              const double* __restrict__ Tin, const float* __restrict__ g4in,
-                                              float* __restrict__ fout, float* __restrict__ mout,
-                                              double* __restrict__ Tout, int* __restrict__ niter_out,
-                                              const float* __restrict__ guess, const SplitPending& pend,
-                                              const SplitArgs& a) {
+// The WENO5 as written (unstable in 3D; kept for parity runs): one lane per cell.  First pass: every
+// cell iterates up to a.pass1_iters times.  A wave runs as long as its slowest cell, and on contact
+// discontinuities and shocks a thin layer of cells needs several times the mean, so cells still
+// unconverged after the first pass are appended to a list (wave-aggregated: one atomic per wave) and
+// finished by k_step_split27_rest, whose waves hold only such cells.  Each cell's arithmetic is the
+// same as in a single pass.
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_step_split27_written(
+    const float* __restrict__ fin, const float* __restrict__ min, const double* __restrict__ Tin,
+    const float* __restrict__ g4in, float* __restrict__ fout, float* __restrict__ mout, double* __restrict__ Tout,
+    int* __restrict__ niter_out, const float* __restrict__ guess, SplitPending pend, const SplitArgs a) {
   const Grid& g = a.g;
   int x, y, z;
   const bool live = tile_cell(g, xcd_block(blockIdx.x, gridDim.x), threadIdx.x, x, y, z);
@@ -1220,7 +1211,7 @@ __device__ __forceinline__ void split27_pass1(const float* __restrict__ fin, con
   if (live) {
     split27_start(min, Tin, guess, niter_out, cell, st, a);
     const NodeSrcF src = make_src(fin, g4in, g);
-    const bool conv = split27_iterate<INTERP>(src, fout, cell, x, y, z, min, Tin, st, a.pass1_iters, a);
+    const bool conv = split27_iterate(src, fout, cell, x, y, z, min, Tin, st, a.pass1_iters, a);
     pending = !conv && st.niter - st.base < a.max_iter;
     if (!pending) split27_finish(fout, mout, Tout, niter_out, cell, st, a);
   }
@@ -1235,137 +1226,12 @@ __device__ __forceinline__ void split27_pass1(const float* __restrict__ fin, con
   }
 }
 
-// The D3Q27 split kernels are held to at least two waves per SIMD (256 registers): the WENO5C
-// and Lagrange-4 passes, with their node loads one step ahead, would otherwise take a few more
-// registers and drop to one wave, which leaves the load latency unhidden; held to two, they keep
-// a few rarely used values in scratch instead.
-#define POND_SPLIT27_KERNEL __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
-template <int INTERP>
-POND_SPLIT27_KERNEL void k_step_split27(const float* __restrict__ fin, const float* __restrict__ min,
-                                                     const double* __restrict__ Tin, const float* __restrict__ g4in,
-                                                     float* __restrict__ fout, float* __restrict__ mout,
-                                                     double* __restrict__ Tout, int* __restrict__ niter_out,
-                                                     const float* __restrict__ guess, SplitPending pend,
-                                                     const SplitArgs a) {
-  split27_pass1<INTERP>(fin, min, Tin, g4in, fout, mout, Tout, niter_out, guess, pend, a);
-}
-
-
-// Persistent refill waves (below) are built but not used: on the 384^3 shock-bubble they took
-// the WENO5C step from 157.8 to 155.2 ms, but the 256^3 vortex from 66.2 to 78.7 ms, the 384^3
-// Taylor-Green from 179.3 to 208.6 ms and the Lagrange-4 shock-bubble from 224 to 294 ms (a
-// wave handing over from one row to the next spans two distant rows, and the fetches from
-// beyond L2 double), so every kernel keeps one chunk per workgroup.
-constexpr bool kRefillPersistent[4] = {false, false, false, false};
-
-// Single pass with lane refill.  Cells are dealt in chunks of `chunk` consecutive 64-cell tiles
-// (a whole x row by default).  Whenever lanes of a wave finish their cells, they take the next
-// unstarted cells of its chunk in order (one ballot per iteration), so a lane is idle only when
-// no unstarted cell is left.  On the shock-bubble the mean gauge iterations per cell are about
-// 1.3 while the slowest cell of a 64-cell tile needs 3.5-5, so lanes of the one-tile-per-wave
-// step sit idle most of the time.
-//
-// Each workgroup owns one chunk, in the XCD-contiguous order of xcd_block.  Where
-// kRefillPersistent is set (for no interpolator at present, see there) the waves are persistent
-// instead: the grid is what the GPU holds at once, and a wave whose chunk has no unstarted cell
-// left claims the next chunk while its lanes still finish the old one, so the tail of a chunk
-// (the lanes of its last, slowest cells) is filled from the next one.  With one chunk per wave,
-// 30-40 % of the lane-iterations of the 384^3 shock-bubble step are such tails.
-// The chunks are split into eight contiguous slabs, one per XCD (workgroups are dealt to the XCDs
-// in turn, so a wave's XCD is its block index mod 8), and the waves of XCD k claim the chunks of
-// slab k in order from the counter claim[k] (zeroed before the launch), so the waves resident on
-// one XCD work on neighbouring rows and share their stencil halo in its L2.  Each cell's
-// arithmetic is the same as in k_step_split27 (bitwise the same results, whichever wave runs
-// it); the active cells of a wave stay within a window of one or two chunks, so node loads
-// remain close together.
-template <int INTERP>
-__device__ __forceinline__ void split27_refill(const float* __restrict__ fin, const float* __restrict__ min,
-                                               const double* __restrict__ Tin, const float* __restrict__ g4in,
-                                               float* __restrict__ fout, float* __restrict__ mout,
-                                               double* __restrict__ Tout, int* __restrict__ niter_out,
-                                               const float* __restrict__ guess, const SplitArgs& a, int chunk,
-                                               int* __restrict__ claim) {
-  const Grid& g = a.g;
-  const int lane = threadIdx.x;
-  const int64_t ntiles = g.ntiles;
-  const int64_t nchunks = (ntiles + chunk - 1) / chunk;
-  constexpr int kXcd = 8;
-  const int xk = (int)(blockIdx.x % kXcd);
-  const int64_t q = nchunks / kXcd, rq = nchunks % kXcd;
-  const int64_t c_lo = xk * q + (xk < rq ? xk : rq), c_hi = c_lo + q + (xk < rq ? 1 : 0);
-  const NodeSrcF src = make_src(fin, g4in, g);
-  int64_t t0 = 0, total = 0;  // first tile and cell slots of the current chunk
-  int64_t next = 0;           // first unstarted slot (the same in every lane)
-  bool more = true;           // the slab may still hold unclaimed chunks
-  if constexpr (!kRefillPersistent[INTERP]) {
-    // one chunk per workgroup, in the XCD-contiguous order of xcd_block
-    t0 = xcd_block(blockIdx.x, gridDim.x) * chunk;
-    total = (ntiles - t0 < chunk ? ntiles - t0 : chunk) * 64;
-    more = false;
-  }
-  bool active = false;
-  int64_t cell = 0;
-  int x = 0, y = 0, z = 0;
-  SplitIter st;
-  while (true) {
-    const uint64_t want = __ballot(!active);
-    if (kRefillPersistent[INTERP] && want != 0 && next >= total && more) {
-      // lanes are free and the chunk has no unstarted cell: claim the slab's next chunk
-      int idx = 0;
-      if (lane == 0) idx = atomicAdd(&claim[xk], 1);
-      idx = __shfl(idx, 0);
-      const int64_t c = c_lo + idx;
-      if (c < c_hi) {
-        t0 = c * chunk;
-        total = (ntiles - t0 < chunk ? ntiles - t0 : chunk) * 64;
-        next = 0;
-      } else {
-        more = false;
-      }
-    }
-    // lanes without a cell take the next slots, in lane order; a slot outside the grid (ragged
-    // last tile) is used up without a cell
-    const int rank = __popcll(want & ((1ull << lane) - 1ull));
-    if (!active) {
-      const int64_t slot = next + rank;
-      if (slot < total && tile_cell(g, t0 + slot / 64, (int)(slot % 64), x, y, z)) {
-        cell = cell_index(g, x, y, z);
-        split27_start(min, Tin, guess, niter_out, cell, st, a);
-        active = true;
-      }
-    }
-    next += __popcll(want);
-    if (__ballot(active) == 0 && next >= total && !more) break;
-    if (active) {
-      // the loop condition of split27_iterate, one iteration per trip
-      bool done = st.niter - st.base >= a.max_iter;
-      if (!done)
-        done = split27_once<INTERP>(src, fout, cell, x, y, z, min, Tin, st, a) || st.niter - st.base >= a.max_iter;
-      if (done) {
-        split27_finish(fout, mout, Tout, niter_out, cell, st, a);
-        active = false;
-      }
-    }
-  }
-}
-
-template <int INTERP>
-POND_SPLIT27_KERNEL void k_step_split27_refill(
-    const float* __restrict__ fin, const float* __restrict__ min, const double* __restrict__ Tin,
-    const float* __restrict__ g4in, float* __restrict__ fout, float* __restrict__ mout, double* __restrict__ Tout,
-    int* __restrict__ niter_out, const float* __restrict__ guess, const SplitArgs a, int chunk, int* claim) {
-  split27_refill<INTERP>(fin, min, Tin, g4in, fout, mout, Tout, niter_out, guess, a, chunk, claim);
-}
-
-
 // Second pass: a fixed grid of waves walks the pending list; every cell resumes its iteration
 // where the first pass left it.
-template <int INTERP>
-__device__ __forceinline__ void split27_rest(const float* __restrict__ fin, const float* __restrict__ min,
-                                             const double* __restrict__ Tin, const float* __restrict__ g4in,
-                                             float* __restrict__ fout, float* __restrict__ mout,
-                                             double* __restrict__ Tout, int* __restrict__ niter_out,
-                                             const SplitPending& pend, const SplitArgs& a) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_step_split27_rest(
+    const float* __restrict__ fin, const float* __restrict__ min, const double* __restrict__ Tin,
+    const float* __restrict__ g4in, float* __restrict__ fout, float* __restrict__ mout, double* __restrict__ Tout,
+    int* __restrict__ niter_out, SplitPending pend, const SplitArgs a) {
   const Grid& g = a.g;
   const int count = *pend.count;
   const NodeSrcF src = make_src(fin, g4in, g);
@@ -1386,48 +1252,118 @@ __device__ __forceinline__ void split27_rest(const float* __restrict__ fin, cons
     st.base = (meta >> 8) & 0xff;
     st.learned = (meta & 0x10000) != 0;
     st.contracted = (meta & 0x20000) != 0;
-    split27_iterate<INTERP>(src, fout, cell, x, y, z, min, Tin, st, 0x7fffffff, a);
+    split27_iterate(src, fout, cell, x, y, z, min, Tin, st, 0x7fffffff, a);
     split27_finish(fout, mout, Tout, niter_out, cell, st, a);
   }
 }
 
+// WENO5C and Lagrange-4 (INTERP 2, 1; 3: Lagrange-4 with mirror walls): three lanes per cell, lane =
+// ez pass of nine targets, 21 cells per wave.
+//
+// With one lane per cell (its three passes one after the other) a wave spanned 64 cells: a third of
+// its lane-iterations went to row ends waiting for the last slow cells, each pass fetched the same
+// neighbourhood again, and a cell at the cap of 100 iterations took 17 ms by itself.  Side by side,
+// the passes of a cell share their node loads (the lanes ask for the same cache lines wherever their z
+// rows coincide), the iterate stays in LDS instead of going through global memory, and a slot takes the
+// next cell of the wave's run when its own has converged.  Each cell's arithmetic and its order are the
+// same (bit for bit).  Per step, before and after: 256^3 vortex 65.3 -> 39.6 ms, 256^3 shock-bubble
+// 107 -> 69.7 ms, 32^3 shock-bubble 16.9 -> 5.6 ms; Lagrange-4 192^3 Taylor-Green 81 -> 37.5 ms,
+// 150x101x94 22.0 -> 8.5 ms.  256^3 vortex: VALU busy 85 % (57 of 64 lanes), texture-address unit 71 %.
+// Two waves per SIMD (256 registers): with more registers the load latency would be left unhidden.
 template <int INTERP>
-POND_SPLIT27_KERNEL void k_step_split27_rest(const float* __restrict__ fin, const float* __restrict__ min,
-                                                          const double* __restrict__ Tin, const float* __restrict__ g4in,
-                                                          float* __restrict__ fout, float* __restrict__ mout,
-                                                          double* __restrict__ Tout, int* __restrict__ niter_out,
-                                                          SplitPending pend, const SplitArgs a) {
-  split27_rest<INTERP>(fin, min, Tin, g4in, fout, mout, Tout, niter_out, pend, a);
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_step_split27_cells(
+    const float* __restrict__ fin, const float* __restrict__ min, const double* __restrict__ Tin,
+    const float* __restrict__ g4in, float* __restrict__ fout, float* __restrict__ mout, double* __restrict__ Tout,
+    int* __restrict__ niter_out, const float* __restrict__ guess, const SplitArgs a, int cells) {
+  constexpr int FS = 28;
+  __shared__ __align__(16) float s_f[22][FS];  // the iterate's populations, [cell][9 (ez+1) + 3 (ey+1) + ex+1]
+  __shared__ float s_w[FS];
+  const Grid& g = a.g;
+  const int64_t P = g.plane;
+  const int lane = threadIdx.x;
+  const int slot = lane / 3, pz = lane - 3 * slot;  // lane 63 has no cell
+  constexpr uint64_t kHeads = 0x1249249249249249ull;  // lanes 0, 3, .., 60
+  if (lane < FS) s_w[lane] = lane < 27 ? a.w[lane] : 0.f;
+  const int64_t q0 = xcd_block(blockIdx.x, gridDim.x) * cells;
+  const int64_t total = g.ntiles * 64 - q0 < cells ? g.ntiles * 64 - q0 : cells;  // cell slots of the wave
+  const NodeSrcF src = make_src(fin, g4in, g);
+  int64_t next = 0;  // first unstarted slot (the same in every lane)
+  bool active = false;
+  int64_t cell = 0;
+  int x = 0, y = 0, z = 0;
+  SplitIter st;
+  while (true) {
+    const uint64_t want = __ballot(!active) & kHeads;
+    if (!active && slot < 21) {
+      const int64_t q = next + __popcll(want & ((1ull << (3 * slot)) - 1ull));
+      // (a slot outside the grid, in a ragged last tile, is used up without a cell)
+      if (q < total && tile_cell(g, (q0 + q) / 64, (int)((q0 + q) % 64), x, y, z)) {
+        cell = cell_index(g, x, y, z);
+        split27_start(min, Tin, guess, niter_out, cell, st, a);
+        active = true;
+      }
+    }
+    next += __popcll(want);
+    if (__ballot(active) == 0 && next >= total) break;
+    double s = 0;
+    if (active) {
+      s = sqrt(st.gc[3] / a.tlat);
+      float* o = &s_f[slot][9 * pz];
+      if constexpr (INTERP == 2) interp_pass_weno5c(src, x, y, z, s, st.gc, pz - 1, (float)a.sqrt_tbase, o);
+      else interp_pass_lagr4<INTERP == 3>(src, x, y, z, s, st.gc, pz - 1, (float)a.sqrt_tbase, o);
+    }
+    wave_lds_order();
+    if (active) {
+      // the cell's sums in the order (ey, ez, ex), in each of its lanes
+      float f[FS];
+#pragma unroll
+      for (int q = 0; q < 7; q++) {
+        const float4 v = *reinterpret_cast<const float4*>(&s_f[slot][4 * q]);
+        f[4 * q] = v.x; f[4 * q + 1] = v.y; f[4 * q + 2] = v.z; f[4 * q + 3] = v.w;
+      }
+      SplitSums sums;
+#pragma unroll
+      for (int ey = 0; ey < 3; ey++)
+#pragma unroll
+        for (int ez = 0; ez < 3; ez++)
+#pragma unroll
+          for (int ex = 0; ex < 3; ex++) sums.add(ex - 1, ey - 1, ez - 1, f[9 * ez + 3 * ey + ex]);
+      if (split27_update(sums, s, cell, min, Tin, st, a) || st.niter - st.base >= a.max_iter) {
+        // BGK in FP32 (steps.cu:557-564) and the cell's outputs: quad planes pz, pz + 3, pz + 6
+        active = false;
+        const float rf = (float)st.rho, dt = (float)a.dtau;
+#pragma unroll
+        for (int q = 0; q < 7; q++) {
+          if (q % 3 != pz) continue;
+          float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const int i = 4 * q + e;
+            if (i < 27) {
+              const float fi = f[9 * (kE27[i][2] + 1) + 3 * (kE27[i][1] + 1) + kE27[i][0] + 1];
+              v[e] = __builtin_fmaf(dt, rf * s_w[i] - fi, fi);
+            }
+          }
+          reinterpret_cast<float4*>(fout)[q * P + cell] = make_float4(v[0], v[1], v[2], v[3]);
+        }
+        if (pz == 0) {
+          mout[cell] = rf;
+          mout[P + cell] = (float)st.gc[0];
+        } else if (pz == 1) {
+          mout[2 * P + cell] = (float)st.gc[1];
+          mout[3 * P + cell] = (float)st.gc[2];
+        } else {
+          Tout[cell] = st.gc[3];
+          niter_out[cell] = st.niter;
+        }
+      }
+    }
+    wave_lds_order();
+  }
 }
-
 
 __global__ void k_zero_count(int* c) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *c = 0;
-}
-
-__global__ void k_zero_ints(int* p, int n) {
-  if (blockIdx.x == 0 && (int)threadIdx.x < n) p[threadIdx.x] = 0;
-}
-
-// Workgroups of the persistent refill kernel: 16 64-lane blocks per CU, twice what two waves per
-// SIMD hold (blocks beyond those resident start when others have ended, find their slab used up
-// and end), a multiple of 8 (one share per XCD slab; at least 8 so that every slab has waves),
-// never more than the chunks, and one per chunk when there are fewer than 8.
-static unsigned refill_blocks(int64_t nchunks) {
-  static int cus = 0;
-  if (cus == 0) {
-    int dev = 0;
-    hipDeviceProp_t prop;
-    cus = (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess &&
-           prop.multiProcessorCount > 0)
-              ? prop.multiProcessorCount
-              : 256;
-  }
-  if (nchunks < 8) return (unsigned)nchunks;
-  const int64_t resident = (int64_t)16 * cus;
-  int64_t b = resident < nchunks ? resident : nchunks;
-  b -= b % 8;
-  return (unsigned)(b < 8 ? 8 : b);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1834,38 +1770,45 @@ hipError_t launch_step_split(int lattice, int interp, const SplitPtrs& in, const
     return hipGetLastError();
   }
   if (lattice != kD3Q27) return hipErrorInvalidValue;
-  const unsigned blocks = (unsigned)(a.g.ntiles);
+  if (interp != 0) {
+    const int64_t slots = a.g.ntiles * 64;
+    // Cells per wave.  Where the cells go by x rows (row patches): whole rows, at least 128 cells, so
+    // that the waves resident on an XCD cover a compact patch of rows, but no so many that SIMDs go
+    // without two waves.  In linear order: 128 cells on large grids, one per slot below (the waves in
+    // flight then cover fewer planes, and more of them even out the last round).  ms per step with
+    // 21, 42, 64, 128, 192, 256, 384 cells, WENO5C vortex: 64^3 1.03, 0.98, 0.86, 0.84, 1.10, 1.36,
+    // 1.96; 128^3 6.79, 6.24, 5.95, 5.43, 5.66, 5.36, 5.73; 192^3 22.4, 20.4, 19.2, 17.8, 17.0, 17.5,
+    // 16.9; 250x200x180 28.8, 26.3, 25.6, 23.0, 28.3, 22.1, 27.0; shock-bubble 32^3 5.60, 5.79, 5.86,
+    // 6.34, -, 6.22; Lagrange-4 150x101x94 8.45, 8.84, 9.97, 10.4, -, 11.3.
+    int64_t cells;
+    if (a.refill_chunk >= 0) {
+      cells = a.refill_chunk > 0 ? 64ll * a.refill_chunk : 64;
+    } else if (a.g.rp > 0) {
+      cells = a.g.nx * ((128ll + a.g.nx - 1) / a.g.nx);
+      while (cells > 21 && slots / cells < 2048) cells /= 2;
+      if (cells < 21) cells = 21;
+    } else {
+      cells = a.g.n >= (1 << 22) ? 128 : 21;
+    }
+    if (cells > slots) cells = slots;
+    const dim3 nb((unsigned)((slots + cells - 1) / cells));
+#define POND_LAUNCH(I)                                                                                             \
+  hipLaunchKernelGGL(k_step_split27_cells<I>, nb, dim3(64), 0, st, in.f, in.m, in.T, g4, out.f, out.m, out.T, niter, \
+                     guess, a, (int)cells)
+    if (interp == 2) POND_LAUNCH(2);
+    else if (a.g.mirror) POND_LAUNCH(3);
+    else POND_LAUNCH(1);
+#undef POND_LAUNCH
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(k_zero_count, dim3(1), dim3(64), 0, st, pend.count);
   // second-pass grid: enough waves to fill the chip several times, never more than the cells
   const int64_t w2 = (a.g.n + 63) / 64;
   const unsigned blocks2 = (unsigned)(w2 < 16384 ? w2 : 16384);
-#define POND_LAUNCH_S(K, I)                                                                                       \
-  do {                                                                                                            \
-    hipLaunchKernelGGL((K), dim3(blocks), dim3(64), 0, st, in.f, in.m, in.T, g4, out.f, out.m, out.T, niter, guess, \
-                       pend, a);                                                                                  \
-    hipLaunchKernelGGL((k_step_split27_rest<I>), dim3(blocks2), dim3(64), 0, st, in.f, in.m, in.T, g4, out.f,     \
-                       out.m, out.T, niter, pend, a);                                                             \
-  } while (0)
-  if (interp != 0 && a.refill_chunk > 0 && a.pass1_iters >= a.max_iter + kLearnedBudget) {
-    const int64_t nchunks = ((int64_t)blocks + a.refill_chunk - 1) / a.refill_chunk;
-    // the slabs' chunk counters, in the pending list's header (its count is the first int)
-    int* claim = pend.count + 16;
-    hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, st, claim, 8);
-#define POND_LAUNCH_R(I)                                                                                              \
-  hipLaunchKernelGGL(k_step_split27_refill<I>, dim3(kRefillPersistent[I] ? refill_blocks(nchunks) : (unsigned)nchunks), \
-                     dim3(64), 0, st, in.f, in.m, in.T, g4,                                                              \
-                     out.f, out.m, out.T, niter, guess, a, a.refill_chunk, claim)
-    if (interp == 2) POND_LAUNCH_R(2);
-    else if (a.g.mirror) POND_LAUNCH_R(3);
-    else POND_LAUNCH_R(1);
-#undef POND_LAUNCH_R
-    return hipGetLastError();
-  }
-  if (interp == 1 && a.g.mirror) POND_LAUNCH_S(k_step_split27<3>, 3);
-  else if (interp == 1) POND_LAUNCH_S(k_step_split27<1>, 1);
-  else if (interp == 2) POND_LAUNCH_S(k_step_split27<2>, 2);
-  else POND_LAUNCH_S(k_step_split27<0>, 0);
-#undef POND_LAUNCH_S
+  hipLaunchKernelGGL(k_step_split27_written, dim3((unsigned)a.g.ntiles), dim3(64), 0, st, in.f, in.m, in.T, g4, out.f,
+                     out.m, out.T, niter, guess, pend, a);
+  hipLaunchKernelGGL(k_step_split27_rest, dim3(blocks2), dim3(64), 0, st, in.f, in.m, in.T, g4, out.f, out.m, out.T,
+                     niter, pend, a);
   return hipGetLastError();
 }
 
