@@ -54,6 +54,9 @@ __device__ __forceinline__ TgtF make_tgtf(int k, const double* g) {
   return t;
 }
 
+__device__ __forceinline__ int min3(int a, int b, int c) { return min(a, min(b, c)); }
+__device__ __forceinline__ int max3(int a, int b, int c) { return max(a, max(b, c)); }
+
 // basis values L[j], j = source component -1,0,+1, of one axis (structs.cuh:530-538)
 __device__ __forceinline__ void basis3(float D, float sq0, bool kn, float c, float T1, float w, float L[3]) {
 #pragma unroll
@@ -518,6 +521,61 @@ __device__ void interp_group_weno5c(const NodeSrcF& src, int x, int y, int z, do
   }
 }
 
+// What the three ey groups of an ez pass share of one stencil node: with the node's contraction over
+// the z source components, sz[ja][jb] = sum_jc Lz[jc] f(ja, jb, jc), the x basis of the three targets
+// is A_j (A_j - c) or A_j^2 - T1 with A_j = Dx - (j-1) sq0, so the x moments R = sum_ja sz, Q = sum_ja
+// A_ja sz, P = sum_ja A_ja^2 sz per source y component jb serve every group
+struct NodePass {
+  float xr[3], xq[3], xp[3];
+  float Ay0, Ay1, Ay2;  // the y basis' A_j
+};
+
+__device__ __forceinline__ NodePass node_pass(const float f[27], const Gauge4& n, float u1x, float u1xl, float u1y,
+                                              float u1yl, float u1z, float u1zl, float sqTb, float czb, float Tzb) {
+  NodePass o;
+  float Lz[3];
+  basis3u(((u1z - n.uz) + u1zl) * sqTb, n.sq, czb, Tzb, Lz);
+  float szz[3][3];
+#pragma unroll
+  for (int ja = 0; ja < 3; ja++)
+#pragma unroll
+    for (int jb = 0; jb < 3; jb++) {
+      float sz = 0.f;
+#pragma unroll
+      for (int jc = 0; jc < 3; jc++) sz = __builtin_fmaf(Lz[jc], f[kIdx27.v[ja][jb][jc]], sz);
+      szz[ja][jb] = sz;
+    }
+  const float Dy = ((u1y - n.uy) + u1yl) * sqTb;
+  const float Dx = ((u1x - n.ux) + u1xl) * sqTb;
+  const float A0 = Dx + n.sq, A1 = Dx, A2 = Dx - n.sq;
+  const float B0 = A0 * A0, B1 = A1 * A1, B2 = A2 * A2;
+#pragma unroll
+  for (int jb = 0; jb < 3; jb++) {
+    o.xr[jb] = (szz[0][jb] + szz[1][jb]) + szz[2][jb];
+    o.xq[jb] = __builtin_fmaf(A2, szz[2][jb], __builtin_fmaf(A1, szz[1][jb], A0 * szz[0][jb]));
+    o.xp[jb] = __builtin_fmaf(B2, szz[2][jb], __builtin_fmaf(B1, szz[1][jb], B0 * szz[0][jb]));
+  }
+  o.Ay0 = Dy + n.sq;
+  o.Ay1 = Dy;
+  o.Ay2 = Dy - n.sq;
+  return o;
+}
+
+// the node's values for the three targets of group ey (without the per-axis basis factors): the y
+// contraction of the x moments, then P + sq1 Q, P - T1 R and P - sq1 Q
+__device__ __forceinline__ void node_group(const NodePass& p, int ey, float sq1, float T1, float Tt[3]) {
+  // basis3u of the group: fma(A, A - c, -T) with (c, T) of a moving or resting y axis
+  const float cyb = ey ? (float)ey * sq1 : 0.0f, Tyb = ey ? 0.0f : T1;
+  const float Ly0 = __builtin_fmaf(p.Ay0, p.Ay0 - cyb, -Tyb), Ly1 = __builtin_fmaf(p.Ay1, p.Ay1 - cyb, -Tyb),
+              Ly2 = __builtin_fmaf(p.Ay2, p.Ay2 - cyb, -Tyb);
+  const float R = __builtin_fmaf(Ly2, p.xr[2], __builtin_fmaf(Ly1, p.xr[1], Ly0 * p.xr[0]));
+  const float Q = __builtin_fmaf(Ly2, p.xq[2], __builtin_fmaf(Ly1, p.xq[1], Ly0 * p.xq[0]));
+  const float Pp = __builtin_fmaf(Ly2, p.xp[2], __builtin_fmaf(Ly1, p.xp[1], Ly0 * p.xp[0]));
+  Tt[0] = __builtin_fmaf(sq1, Q, Pp);
+  Tt[1] = __builtin_fmaf(-T1, R, Pp);
+  Tt[2] = __builtin_fmaf(-sq1, Q, Pp);
+}
+
 // WENO5C for the nine targets that share ez (ey, ex = -1, 0, 1): one pass over the union of
 // their stencil nodes.  Their departure points share the z rows, and the x windows depend on ex
 // only; the y rows of the three ey groups differ by at most a row or two (they coincide wherever
@@ -641,51 +699,15 @@ __device__ __forceinline__ void interp_pass_weno5c(const NodeSrcF& src, int x, i
       for (int b = 0; b < 3; b++) {
         const uint32_t zb = b == 0 ? zo[0] : b == 1 ? zo[1] : zo[2];
         const float fzb = b == 0 ? Fz[0] : b == 1 ? Fz[1] : Fz[2];
-        const Gauge4 n = nb[b];
-        // shared by the three groups: the z basis and contraction, the y and x differences
-        float Lz[3];
-        basis3u(((u1z - n.uz) + u1zl) * sqTb, n.sq, czb, Tzb, Lz);
-        float szz[3][3];
-#pragma unroll
-        for (int ja = 0; ja < 3; ja++)
-#pragma unroll
-          for (int jb = 0; jb < 3; jb++) {
-            float sz = 0.f;
-#pragma unroll
-            for (int jc = 0; jc < 3; jc++) sz = __builtin_fmaf(Lz[jc], fb[b][kIdx27.v[ja][jb][jc]], sz);
-            szz[ja][jb] = sz;
-          }
-        // the x basis of the three targets is A_j (A_j - c) or A_j^2 - T1 with A_j = Dx - (j-1) sq0:
-        // the x moments R = sum_ja sz, Q = sum_ja A_ja sz, P = sum_ja A_ja^2 sz of the z sums, per
-        // source y component jb, are common to every group; each group then contracts them
-        // over y and its three targets take P + sq1 Q, P - T1 R and P - sq1 Q
-        const float Dy = ((u1y - n.uy) + u1yl) * sqTb;
-        const float Dx = ((u1x - n.ux) + u1xl) * sqTb;
-        const float A0 = Dx + n.sq, A1 = Dx, A2 = Dx - n.sq;
-        const float B0 = A0 * A0, B1 = A1 * A1, B2 = A2 * A2;
-        float xr[3], xq[3], xp[3];
-#pragma unroll
-        for (int jb = 0; jb < 3; jb++) {
-          xr[jb] = (szz[0][jb] + szz[1][jb]) + szz[2][jb];
-          xq[jb] = __builtin_fmaf(A2, szz[2][jb], __builtin_fmaf(A1, szz[1][jb], A0 * szz[0][jb]));
-          xp[jb] = __builtin_fmaf(B2, szz[2][jb], __builtin_fmaf(B1, szz[1][jb], B0 * szz[0][jb]));
-        }
-        const float Ay0 = Dy + n.sq, Ay1 = Dy, Ay2 = Dy - n.sq;
+        const NodePass np = node_pass(fb[b], nb[b], u1x, u1xl, u1y, u1yl, u1z, u1zl, sqTb, czb, Tzb);
 #pragma unroll
         for (int e = 0; e < 3; e++) {
           const int a = ya[e];
           if (a < 0 || a > 2) continue;
-          const int ey = e - 1;
-          // basis3u of the group: fma(A, A - c, -T) with (c, T) of a moving or resting y axis
-          const float cyb = ey ? (float)ey * sq1 : 0.0f, Tyb = ey ? 0.0f : T1;
-          const float Ly0 = __builtin_fmaf(Ay0, Ay0 - cyb, -Tyb), Ly1 = __builtin_fmaf(Ay1, Ay1 - cyb, -Tyb),
-                      Ly2 = __builtin_fmaf(Ay2, Ay2 - cyb, -Tyb);
-          const float R = __builtin_fmaf(Ly2, xr[2], __builtin_fmaf(Ly1, xr[1], Ly0 * xr[0]));
-          const float Q = __builtin_fmaf(Ly2, xq[2], __builtin_fmaf(Ly1, xq[1], Ly0 * xq[0]));
-          const float Pp = __builtin_fmaf(Ly2, xp[2], __builtin_fmaf(Ly1, xp[1], Ly0 * xp[0]));
+          float Tt[3];
+          node_group(np, e - 1, sq1, T1, Tt);
           const float fya = a == 0 ? Fy[e][0] : a == 1 ? Fy[e][1] : Fy[e][2];
           const float wab = fya * fzb;
-          const float Tt[3] = {__builtin_fmaf(sq1, Q, Pp), __builtin_fmaf(-T1, R, Pp), __builtin_fmaf(-sq1, Q, Pp)};
 #pragma unroll
           for (int t = 0; t < 3; t++) yz[e][t] = __builtin_fmaf(wab, Tt[t], yz[e][t]);
           // the smoothness samples are the middle node's values: the middle z row (b, uniform
@@ -762,8 +784,9 @@ __device__ __forceinline__ void kahan_add(float& s, float& c, float v) {
 // are read only as nodes.  FP32 ranges: a population or gauge beyond FP32 range is already
 // infinite in the split state.
 __global__ void k_node_gauge(float* __restrict__ f, const float* __restrict__ m, const double* __restrict__ T,
-                             float* __restrict__ g4, int64_t n, int64_t plane) {
+                             float* __restrict__ g4, int64_t n, int64_t plane, int* __restrict__ count) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c == 0) *count = 0;  // the step's list of pending cells
   if (c >= n) return;
   const double t = T[c];
   float4 v;
@@ -1257,6 +1280,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
   }
 }
 
+// the list of slow cells: entry 0 is their number, the cells start here
+constexpr int kSlowList = 64;
+
 // WENO5C and Lagrange-4 (INTERP 2, 1; 3: Lagrange-4 with mirror walls): three lanes per cell, lane =
 // ez pass of nine targets, 21 cells per wave.
 //
@@ -1274,7 +1300,8 @@ template <int INTERP>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_step_split27_cells(
     const float* __restrict__ fin, const float* __restrict__ min, const double* __restrict__ Tin,
     const float* __restrict__ g4in, float* __restrict__ fout, float* __restrict__ mout, double* __restrict__ Tout,
-    int* __restrict__ niter_out, const float* __restrict__ guess, const SplitArgs a, int cells) {
+    int* __restrict__ niter_out, const float* __restrict__ guess, int* __restrict__ slow, const SplitArgs a, int cells,
+    int wide_after) {
   constexpr int FS = 28;
   __shared__ __align__(16) float s_f[22][FS];  // the iterate's populations, [cell][9 (ez+1) + 3 (ey+1) + ex+1]
   __shared__ float s_w[FS];
@@ -1293,6 +1320,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
   int x = 0, y = 0, z = 0;
   SplitIter st;
   while (true) {
+    if (INTERP == 2 && active && st.niter >= wide_after) {
+      // left to k_step_split27_wide, its state in three of the cell's output quads (arguments for
+      // separate arrays cost the pass scratch registers: 39.7 -> 49.8 ms on the 256^3 vortex)
+      active = false;
+      const int64_t meta =
+          st.niter | ((int64_t)st.base << 16) | (st.learned ? 1ll << 32 : 0) | (st.contracted ? 1ll << 33 : 0);
+      reinterpret_cast<double2*>(fout)[pz * P + cell] =
+          make_double2(pz == 0 ? st.gc[0] : pz == 1 ? st.gc[2] : st.res_prev,
+                       pz == 0 ? st.gc[1] : pz == 1 ? st.gc[3] : __longlong_as_double(meta));
+      if (pz == 0) slow[kSlowList + atomicAdd(slow, 1)] = (int)cell;
+    }
     const uint64_t want = __ballot(!active) & kHeads;
     if (!active && slot < 21) {
       const int64_t q = next + __popcll(want & ((1ull << (3 * slot)) - 1ull));
@@ -1359,6 +1397,178 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
       }
     }
     wave_lds_order();
+  }
+}
+
+// The WENO5C cells that k_step_split27_cells left unconverged: one workgroup per cell.
+//
+// A few cells on shocks and contacts go on to the cap of 100 iterations.  Three lanes take 50 us for such
+// an iteration (63 chained steps of three nodes), so on grids up to 128^3 they held up the whole step.
+// Here the nodes of the three passes are spread over the threads (189 for a seven-slice window on
+// three rows), their values for the targets laid down in LDS, and the sums over them run target
+// by target in the pass's order, so every value is the one the pass gives.  6.5 us per iteration, bound by the
+// chain of its six dependent parts (8.5 us with one wave per cell and three nodes per lane).
+// Shock-bubble, ms per step before and after: 32^3 5.6 -> 1.0, 64^3 6.7 -> 2.5, 128^3 14.5 -> 11.6.
+//
+// Every thread of the group forms the same sums and the same gauge from LDS, so the group leaves its
+// loop together and each barrier is met by all.
+constexpr int kWideThreads = 256;
+__global__ __launch_bounds__(kWideThreads) void k_step_split27_wide(
+    const float* __restrict__ fin, const float* __restrict__ min, const double* __restrict__ Tin,
+    const float* __restrict__ g4in, float* __restrict__ fout, float* __restrict__ mout, double* __restrict__ Tout,
+    int* __restrict__ niter_out, const int* __restrict__ slow, const SplitArgs a) {
+  constexpr int MS = 9, MR = 5;             // most slices and rows of a pass
+  __shared__ float s_T[3 * MS * MR * 3][9];  // a node's values for the targets 3 e + t
+  __shared__ float s_yz[27][MS];            // y/z sums of a target's slices
+  __shared__ float s_f[28];                 // the iterate, [9 (ez+1) + 3 (ey+1) + ex+1]
+  __shared__ float s_Fy[9], s_Fz[9];
+  const Grid& g = a.g;
+  const int64_t P = g.plane;
+  const int lane = threadIdx.x;
+  const NodeSrcF src = make_src(fin, g4in, g);
+  const float sqTb = (float)a.sqrt_tbase;
+  const int count = *slow;
+  for (int64_t e0 = blockIdx.x; e0 < count; e0 += gridDim.x) {
+    const int64_t cell = slow[kSlowList + e0];
+    const int x = (int)(cell % g.nx);
+    const int y = (int)((cell / g.nx) % g.ny);
+    const int z = (int)(cell / ((int64_t)g.nx * g.ny));
+    const double2* so = reinterpret_cast<const double2*>(fout) + cell;
+    const double2 g01 = so[0], g23 = so[P], rm = so[2 * P];
+    const int64_t meta = __double_as_longlong(rm.y);
+    SplitIter st;
+    st.gc[0] = g01.x;
+    st.gc[1] = g01.y;
+    st.gc[2] = g23.x;
+    st.gc[3] = g23.y;
+    st.res_prev = rm.x;
+    st.rho = 0;
+    st.niter = (int)(meta & 0xffff);
+    st.base = (int)((meta >> 16) & 0xffff);
+    st.learned = (meta >> 32) & 1;
+    st.contracted = (meta >> 33) & 1;
+    bool conv = false;
+    while (!conv && st.niter - st.base < a.max_iter) {
+      const double* gc = st.gc;
+      const double s = sqrt(gc[3] / a.tlat);
+      // the pass's constants (interp_pass_weno5c)
+      const float u1x = (float)gc[0], u1y = (float)gc[1], u1z = (float)gc[2];
+      const float u1xl = (float)(gc[0] - (double)u1x), u1yl = (float)(gc[1] - (double)u1y),
+                  u1zl = (float)(gc[2] - (double)u1z);
+      const float T1 = (float)gc[3];
+      const float h = 1.0f / (2.0f * T1), mm = -1.0f / T1;
+      const float sq1 = sqrtf(fabsf(T1)) * (float)((0.0f < T1) - (T1 < 0.0f));
+      int rz[3], ry[3], r[3];
+      float c[3];
+#pragma unroll
+      for (int q = 0; q < 3; q++) {
+        const double cz = (double)z - (s * (double)(q - 1) + gc[2]), cy = (double)y - (s * (double)(q - 1) + gc[1]);
+        const double cx = (double)x - (s * (double)(q - 1) + gc[0]);
+        rz[q] = floor_int(cz + 0.5) - 1;
+        ry[q] = floor_int(cy + 0.5) - 1;
+        r[q] = floor_int(cx + 0.5);
+        c[q] = (float)(cx - r[q]);
+        float Fz[3], Fy[3];
+        lag3f((float)(cz - rz[q]), Fz);
+        lag3f((float)(cy - ry[q]), Fy);
+        if (lane == 0) {
+#pragma unroll
+          for (int m = 0; m < 3; m++) { s_Fz[3 * q + m] = Fz[m]; s_Fy[3 * q + m] = Fy[m]; }
+        }
+      }
+      const int xlo = min3(r[0], r[1], r[2]) - 2, xhi = max3(r[0], r[1], r[2]) + 2;
+      const int ylo = min3(ry[0], ry[1], ry[2]), yhi = max3(ry[0], ry[1], ry[2]) + 2;
+      __syncthreads();
+      if ((int64_t)xhi - (int64_t)xlo > MS - 1 || (int64_t)yhi - (int64_t)ylo > MR - 1) {
+        if (lane < 9) {
+          float f3[3];
+          interp_group_weno5c(src, x, y, z, s, gc, lane % 3 - 1, lane / 3 - 1, sqTb, f3);
+#pragma unroll
+          for (int t = 0; t < 3; t++) s_f[3 * lane + t] = f3[t];
+        }
+      } else {
+        const int nsl = xhi - xlo + 1, nrw = yhi - ylo + 1;
+        for (int it = lane; it < 9 * nsl * nrw; it += kWideThreads) {
+          const int st3 = it / 3, b = it - 3 * st3, sl3 = st3 / nrw, rw = st3 - nrw * sl3;
+          const int ez = (sl3 >= nsl) + (sl3 >= 2 * nsl), sl = sl3 - nsl * ez;
+          const int rzi = ez == 0 ? rz[0] : ez == 1 ? rz[1] : rz[2];
+          const uint32_t off = ((uint32_t)wrapi(xlo + sl, g.nx) + (uint32_t)wrapi(ylo + rw, g.ny) * (uint32_t)g.nx +
+                                (uint32_t)wrapi(rzi + b, g.nz) * ((uint32_t)g.nx * (uint32_t)g.ny)) * 4u;
+          float f[27];
+          load27(src.f, off, f);
+          const float czb = ez != 1 ? (float)(ez - 1) * sq1 : 0.0f, Tzb = ez != 1 ? 0.0f : T1;
+          const NodePass np = node_pass(f, ldg4(src, off), u1x, u1xl, u1y, u1yl, u1z, u1zl, sqTb, czb, Tzb);
+#pragma unroll
+          for (int e = 0; e < 3; e++) {
+            float Tt[3];
+            node_group(np, e - 1, sq1, T1, Tt);
+#pragma unroll
+            for (int t = 0; t < 3; t++) s_T[it][3 * e + t] = Tt[t];
+          }
+        }
+        __syncthreads();
+        // y/z sums of every target's slices
+        for (int ch = lane; ch < 27 * nsl; ch += kWideThreads) {
+          const int sl = ch / 27, tg = ch - 27 * sl, ez = tg / 9, et = tg - 9 * ez, e = et / 3;
+          const int rye = e == 0 ? ry[0] : e == 1 ? ry[1] : ry[2];
+          float yz = 0.f;
+          for (int aa = 0; aa < 3; aa++) {  // the group's three rows
+            const int it = (ez * nsl + sl) * nrw + (rye + aa - ylo);
+#pragma unroll
+            for (int b = 0; b < 3; b++) {
+              const float wab = s_Fy[3 * e + aa] * s_Fz[3 * ez + b];
+              yz = __builtin_fmaf(wab, s_T[3 * it + b][et], yz);
+            }
+          }
+          s_yz[tg][sl] = yz;
+        }
+        __syncthreads();
+        // sub-stencil sums, smoothness samples and the WENO combination, one lane per target
+        if (lane < 27) {
+          const int ez = lane / 9, et = lane - 9 * ez, e = et / 3, t = et - 3 * e;
+          const int rt = t == 0 ? r[0] : t == 1 ? r[1] : r[2], rye = e == 0 ? ry[0] : e == 1 ? ry[1] : ry[2];
+          const float ct = t == 0 ? c[0] : t == 1 ? c[1] : c[2];
+          const float wz = ez != 1 ? h : mm;
+          const float wyz = ((e != 1) ? h : mm) * wz;
+          const float wt = (t != 1 ? h : mm) * wyz;
+          const int sl0 = (rt - 2) - xlo;  // the window's first slice
+          float S[3], ub[5];
+#pragma unroll
+          for (int k = 0; k < 3; k++) {
+            const float sk = ct + (float)(2 - k);
+            const float w0 = 0.5f * (sk - 1.0f) * (sk - 2.0f), w1 = -sk * (sk - 2.0f), w2 = 0.5f * sk * (sk - 1.0f);
+            float v = 0.f;
+            v = __builtin_fmaf(w0, s_yz[lane][sl0 + k], v);
+            v = __builtin_fmaf(w1, s_yz[lane][sl0 + k + 1], v);
+            v = __builtin_fmaf(w2, s_yz[lane][sl0 + k + 2], v);
+            S[k] = v * wt;
+          }
+#pragma unroll
+          for (int j = 0; j < 5; j++) ub[j] = s_T[3 * ((ez * nsl + sl0 + j) * nrw + (rye + 1 - ylo)) + 1][et] * wt;
+          s_f[lane] = weno5_combine(ct, ub, S);
+        }
+      }
+      __syncthreads();
+      SplitSums sums;
+#pragma unroll
+      for (int ey = 0; ey < 3; ey++)
+#pragma unroll
+        for (int ez = 0; ez < 3; ez++)
+#pragma unroll
+          for (int ex = 0; ex < 3; ex++) sums.add(ex - 1, ey - 1, ez - 1, s_f[9 * ez + 3 * ey + ex]);
+      conv = split27_update(sums, s, cell, min, Tin, st, a);
+    }
+    // BGK in FP32 (steps.cu:557-564) and the cell's outputs
+    const float rf = (float)st.rho, dt = (float)a.dtau;
+    if (lane < 27) {
+      const int ex = kE27[lane][0], ey = kE27[lane][1], ez = kE27[lane][2];
+      const float fi = s_f[9 * (ez + 1) + 3 * (ey + 1) + ex + 1];
+      fout[split27_fidx(lane, cell, P)] = __builtin_fmaf(dt, rf * a.w[lane] - fi, fi);
+    }
+    if (lane < 4) mout[lane * P + cell] = lane == 0 ? rf : (float)(lane == 1 ? st.gc[0] : lane == 2 ? st.gc[1] : st.gc[2]);
+    if (lane == 4) Tout[cell] = st.gc[3];
+    if (lane == 5) niter_out[cell] = st.niter;
+    __syncthreads();
   }
 }
 
@@ -1752,8 +1962,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
 }
 
 hipError_t launch_node_gauge(float* f, const float* m, const double* T, float* g4, int64_t n, int64_t plane,
-                             hipStream_t st) {
-  hipLaunchKernelGGL(k_node_gauge, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, f, m, T, g4, n, plane);
+                             int* pending_count, hipStream_t st) {
+  hipLaunchKernelGGL(k_node_gauge, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, f, m, T, g4, n, plane,
+                     pending_count);
   return hipGetLastError();
 }
 
@@ -1794,14 +2005,27 @@ hipError_t launch_step_split(int lattice, int interp, const SplitPtrs& in, const
     const dim3 nb((unsigned)((slots + cells - 1) / cells));
 #define POND_LAUNCH(I)                                                                                             \
   hipLaunchKernelGGL(k_step_split27_cells<I>, nb, dim3(64), 0, st, in.f, in.m, in.T, g4, out.f, out.m, out.T, niter, \
-                     guess, a, (int)cells)
-    if (interp == 2) POND_LAUNCH(2);
-    else if (a.g.mirror) POND_LAUNCH(3);
-    else POND_LAUNCH(1);
+                     guess, pend.count, a, (int)cells, wide_after)
+    // The iteration after which a cell goes to k_step_split27_wide.  A workgroup there serves a cell's
+    // iteration eight times sooner, but the chip gets through far fewer of them: early where the
+    // cells kernel leaves it idle.  ms per step for 4, 6, 8, 12, 16 and never, shock-bubble: 32^3 1.03, 0.98,
+    // 1.02, 1.18, 1.36, 5.29; 64^3 2.99, 2.67, 2.54, 2.53, 2.59, 6.70; 128^3 14.2, 12.9, 11.97, 11.61,
+    // 11.60, 14.5; 256^3 -, 73.9, 70.7, 69.5, 69.4, 69.8 (vortex, at most 10 iterations: 41.4, 39.82,
+    // 39.78, -, -, 39.74).
+    const int wide_after = a.g.n < (1 << 19) ? 8 : 16;
+    if (interp == 2) {
+      POND_LAUNCH(2);
+      const unsigned nw = (unsigned)(a.g.n < 1024 ? a.g.n : 1024);
+      hipLaunchKernelGGL(k_step_split27_wide, dim3(nw), dim3(kWideThreads), 0, st, in.f, in.m, in.T, g4, out.f, out.m, out.T, niter,
+                         pend.count, a);
+    } else if (a.g.mirror) {
+      POND_LAUNCH(3);
+    } else {
+      POND_LAUNCH(1);
+    }
 #undef POND_LAUNCH
     return hipGetLastError();
   }
-  hipLaunchKernelGGL(k_zero_count, dim3(1), dim3(64), 0, st, pend.count);
   // second-pass grid: enough waves to fill the chip several times, never more than the cells
   const int64_t w2 = (a.g.n + 63) / 64;
   const unsigned blocks2 = (unsigned)(w2 < 16384 ? w2 : 16384);
