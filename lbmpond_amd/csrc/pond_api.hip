@@ -742,7 +742,8 @@ pond_status pond_step(pond_ctx* ctx, int nsteps) {
       ctx->mlp_pending = true;
     }
     if (!ctx->split && !line && ctx->p.lattice != POND_D3Q125) {
-      he = launch_node_prep(ctx->p.lattice, ctx->f64[in].m, ctx->nodeP, ctx->g.n, ctx->g.plane, ctx->stream);
+      he = launch_node_prep(ctx->p.lattice, ctx->f64[in].m, ctx->nodeP, ctx->g.n, ctx->g.plane,
+                            pending_view(ctx).count, ctx->stream);
       if (he != hipSuccess) return fail(ctx, POND_ERR_HIP, std::string("node prep kernel: ") + hipGetErrorString(he));
     }
     // the event pair brackets the step kernel alone

@@ -57,7 +57,8 @@ struct MlpCtx {
   int* idx = nullptr;
 };
 
-hipError_t launch_node_prep(int lattice, const double* m, double* P, int64_t n, int64_t plane, hipStream_t st);
+hipError_t launch_node_prep(int lattice, const double* m, double* P, int64_t n, int64_t plane, int* pending_count,
+                            hipStream_t st);
 hipError_t launch_step_f64(int lattice, int interp, const double* fin, const double* min, const double* Pin,
                            double* fout, double* mout, int* niter, const Pending& pend, const StepArgs& a,
                            hipStream_t st);

@@ -65,7 +65,9 @@ __device__ __forceinline__ int64_t pending_slot(const Pending& p, bool pending, 
   return (int64_t)base + rank;
 }
 
-__global__ void k_zero_count(int* c);
+// D3Q27 steps use the list's memory as a plain list of slow cells, whose state waits in the step's
+// output buffers: entry 0 is their number, the cells start here
+constexpr int kSlowList = 64;
 
 __device__ __forceinline__ int isign_d(double v) { return (0.0 < v) - (v < 0.0); }
 

@@ -1099,7 +1099,8 @@ __device__ __forceinline__ void f64_group(const SRC& src, int x, int y, int z, i
 template <int INTERP, bool BUF>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_step_f64_27(
     const NodeSrc gsrc, double* __restrict__ fout, double* __restrict__ mout, int* __restrict__ niter_out,
-    const StepArgs a, int cells) {
+    int* __restrict__ slow, const StepArgs a, int cells, int wide_after) {
+  constexpr bool WENO = INTERP != 1 && INTERP != 3;
   using Src = typename std::conditional<BUF, NodeBuf, NodeSrc>::type;
   Src src;
   if constexpr (BUF) src = make_nodebuf(gsrc);
@@ -1186,8 +1187,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
       niter++;
 #pragma unroll
       for (int k = 0; k < 4; k++) c0[k] = mn[k];
-      if ((bad & 0x1ff) == 0 || niter >= a.max_iter) {
-        // BGK towards rho*w_i (steps.cu:557-564), two populations per lane and store
+      const bool done = (bad & 0x1ff) == 0 || niter >= a.max_iter;
+      if (done || (WENO && niter >= wide_after)) {
+        // BGK towards rho*w_i (steps.cu:557-564), two populations per lane and store; a cell left to
+        // k_step_f64_27_wide stores its iterate as it is
         active = false;
 #pragma unroll
         for (int h = 0; h < 2; h++) {
@@ -1198,7 +1201,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
             for (int k = 0; k < 2; k++) {
               f[k] = s_fn[slot][2 * p + k];
               const double feq = rho * s_w[2 * p + k];
-              f[k] += a.dtau * (feq - f[k]);
+              const double fb = f[k] + a.dtau * (feq - f[k]);
+              f[k] = !WENO || done ? fb : f[k];
             }
             if (p < 13) reinterpret_cast<double2*>(fout)[p * P + cell] = make_double2(f[0], f[1]);
             else fout[(p * P + cell) * 2] = f[0];
@@ -1206,9 +1210,153 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
         }
         if (gi < 5) mout[gi * P + cell] = gi == 0 ? rho : gi == 1 ? m0 : gi == 2 ? m1 : gi == 3 ? m2 : m3;
         if (gi == 5) niter_out[cell] = niter;
+        if (WENO && !done && gi == 6) slow[kSlowList + atomicAdd(slow, 1)] = (int)cell;
       }
     }
     wave_lds_order();
+  }
+}
+
+// The WENO5 cells that k_step_f64_27 left unconverged: one workgroup per cell.
+//
+// A few cells on shocks and contacts go on to the cap of 100 iterations, and nine lanes take 100 us for
+// such an iteration (63 chained steps of one node).  Here the (target, window position, node) transfers
+// of an iteration, 1215 or 1350 of them, are spread over the threads and laid down in LDS; the 81
+// sub-stencil sums run over them in the order of interp_weno5, one thread each, and one wave forms the
+// 27 values and the moments.  Bound by the chain of these parts (128 to 512 threads take the same time
+// within 4 %).  Shock-bubble, ms per step before and after: 32^3 10.4 -> 4.1, 64^3 20.5 -> 16.9, 100^3
+// 54.4 -> 52.1; 33x18x14 vortex (at most 10 iterations) 0.81 -> 0.65.
+constexpr int kWideThreads64 = 256;
+template <int VAR>
+__global__ __launch_bounds__(kWideThreads64) void k_step_f64_27_wide(const NodeSrc src, double* __restrict__ fout,
+                                                                    double* __restrict__ mout,
+                                                                    int* __restrict__ niter_out,
+                                                                    const int* __restrict__ slow, const StepArgs a) {
+  constexpr bool CENTRED = VAR == 1;
+  __shared__ double s_T[27 * 5][10];  // target, window position: the nodes (a, b) and (as written) the sample
+  __shared__ double s_S[27][3];       // sub-stencil sums
+  __shared__ double s_fn[27];         // the iterate, [9 (ey+1) + 3 (ez+1) + ex+1]
+  __shared__ double s_g[4];
+  __shared__ int s_conv;
+  const Grid& g = a.g;
+  const int64_t P = g.plane;
+  const int tid = threadIdx.x;
+  const int count = *slow;
+  for (int64_t e0 = blockIdx.x; e0 < count; e0 += gridDim.x) {
+    const int64_t cell = slow[kSlowList + e0];
+    const int x = (int)(cell % g.nx), y = (int)((cell / g.nx) % g.ny), z = (int)(cell / ((int64_t)g.nx * g.ny));
+    double uT[4], rho = 0, fo = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) uT[k] = mout[(k + 1) * P + cell];
+    const int ti = tid < 27 ? tid : 0;  // target of a thread of the tail
+    const int te = ti / 9 - 1, tz = (ti / 3) % 3 - 1, tx = ti % 3 - 1;
+    const int idx = kIdx27.v[tx + 1][te + 1][tz + 1];
+    if (tid < 27) fo = fout[f64_fidx(kD3Q27, idx, cell, P)];
+    int niter = niter_out[cell];
+    bool conv = false;
+    while (!conv && niter < a.max_iter) {
+      niter++;
+      const double s = sqrt(uT[3] / a.tlat);
+      // transfers of the nodes (a, b) of every target's window position j, and its sample
+      constexpr int NI = CENTRED ? 9 : 10;
+#pragma unroll 1
+      for (int it = tid; it < 27 * 5 * NI; it += kWideThreads64) {
+        const int tj = it / NI, q = it - NI * tj, tg = tj / 5, j = tj - 5 * tg;
+        const int ey = tg / 9 - 1, ez = (tg / 3) % 3 - 1, ex = tg % 3 - 1;
+        const Tgt27 t = make_tgt27e(ex, ey, ez, uT[0], uT[1], uT[2], uT[3]);
+        const double cx = (double)x - (s * (double)ex + uT[0]);
+        const double cy = (double)y - (s * (double)ey + uT[1]), cz = (double)z - (s * (double)ez + uT[2]);
+        const int r = floor_int(cx + 0.5);
+        const int ry = floor_int(cy + 0.5) - (CENTRED ? 1 : 0), rz = floor_int(cz + 0.5) - (CENTRED ? 1 : 0);
+        const int yn = q < 9 ? ry + q / 3 : r, zn = q < 9 ? rz + q % 3 : r;
+        s_T[tj][q] = transfer27(src, node_off(g, wrapi(r - 2 + j, g.nx), wrapi(yn, g.ny), wrapi(zn, g.nz)), t,
+                                a.sqrt_tbase);
+      }
+      __syncthreads();
+      // sums of a target's sub-stencil, in the order of interp_weno5
+      if (tid < 81) {
+        const int tg = tid / 3, q = tid - 3 * tg;
+        const int ey = tg / 9 - 1, ez = (tg / 3) % 3 - 1, ex = tg % 3 - 1;
+        const double cx = (double)x - (s * (double)ex + uT[0]);
+        const double cy = (double)y - (s * (double)ey + uT[1]), cz = (double)z - (s * (double)ez + uT[2]);
+        const int r = floor_int(cx + 0.5);
+        const int ry = floor_int(cy + 0.5) - (CENTRED ? 1 : 0), rz = floor_int(cz + 0.5) - (CENTRED ? 1 : 0);
+        double Fx[3][2], Fy[3][2], Fz[3][2];
+        lag3_factors(cx - (r - 2 + q), Fx);
+        lag3_factors(cy - ry, Fy);
+        lag3_factors(cz - rz, Fz);
+        double S = 0;
+#pragma unroll
+        for (int ix = 0; ix < 3; ix++) {
+          const double p = 1 * Fx[ix][0] * Fx[ix][1];
+#pragma unroll
+          for (int aa = 0; aa < 3; aa++)
+#pragma unroll
+            for (int b = 0; b < 3; b++)
+              S += p * Fy[aa][0] * Fy[aa][1] * Fz[b][0] * Fz[b][1] * s_T[5 * tg + q + ix][3 * aa + b];
+        }
+        s_S[tg][q] = S;
+      }
+      __syncthreads();
+      if (tid < 64) {
+        double fn = 0;
+        if (tid < 27) {
+          const double cx = (double)x - (s * (double)tx + uT[0]);
+          const int r = floor_int(cx + 0.5);
+          double ub[5];
+#pragma unroll
+          for (int j = 0; j < 5; j++) ub[j] = s_T[5 * tid + j][CENTRED ? 4 : 9];
+          fn = weno5_combine_f64<VAR>(cx - r, ub, s_S[tid][0], s_S[tid][1], s_S[tid][2]);
+          s_fn[idx] = fn;
+        }
+        bool same = true;
+        if (tid < 27 && fabs(fn - fo) >= a.tol_abs + a.tol_rel * fabs(fn)) same = false;
+        fo = fn;
+        wave_lds_order();
+        // Cell::calcMoments: lane q < 5 sums moment q over the populations in order, as in k_step_f64_27
+        const int mq = tid < 5 ? tid : 0;
+        double wx[3], wy[3], wz[3];
+#pragma unroll
+        for (int e = 0; e < 3; e++) {
+          const double vx = s * (double)(e - 1) + uT[0], vy = s * (double)(e - 1) + uT[1],
+                       vz = s * (double)(e - 1) + uT[2];
+          wx[e] = mq == 0 ? 1.0 : mq == 1 ? vx : mq == 4 ? vx * vx : 0.0;
+          wy[e] = mq == 2 ? vy : mq == 4 ? vy * vy : 0.0;
+          wz[e] = mq == 3 ? vz : mq == 4 ? vz * vz : 0.0;
+        }
+        double acc = 0;
+#pragma unroll
+        for (int i = 0; i < 27; i++) acc += s_fn[i] * (wx[kE27[i][0] + 1] + wy[kE27[i][1] + 1] + wz[kE27[i][2] + 1]);
+        rho = __shfl(acc, 0, 64);
+        if (rho != 0) acc /= rho;
+        const double m0 = __shfl(acc, 1, 64), m1 = __shfl(acc, 2, 64), m2 = __shfl(acc, 3, 64);
+        double m3 = __shfl(acc, 4, 64);
+        m3 = (m3 - m0 * m0 - m1 * m1 - m2 * m2) * a.inv_dim;
+        if (m3 < 0) m3 = uT[3];  // steps.cu:475-478
+        const double mn[4] = {m0, m1, m2, m3};
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+          if (fabs(mn[k] - uT[k]) >= a.tol_abs + a.tol_rel * fabs(mn[k])) same = false;
+        const bool all = __ballot(!same) == 0;
+        if (tid == 0) {
+#pragma unroll
+          for (int k = 0; k < 4; k++) s_g[k] = mn[k];
+          s_conv = all;
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < 4; k++) uT[k] = s_g[k];
+      conv = s_conv != 0;
+    }
+    // BGK towards rho*w_i (steps.cu:557-564) and the cell's outputs
+    if (tid < 27) {
+      const double feq = rho * a.w[idx];
+      fout[f64_fidx(kD3Q27, idx, cell, P)] = fo + a.dtau * (feq - fo);
+    }
+    if (tid < 5) mout[tid * P + cell] = tid == 0 ? rho : tid == 1 ? uT[0] : tid == 2 ? uT[1] : tid == 3 ? uT[2] : uT[3];
+    if (tid == 5) niter_out[cell] = niter;
+    __syncthreads();
   }
 }
 
@@ -1639,10 +1787,11 @@ __global__ __launch_bounds__(64) void k_step_line(const double* __restrict__ fin
 // host-side launchers
 
 // per-step node data of the load state: D3Q27 the gauge record (ux, uy, uz, P) of every cell, 32
-// bytes, D1Q5 the plane of P, with P = sqrt(|T|)*sign(T)
+// bytes, D1Q5 the plane of P, with P = sqrt(|T|)*sign(T); empties the step's list of pending cells
 __global__ void k_node_prep(const double* __restrict__ m, double* __restrict__ P, int64_t n, int64_t plane,
-                            bool record) {
+                            bool record, int* __restrict__ pending_count) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c == 0) *pending_count = 0;
   if (c >= n) return;
   const double Pc = sqrts_d(m[4 * plane + c]);
   if (record) {
@@ -1653,9 +1802,10 @@ __global__ void k_node_prep(const double* __restrict__ m, double* __restrict__ P
   }
 }
 
-hipError_t launch_node_prep(int lattice, const double* m, double* P, int64_t n, int64_t plane, hipStream_t st) {
+hipError_t launch_node_prep(int lattice, const double* m, double* P, int64_t n, int64_t plane, int* pending_count,
+                            hipStream_t st) {
   hipLaunchKernelGGL(k_node_prep, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, m, P, n, plane,
-                     lattice == kD3Q27);
+                     lattice == kD3Q27, pending_count);
   return hipGetLastError();
 }
 
@@ -1704,19 +1854,35 @@ hipError_t launch_step_f64(int lattice, int interp, const double* fin, const dou
     const dim3 nb((unsigned)((slots + cells - 1) / cells));
 #define POND_LAUNCH(I)                                                                                           \
   do {                                                                                                           \
-    if (buf) hipLaunchKernelGGL((k_step_f64_27<I, true>), nb, nt, 0, st, src, fout, mout, niter, a, (int)cells);   \
-    else hipLaunchKernelGGL((k_step_f64_27<I, false>), nb, nt, 0, st, src, fout, mout, niter, a, (int)cells);      \
+    if (buf) hipLaunchKernelGGL((k_step_f64_27<I, true>), nb, nt, 0, st, src, fout, mout, niter, pend.count, a, (int)cells, wide_after);   \
+    else hipLaunchKernelGGL((k_step_f64_27<I, false>), nb, nt, 0, st, src, fout, mout, niter, pend.count, a, (int)cells, wide_after);      \
   } while (0)
-    if (code == 0) POND_LAUNCH(0);
-    else if (code == 1) POND_LAUNCH(1);
-    else if (code == 3) POND_LAUNCH(3);
-    else if (code == 4) POND_LAUNCH(4);
-    else POND_LAUNCH(2);
+    // The iteration after which a WENO5 cell goes to k_step_f64_27_wide, early where the grid leaves the
+    // chip idle.  ms per step for 5, 6, 8, 12, 16 and never: 33x18x14 vortex 0.64, 0.65, 0.75, 0.84, -,
+    // 0.81; shock-bubble 32^3 -, 4.24, 4.10, 4.16, 4.20, 10.4; 64^3 -, 19.5, 17.6, 16.9, 16.9, 20.5;
+    // 100^3 -, 55.6, 53.2, 52.1, 52.1, 54.4; 128^3 -, -, 105, 99.7, 99.5, 99.1.
+    const int wide_after = a.g.n < (1 << 14) ? 6 : a.g.n < (1 << 17) ? 8 : 16;
+    const dim3 nw((unsigned)(a.g.n < 1024 ? a.g.n : 1024)), ntw(kWideThreads64);
+#define POND_WIDE(V) hipLaunchKernelGGL(k_step_f64_27_wide<V>, nw, ntw, 0, st, src, fout, mout, niter, pend.count, a)
+    if (code == 1) {
+      POND_LAUNCH(1);
+    } else if (code == 3) {
+      POND_LAUNCH(3);
+    } else if (code == 0) {
+      POND_LAUNCH(0);
+      POND_WIDE(0);
+    } else if (code == 4) {
+      POND_LAUNCH(4);
+      POND_WIDE(2);
+    } else {
+      POND_LAUNCH(2);
+      POND_WIDE(1);
+    }
+#undef POND_WIDE
 #undef POND_LAUNCH
     return hipGetLastError();
   }
   // D1Q5 off a line and long Lagrange-4 lines: one lane per cell, two passes
-  hipLaunchKernelGGL(k_zero_count, dim3(1), nt, 0, st, pend.count);
   const int64_t w2 = (a.g.n + 63) / 64;
   const dim3 nb1((unsigned)a.g.ntiles), nb2((unsigned)(w2 < 16384 ? w2 : 16384));
 #define POND_LAUNCH(I)                                                                                           \

@@ -1280,9 +1280,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
   }
 }
 
-// the list of slow cells: entry 0 is their number, the cells start here
-constexpr int kSlowList = 64;
-
 // WENO5C and Lagrange-4 (INTERP 2, 1; 3: Lagrange-4 with mirror walls): three lanes per cell, lane =
 // ez pass of nine targets, 21 cells per wave.
 //
@@ -1570,10 +1567,6 @@ __global__ __launch_bounds__(kWideThreads) void k_step_split27_wide(
     if (lane == 5) niter_out[cell] = st.niter;
     __syncthreads();
   }
-}
-
-__global__ void k_zero_count(int* c) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *c = 0;
 }
 
 // ---------------------------------------------------------------------------------------------
