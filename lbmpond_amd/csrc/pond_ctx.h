@@ -99,6 +99,7 @@ struct pond_ctx {
   int* cell_setnew = nullptr;
   double* red = nullptr;    // reduction partials
   int64_t red_len = 0;
+  char* pinned = nullptr;   // host buffers of large reads, allocated by the first one
   int64_t step = 0;
   int64_t bytes = 0;
   // timing of the step kernel launches (HIP events on `stream`)
