@@ -37,15 +37,14 @@ struct MlpState {
 
 hipError_t mlp_launch_infer(const MlpWeightsBF& w, const MlpState& s, float* out, int64_t out_plane, hipStream_t st);
 hipError_t mlp_launch_infer_matrix(const MlpWeightsBF& w, const float* X, int64_t n, float* out, hipStream_t st);
-hipError_t mlp_gemm(const unsigned short* A, int64_t sai, int64_t sak, const unsigned short* B, int64_t sbk,
-                    int64_t sbj, float* C, int64_t ldc, int M, int N, int K, int accum, hipStream_t st);
-hipError_t mlp_bias_relu(const float* Zacc, const float* bias, float* Z, unsigned short* Ab, int rows, int cols, int ld,
-                         int relu, hipStream_t st);
-hipError_t mlp_out_grad(const float* Y, const float* T, float* dY, unsigned short* dYb, float* sqerr, int B, int nout,
-                        int ld, hipStream_t st);
-hipError_t mlp_relu_grad(const float* G, const float* Z, float* dZ, unsigned short* dZb, int64_t n, hipStream_t st);
-hipError_t mlp_colsum(const float* M, int rows, int cols, int ld, float* out, hipStream_t st);
-hipError_t mlp_sum(const float* v, int n, float* out, hipStream_t st);
+// Blocks of a minibatch's gradient pass (B rows, a multiple of 16): 64 rows each, at most 256 (one per
+// CU, each then taking several); a block leaves kMlpGradStride floats of partial sums.
+constexpr int kMlpGradStride = (kMlpParams + 1 + 63) / 64 * 64;
+inline int mlp_grad_blocks(int B) { return (B + 63) / 64 < 256 ? (B + 63) / 64 : 256; }
+// gradients of the mean squared error (2/B (y - t) per row) and, in grad[kMlpParams], the summed
+// squared error; X, T: B normalized feature and target rows
+hipError_t mlp_grad(const MlpWeightsBF& w, const float* X, const float* T, int B, float* part, float* grad,
+                    hipStream_t st);
 hipError_t mlp_to_bf16(const float* src, int rows, int cols, int src_ld, unsigned short* dst, int ld, hipStream_t st);
 hipError_t mlp_adam(float* p, const float* g, float* m, float* v, int n, float lr, float b1, float b2, float eps,
                     float c1, float c2, hipStream_t st);

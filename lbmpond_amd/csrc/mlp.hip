@@ -290,112 +290,241 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 
 // ------------------------------------------------------------------------ training pieces
 
-// generic tile GEMM C[M][N] (+)= sum_k A(i,k) B(k,j), bf16 operands, FP32 accumulation.
-// A(i,k) = A[i*sai + k*sak], B(k,j) = B[k*sbk + j*sbj]; one wave per 16x16 tile of C.
-__global__ __launch_bounds__(64) void k_gemm_bf16(const unsigned short* __restrict__ A, int64_t sai, int64_t sak,
-                                                  const unsigned short* __restrict__ B, int64_t sbk, int64_t sbj,
-                                                  float* __restrict__ C, int64_t ldc, int M, int N, int K, int accum) {
-  const int l = threadIdx.x;
-  const int q = l >> 4, col = l & 15;
-  const int ti = blockIdx.x, tj = blockIdx.y;
-  float4_t acc = {0.f, 0.f, 0.f, 0.f};
-  const int i = 16 * ti + col;  // A row held by this lane
-  const int j = 16 * tj + col;  // B column held by this lane
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    short4_t av, bv;
+// Forward and backward pass of a minibatch, gradients summed per block (k_mlp_grad), then over the
+// blocks (k_mlp_grad_sum).
+//
+// A block takes 64 rows at a time, 16 per wave.  With A[i][k] and B[k][j] of the same register layout,
+// the same two registers give a product (rows on j) and its transpose (rows on i), so every layer is
+// formed both ways: with the units in a lane's registers it is the next layer's operand, with the rows
+// there it is an operand of the weight gradients (sums over rows), and nothing is transposed in
+// memory.  The weight gradients' operands go through LDS to all four waves; each wave keeps 14 of
+// the 56 gradient tiles in registers.  BF16 rounding points and the order over k in every product
+// over units or features are those of separate GEMMs per layer.
+//
+// The chain of one tile bounds it (about 170 matrix instructions and the loads of the weights).  As
+// fifteen launches with one wave per gradient tile running down all the rows, a pass over 4096
+// rows took 430 us on the GPU (82 % in the one-wave GEMMs); now 21 + 4 us, and a batch given from
+// the host 550 -> 154 us, most of what is left being the copies of the batch.
+constexpr int kGradBlkX = 0;    // operand blocks of a wave, 64 lanes x 4 bf16 each: x, rows in registers (9)
+constexpr int kGradBlkN = 9;    // first x, features in registers (9); then h1 (4), h2 (4) and dy (1)
+constexpr int kGradBlkD = 18;   // dz2 (4), dz1 (4)
+constexpr int kGradBlks = 26;
+
+// relu'(z) of four values
+__device__ __forceinline__ float4_t relu_mask(const float4_t& g, const float4_t& z) {
+  float4_t d;
+#pragma unroll
+  for (int e = 0; e < 4; e++) d[e] = z[e] > 0.f ? g[e] : 0.f;
+  return d;
+}
+
+__global__ __launch_bounds__(256) void k_mlp_grad(const MlpWeightsBF w, const float* __restrict__ X,
+                                                  const float* __restrict__ T, int B, float* __restrict__ part) {
+  __shared__ short4_t s_op[4][kGradBlks][64];
+  __shared__ float s_b[4][2 * kMlpH + kMlpOut + 1];
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, q = lane >> 4, col = lane & 15;
+  const short4_t zero4 = {0, 0, 0, 0};
+  const float4_t zf = {0.f, 0.f, 0.f, 0.f};
+  // weights: lane's unit (output) on the first axis, four consecutive k on the second
+  short4_t w1[4][9], w2[4][4], w3[4], w2r[4][4], w3r[4];
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+#pragma unroll
+    for (int k = 0; k < 9; k++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) w1[t][k][e] = (short)w.W1[(16 * k + 4 * q + e) * kMlpH + 16 * t + col];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+#pragma unroll
+      for (int e = 0; e < 4; e++) w2[t][k][e] = (short)w.W2[(16 * k + 4 * q + e) * kMlpH + 16 * t + col];
+      w2r[t][k] = *reinterpret_cast<const short4_t*>(w.W2 + (16 * t + col) * kMlpH + 16 * k + 4 * q);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) w3[t][e] = (short)w.W3[(16 * t + 4 * q + e) * kMlpOutPad + col];
+    w3r[t] = *reinterpret_cast<const short4_t*>(w.W3 + (16 * t + col) * kMlpOutPad + 4 * q);
+  }
+  float4_t b1t[4], b2t[4];
+  float b1n[4], b2n[4];
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      const int k = k0 + 4 * q + e;
-      av[e] = (short)((i < M && k < K) ? A[i * sai + k * sak] : 0);
-      bv[e] = (short)((j < N && k < K) ? B[k * sbk + j * sbj] : 0);
+      b1t[t][e] = w.b1[16 * t + 4 * q + e];
+      b2t[t][e] = w.b2[16 * t + 4 * q + e];
     }
-    acc = mfma16(av, bv, acc);
+    b1n[t] = w.b1[16 * t + col];
+    b2n[t] = w.b2[16 * t + col];
   }
+  const float b3n = col < kMlpOut ? w.b3[col] : 0.f;
+  float4_t g1[9], g2[4], g3 = zf;  // gradient tiles: W1 (features k, units 16 wv), W2 (k, 16 wv), W3 (16 wv)
 #pragma unroll
-  for (int e = 0; e < 4; e++) {
-    const int r = 16 * ti + 4 * q + e;
-    if (r < M && j < N) {
-      float* p = C + (int64_t)r * ldc + j;
-      *p = accum ? *p + acc[e] : acc[e];
+  for (int k = 0; k < 9; k++) g1[k] = zf;
+#pragma unroll
+  for (int k = 0; k < 4; k++) g2[k] = zf;
+  float sb1[4] = {0, 0, 0, 0}, sb2[4] = {0, 0, 0, 0}, sb3 = 0.f, se = 0.f;
+  const int tiles = B / 16;
+  for (int tb = 4 * blockIdx.x; tb < tiles; tb += 4 * gridDim.x) {
+    const int tile = tb + wv;
+    short4_t(*op)[64] = s_op[wv];
+    if (tile < tiles) {
+      // the tile's 16 x 135 features, rounded and laid out both ways (the padding is zero)
+      op[kGradBlkX + 8][lane] = zero4;
+      op[kGradBlkN + 8][lane] = zero4;
+      wave_lds_order();
+      const float4_t* xs = reinterpret_cast<const float4_t*>(X + (int64_t)tile * 16 * kMlpIn);
+#pragma unroll
+      for (int n = 0; n < 9; n++) {
+        const int i4 = 64 * n + lane;
+        if (i4 < 16 * kMlpIn / 4) {
+          const float4_t v = xs[i4];
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const int r = (4 * i4 + e) / kMlpIn, f = 4 * i4 + e - kMlpIn * r, fl = f & 15;
+            const short h = f2bf(v[e]);
+            reinterpret_cast<short*>(&op[kGradBlkX + (f >> 4)][16 * (r >> 2) + fl])[r & 3] = h;
+            reinterpret_cast<short*>(&op[kGradBlkN + (f >> 4)][16 * (fl >> 2) + r])[fl & 3] = h;
+          }
+        }
+      }
+      wave_lds_order();
+      short4_t x[9], h1[4], h2[4], h1n[4], h2n[4], d2[4];
+#pragma unroll
+      for (int k = 0; k < 9; k++) x[k] = op[kGradBlkN + k][lane];
+      float4_t z1n[4], z2t[4], z2n[4];
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        float4_t a = zf, n = zf;
+#pragma unroll
+        for (int k = 0; k < 9; k++) {
+          a = mfma16(w1[t][k], x[k], a);
+          n = mfma16(x[k], w1[t][k], n);
+        }
+        a += b1t[t];
+        z1n[t] = n + b1n[t];
+        h1[t] = pack_bf16x4(fmaxf(a[0], 0.f), fmaxf(a[1], 0.f), fmaxf(a[2], 0.f), fmaxf(a[3], 0.f));
+        h1n[t] = pack_bf16x4(fmaxf(z1n[t][0], 0.f), fmaxf(z1n[t][1], 0.f), fmaxf(z1n[t][2], 0.f), fmaxf(z1n[t][3], 0.f));
+      }
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        float4_t a = zf, n = zf;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          a = mfma16(w2[t][k], h1[k], a);
+          n = mfma16(h1[k], w2[t][k], n);
+        }
+        z2t[t] = a + b2t[t];
+        z2n[t] = n + b2n[t];
+        h2[t] = pack_bf16x4(fmaxf(z2t[t][0], 0.f), fmaxf(z2t[t][1], 0.f), fmaxf(z2t[t][2], 0.f), fmaxf(z2t[t][3], 0.f));
+        h2n[t] = pack_bf16x4(fmaxf(z2n[t][0], 0.f), fmaxf(z2n[t][1], 0.f), fmaxf(z2n[t][2], 0.f), fmaxf(z2n[t][3], 0.f));
+      }
+      float4_t yt = zf, yn = zf;
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        yt = mfma16(w3[k], h2[k], yt);
+        yn = mfma16(h2[k], w3[k], yn);
+      }
+      // dY = 2 (Y - T)/B: outputs 0..3 of row col in the lanes with q = 0, rows 4q.. of output col < 4
+      float4_t dt = zf, dn = zf;
+      const int64_t row0 = (int64_t)tile * 16;
+      if (q == 0) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const float er = yt[e] + w.b3[e] - T[(row0 + col) * kMlpOut + e];
+          se += er * er;
+          dt[e] = 2.0f * er / (float)B;
+        }
+      }
+      if (col < kMlpOut) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) dn[e] = 2.0f * (yn[e] + b3n - T[(row0 + 4 * q + e) * kMlpOut + col]) / (float)B;
+      }
+      sb3 += (dn[0] + dn[1]) + (dn[2] + dn[3]);
+      const short4_t db = pack_bf16x4(dt[0], dt[1], dt[2], dt[3]);
+      op[kGradBlkN + 8][lane] = pack_bf16x4(dn[0], dn[1], dn[2], dn[3]);
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        op[kGradBlkN + t][lane] = h1n[t];
+        op[kGradBlkN + 4 + t][lane] = h2n[t];
+        const float4_t d = relu_mask(mfma16(w3r[t], db, zf), z2t[t]);
+        const float4_t n = relu_mask(mfma16(db, w3r[t], zf), z2n[t]);
+        d2[t] = pack_bf16x4(d[0], d[1], d[2], d[3]);
+        op[kGradBlkD + t][lane] = pack_bf16x4(n[0], n[1], n[2], n[3]);
+        sb2[t] += (n[0] + n[1]) + (n[2] + n[3]);
+      }
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        float4_t n = zf;
+#pragma unroll
+        for (int k = 0; k < 4; k++) n = mfma16(d2[k], w2r[t][k], n);
+        n = relu_mask(n, z1n[t]);
+        op[kGradBlkD + 4 + t][lane] = pack_bf16x4(n[0], n[1], n[2], n[3]);
+        sb1[t] += (n[0] + n[1]) + (n[2] + n[3]);
+      }
     }
-  }
-}
-
-// Z = Zacc + bias (FP32), A = bf16(relu(Z)) ; rows x cols, row stride ld
-__global__ void k_bias_relu(const float* __restrict__ Zacc, const float* __restrict__ bias, float* __restrict__ Z,
-                            unsigned short* __restrict__ Ab, int rows, int cols, int ld, int relu) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (int64_t)rows * ld) return;
-  const int c = (int)(t % ld);
-  if (c >= cols) {
-    Ab[t] = 0;
-    Z[t] = 0.f;
-    return;
-  }
-  const float z = Zacc[t] + bias[c];
-  Z[t] = z;
-  Ab[t] = f2bf(relu ? fmaxf(z, 0.f) : z);
-}
-
-// dY = 2 (Y - T)/B (FP32, padded to ld columns), dYb = bf16(dY), per-row squared error
-__global__ void k_out_grad(const float* __restrict__ Y, const float* __restrict__ T, float* __restrict__ dY,
-                           unsigned short* __restrict__ dYb, float* __restrict__ sqerr, int B, int nout, int ld) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B) return;
-  float se = 0.f;
-  for (int c = 0; c < ld; c++) {
-    float d = 0.f;
-    if (c < nout) {
-      const float e = Y[(int64_t)b * ld + c] - T[(int64_t)b * nout + c];
-      se += e * e;
-      d = 2.0f * e / (float)B;
+    __syncthreads();
+    const int live = tiles - tb < 4 ? tiles - tb : 4;
+    for (int r = 0; r < live; r++) {
+      const short4_t d1 = s_op[r][kGradBlkD + 4 + wv][lane], d2v = s_op[r][kGradBlkD + wv][lane];
+#pragma unroll
+      for (int k = 0; k < 9; k++) g1[k] = mfma16(s_op[r][kGradBlkX + k][lane], d1, g1[k]);
+#pragma unroll
+      for (int k = 0; k < 4; k++) g2[k] = mfma16(s_op[r][kGradBlkN + k][lane], d2v, g2[k]);
+      g3 = mfma16(s_op[r][kGradBlkN + 4 + wv][lane], s_op[r][kGradBlkN + 8][lane], g3);
     }
-    dY[(int64_t)b * ld + c] = d;
-    dYb[(int64_t)b * ld + c] = f2bf(d);
-  }
-  sqerr[b] = se;
-}
-
-// dZ = G * (Z > 0), dZb = bf16(dZ)
-__global__ void k_relu_grad(const float* __restrict__ G, const float* __restrict__ Z, float* __restrict__ dZ,
-                            unsigned short* __restrict__ dZb, int64_t n) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const float d = Z[t] > 0.f ? G[t] : 0.f;
-  dZ[t] = d;
-  dZb[t] = f2bf(d);
-}
-
-// column sums of a rows x cols matrix (row stride ld) into out[cols] (bias gradients)
-// column sums of a rows x cols matrix (stride ld): one 256-thread block per column
-__global__ __launch_bounds__(256) void k_colsum(const float* __restrict__ M, int rows, int cols, int ld,
-                                                float* __restrict__ out) {
-  __shared__ float sh[256];
-  const int c = blockIdx.x;
-  if (c >= cols) return;
-  float s = 0.f;
-  for (int r = threadIdx.x; r < rows; r += 256) s += M[(int64_t)r * ld + c];
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[c] = sh[0];
+  // the block's sums
+  float* o = part + (int64_t)blockIdx.x * kMlpGradStride;
+#pragma unroll
+  for (int k = 0; k < 9; k++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int f = 16 * k + 4 * q + e;
+      if (f < kMlpIn) o[kOffW1 + f * kMlpH + 16 * wv + col] = g1[k][e];
+    }
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) o[kOffW2 + (16 * k + 4 * q + e) * kMlpH + 16 * wv + col] = g2[k][e];
+  if (col < kMlpOut)
+#pragma unroll
+    for (int e = 0; e < 4; e++) o[kOffW3 + (16 * wv + 4 * q + e) * kMlpOut + col] = g3[e];
+  auto over_q = [](float v) {
+    v += __shfl_xor(v, 16, 64);
+    return v + __shfl_xor(v, 32, 64);
+  };
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    const float v1 = over_q(sb1[t]), v2 = over_q(sb2[t]);
+    if (q == 0) {
+      s_b[wv][16 * t + col] = v1;
+      s_b[wv][kMlpH + 16 * t + col] = v2;
+    }
+  }
+  const float v3 = over_q(sb3);
+  if (lane < kMlpOut) s_b[wv][2 * kMlpH + lane] = v3;
+#pragma unroll
+  for (int m = 1; m < 16; m <<= 1) se += __shfl_xor(se, m, 64);  // (lanes 0..15 hold the rows' errors)
+  if (lane == 0) s_b[wv][2 * kMlpH + kMlpOut] = se;
+  __syncthreads();
+  for (int i = threadIdx.x; i < 2 * kMlpH + kMlpOut + 1; i += 256) {
+    const float v = (s_b[0][i] + s_b[1][i]) + (s_b[2][i] + s_b[3][i]);
+    o[i < kMlpH ? kOffB1 + i : i < 2 * kMlpH ? kOffB2 + i - kMlpH : kOffB3 + i - 2 * kMlpH] = v;
+  }
 }
 
-// sum of n values, one 256-thread block
-__global__ __launch_bounds__(256) void k_sum(const float* __restrict__ v, int n, float* __restrict__ out) {
-  __shared__ float sh[256];
+// sums of the blocks' gradients (and squared error, behind them): four threads per parameter
+__global__ __launch_bounds__(256) void k_mlp_grad_sum(const float* __restrict__ part, int blocks, float* __restrict__ out) {
+  __shared__ float sh[4][64];
+  const int c = threadIdx.x & 63, h = threadIdx.x >> 6;
+  const int i = blockIdx.x * 64 + c;
   float s = 0.f;
-  for (int i = threadIdx.x; i < n; i += 256) s += v[i];
-  sh[threadIdx.x] = s;
+  if (i <= kMlpParams)
+#pragma unroll 8
+    for (int b = h; b < blocks; b += 4) s += part[(int64_t)b * kMlpGradStride + i];
+  sh[h][c] = s;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *out = sh[0];
+  if (h == 0 && i <= kMlpParams) out[i] = (sh[0][c] + sh[1][c]) + (sh[2][c] + sh[3][c]);
 }
 
 // FP32 -> bf16 with row padding: src rows x cols (stride src_ld) -> dst rows x ld
@@ -544,40 +673,13 @@ hipError_t mlp_launch_infer_matrix(const MlpWeightsBF& w, const float* X, int64_
   return hipGetLastError();
 }
 
-hipError_t mlp_gemm(const unsigned short* A, int64_t sai, int64_t sak, const unsigned short* B, int64_t sbk,
-                    int64_t sbj, float* C, int64_t ldc, int M, int N, int K, int accum, hipStream_t st) {
-  hipLaunchKernelGGL(k_gemm_bf16, dim3((M + 15) / 16, (N + 15) / 16), dim3(64), 0, st, A, sai, sak, B, sbk, sbj, C,
-                     ldc, M, N, K, accum);
-  return hipGetLastError();
-}
-
 static unsigned nb(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
-hipError_t mlp_bias_relu(const float* Zacc, const float* bias, float* Z, unsigned short* Ab, int rows, int cols, int ld,
-                         int relu, hipStream_t st) {
-  hipLaunchKernelGGL(k_bias_relu, dim3(nb((int64_t)rows * ld, 256)), dim3(256), 0, st, Zacc, bias, Z, Ab, rows, cols,
-                     ld, relu);
-  return hipGetLastError();
-}
-
-hipError_t mlp_out_grad(const float* Y, const float* T, float* dY, unsigned short* dYb, float* sqerr, int B, int nout,
-                        int ld, hipStream_t st) {
-  hipLaunchKernelGGL(k_out_grad, dim3(nb(B, 256)), dim3(256), 0, st, Y, T, dY, dYb, sqerr, B, nout, ld);
-  return hipGetLastError();
-}
-
-hipError_t mlp_relu_grad(const float* G, const float* Z, float* dZ, unsigned short* dZb, int64_t n, hipStream_t st) {
-  hipLaunchKernelGGL(k_relu_grad, dim3(nb(n, 256)), dim3(256), 0, st, G, Z, dZ, dZb, n);
-  return hipGetLastError();
-}
-
-hipError_t mlp_colsum(const float* M, int rows, int cols, int ld, float* out, hipStream_t st) {
-  hipLaunchKernelGGL(k_colsum, dim3((unsigned)cols), dim3(256), 0, st, M, rows, cols, ld, out);
-  return hipGetLastError();
-}
-
-hipError_t mlp_sum(const float* v, int n, float* out, hipStream_t st) {
-  hipLaunchKernelGGL(k_sum, dim3(1), dim3(256), 0, st, v, n, out);
+hipError_t mlp_grad(const MlpWeightsBF& w, const float* X, const float* T, int B, float* part, float* grad,
+                    hipStream_t st) {
+  const int blocks = mlp_grad_blocks(B);
+  hipLaunchKernelGGL(k_mlp_grad, dim3((unsigned)blocks), dim3(256), 0, st, w, X, T, B, part);
+  hipLaunchKernelGGL(k_mlp_grad_sum, dim3(nb(kMlpParams + 1, 64)), dim3(256), 0, st, part, blocks, grad);
   return hipGetLastError();
 }
 

@@ -37,13 +37,12 @@ pond_status mlp_alloc(pond_ctx* ctx) {
   MlpCtx& m = ctx->mlp;
   if (m.params) return POND_OK;
   MLP_HIP(ctx, dalloc(ctx, &m.params, kMlpParams));
-  MLP_HIP(ctx, dalloc(ctx, &m.grad, kMlpParams));
+  MLP_HIP(ctx, dalloc(ctx, &m.grad, kMlpParams + 1));
   MLP_HIP(ctx, dalloc(ctx, &m.adam_m, kMlpParams));
   MLP_HIP(ctx, dalloc(ctx, &m.adam_v, kMlpParams));
   MLP_HIP(ctx, dalloc(ctx, &m.W1b, (size_t)kMlpInPad * kMlpH));
   MLP_HIP(ctx, dalloc(ctx, &m.W2b, (size_t)kMlpH * kMlpH));
   MLP_HIP(ctx, dalloc(ctx, &m.W3b, (size_t)kMlpH * kMlpOutPad));
-  MLP_HIP(ctx, dalloc(ctx, &m.gw3tmp, (size_t)kMlpH * kMlpOutPad));
   MLP_HIP(ctx, dalloc(ctx, &m.mom, (size_t)16));
   MLP_HIP(ctx, hipMemsetAsync(m.W1b, 0, (size_t)kMlpInPad * kMlpH * 2, ctx->stream));
   MLP_HIP(ctx, hipMemsetAsync(m.W3b, 0, (size_t)kMlpH * kMlpOutPad * 2, ctx->stream));
@@ -55,36 +54,15 @@ pond_status mlp_alloc(pond_ctx* ctx) {
 pond_status mlp_batch_alloc(pond_ctx* ctx, int B) {
   MlpCtx& m = ctx->mlp;
   if (m.bcap >= B) return POND_OK;
-  float** fbufs[] = {&m.bx, &m.bt, &m.z1acc, &m.z1, &m.z2acc, &m.z2, &m.yacc, &m.y, &m.dy, &m.g2, &m.dz2, &m.g1,
-                     &m.dz1, &m.sqerr, &m.loss};
+  float** fbufs[] = {&m.bx, &m.bt, &m.part};
   for (auto p : fbufs)
     if (*p) { (void)hipFree(*p); *p = nullptr; }
-  unsigned short** hbufs[] = {&m.xb, &m.a1b, &m.a2b, &m.dyb, &m.dz2b, &m.dz1b};
-  for (auto p : hbufs)
-    if (*p) { (void)hipFree(*p); *p = nullptr; }
   if (m.idx) { (void)hipFree(m.idx); m.idx = nullptr; }
+  m.bcap = 0;
   const size_t b = (size_t)B;
   MLP_HIP(ctx, dalloc(ctx, &m.bx, b * kMlpIn));
   MLP_HIP(ctx, dalloc(ctx, &m.bt, b * kMlpOut));
-  MLP_HIP(ctx, dalloc(ctx, &m.z1acc, b * kMlpH));
-  MLP_HIP(ctx, dalloc(ctx, &m.z1, b * kMlpH));
-  MLP_HIP(ctx, dalloc(ctx, &m.z2acc, b * kMlpH));
-  MLP_HIP(ctx, dalloc(ctx, &m.z2, b * kMlpH));
-  MLP_HIP(ctx, dalloc(ctx, &m.yacc, b * kMlpOutPad));
-  MLP_HIP(ctx, dalloc(ctx, &m.y, b * kMlpOutPad));
-  MLP_HIP(ctx, dalloc(ctx, &m.dy, b * kMlpOutPad));
-  MLP_HIP(ctx, dalloc(ctx, &m.g2, b * kMlpH));
-  MLP_HIP(ctx, dalloc(ctx, &m.dz2, b * kMlpH));
-  MLP_HIP(ctx, dalloc(ctx, &m.g1, b * kMlpH));
-  MLP_HIP(ctx, dalloc(ctx, &m.dz1, b * kMlpH));
-  MLP_HIP(ctx, dalloc(ctx, &m.sqerr, b));
-  MLP_HIP(ctx, dalloc(ctx, &m.loss, 4));
-  MLP_HIP(ctx, dalloc(ctx, &m.xb, b * kMlpInPad));
-  MLP_HIP(ctx, dalloc(ctx, &m.a1b, b * kMlpH));
-  MLP_HIP(ctx, dalloc(ctx, &m.a2b, b * kMlpH));
-  MLP_HIP(ctx, dalloc(ctx, &m.dyb, b * kMlpOutPad));
-  MLP_HIP(ctx, dalloc(ctx, &m.dz2b, b * kMlpH));
-  MLP_HIP(ctx, dalloc(ctx, &m.dz1b, b * kMlpH));
+  MLP_HIP(ctx, dalloc(ctx, &m.part, (size_t)mlp_grad_blocks(B) * kMlpGradStride));
   MLP_HIP(ctx, dalloc(ctx, &m.idx, b));
   m.bcap = B;
   return POND_OK;
@@ -96,41 +74,6 @@ pond_status mlp_refresh_bf16(pond_ctx* ctx) {
   MLP_HIP(ctx, mlp_to_bf16(m.params + kOffW1, kMlpIn, kMlpH, kMlpH, m.W1b, kMlpH, ctx->stream));
   MLP_HIP(ctx, mlp_to_bf16(m.params + kOffW2, kMlpH, kMlpH, kMlpH, m.W2b, kMlpH, ctx->stream));
   MLP_HIP(ctx, mlp_to_bf16(m.params + kOffW3, kMlpH, kMlpOut, kMlpOut, m.W3b, kMlpOutPad, ctx->stream));
-  return POND_OK;
-}
-
-// forward + backward of one minibatch held in m.bx (normalized X) / m.bt (normalized T);
-// gradients land in m.grad, the summed squared error in m.loss[0].  Training holds the biases
-// at zero and skips their gradients (bias_grad = false); the gradient entry point computes all.
-pond_status mlp_fwd_bwd(pond_ctx* ctx, int B, bool bias_grad) {
-  MlpCtx& m = ctx->mlp;
-  hipStream_t st = ctx->stream;
-  const float* P = m.params;
-  MLP_HIP(ctx, mlp_to_bf16(m.bx, B, kMlpIn, kMlpIn, m.xb, kMlpInPad, st));
-  // forward
-  MLP_HIP(ctx, mlp_gemm(m.xb, kMlpInPad, 1, m.W1b, kMlpH, 1, m.z1acc, kMlpH, B, kMlpH, kMlpInPad, 0, st));
-  MLP_HIP(ctx, mlp_bias_relu(m.z1acc, P + kOffB1, m.z1, m.a1b, B, kMlpH, kMlpH, 1, st));
-  MLP_HIP(ctx, mlp_gemm(m.a1b, kMlpH, 1, m.W2b, kMlpH, 1, m.z2acc, kMlpH, B, kMlpH, kMlpH, 0, st));
-  MLP_HIP(ctx, mlp_bias_relu(m.z2acc, P + kOffB2, m.z2, m.a2b, B, kMlpH, kMlpH, 1, st));
-  MLP_HIP(ctx, mlp_gemm(m.a2b, kMlpH, 1, m.W3b, kMlpOutPad, 1, m.yacc, kMlpOutPad, B, kMlpOutPad, kMlpH, 0, st));
-  // y = yacc + b3 (no activation); the padded columns get bias 0 via cols = kMlpOut
-  MLP_HIP(ctx, mlp_bias_relu(m.yacc, P + kOffB3, m.y, m.dyb, B, kMlpOut, kMlpOutPad, 0, st));
-  // backward
-  MLP_HIP(ctx, mlp_out_grad(m.y, m.bt, m.dy, m.dyb, m.sqerr, B, kMlpOut, kMlpOutPad, st));
-  if (bias_grad) MLP_HIP(ctx, mlp_colsum(m.dy, B, kMlpOut, kMlpOutPad, m.grad + kOffB3, st));
-  MLP_HIP(ctx, mlp_gemm(m.a2b, 1, kMlpH, m.dyb, kMlpOutPad, 1, m.gw3tmp, kMlpOutPad, kMlpH, kMlpOutPad, B, 0, st));
-  // pack the 64x16 padded W3 gradient into the 64x4 parameter block
-  MLP_HIP(ctx, hipMemcpy2DAsync(m.grad + kOffW3, kMlpOut * sizeof(float), m.gw3tmp, kMlpOutPad * sizeof(float),
-                                kMlpOut * sizeof(float), kMlpH, hipMemcpyDeviceToDevice, st));
-  MLP_HIP(ctx, mlp_gemm(m.dyb, kMlpOutPad, 1, m.W3b, 1, kMlpOutPad, m.g2, kMlpH, B, kMlpH, kMlpOutPad, 0, st));
-  MLP_HIP(ctx, mlp_relu_grad(m.g2, m.z2, m.dz2, m.dz2b, (int64_t)B * kMlpH, st));
-  if (bias_grad) MLP_HIP(ctx, mlp_colsum(m.dz2, B, kMlpH, kMlpH, m.grad + kOffB2, st));
-  MLP_HIP(ctx, mlp_gemm(m.a1b, 1, kMlpH, m.dz2b, kMlpH, 1, m.grad + kOffW2, kMlpH, kMlpH, kMlpH, B, 0, st));
-  MLP_HIP(ctx, mlp_gemm(m.dz2b, kMlpH, 1, m.W2b, 1, kMlpH, m.g1, kMlpH, B, kMlpH, kMlpH, 0, st));
-  MLP_HIP(ctx, mlp_relu_grad(m.g1, m.z1, m.dz1, m.dz1b, (int64_t)B * kMlpH, st));
-  if (bias_grad) MLP_HIP(ctx, mlp_colsum(m.dz1, B, kMlpH, kMlpH, m.grad + kOffB1, st));
-  MLP_HIP(ctx, mlp_gemm(m.xb, 1, kMlpInPad, m.dz1b, kMlpH, 1, m.grad + kOffW1, kMlpH, kMlpIn, kMlpH, B, 0, st));
-  MLP_HIP(ctx, mlp_sum(m.sqerr, B, m.loss, st));
   return POND_OK;
 }
 
@@ -190,9 +133,7 @@ MlpWeightsBF pond_mlp_weights(const pond_ctx* ctx) {
 
 void pond_mlp_free(pond_ctx* ctx) {
   MlpCtx& m = ctx->mlp;
-  void* ptrs[] = {m.params, m.grad, m.adam_m, m.adam_v, m.W1b, m.W2b, m.W3b, m.gw3tmp, m.mom, m.X, m.Y, m.bx, m.bt,
-                  m.z1acc, m.z1, m.z2acc, m.z2, m.yacc, m.y, m.dy, m.g2, m.dz2, m.g1, m.dz1, m.sqerr, m.loss, m.xb,
-                  m.a1b, m.a2b, m.dyb, m.dz2b, m.dz1b, m.idx};
+  void* ptrs[] = {m.params, m.grad, m.adam_m, m.adam_v, m.W1b, m.W2b, m.W3b, m.mom, m.X, m.Y, m.bx, m.bt, m.part, m.idx};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   m = MlpCtx();
@@ -323,8 +264,12 @@ pond_status pond_mlp_train(pond_ctx* ctx, int epochs, int batch, float lr, uint6
         ctx->err = "pond_mlp_train: batch gather failed";
         break;
       }
-      st = mlp_fwd_bwd(ctx, batch, false);
-      if (st != POND_OK) break;
+      // (the biases' gradients come with the rest; k_adam holds the biases)
+      if (mlp_grad(pond_mlp_weights(ctx), m.bx, m.bt, batch, m.part, m.grad, ctx->stream) != hipSuccess) {
+        st = POND_ERR_HIP;
+        ctx->err = "pond_mlp_train: gradient pass failed";
+        break;
+      }
       m.adam_t++;
       const float c1 = 1.0f - std::pow(b1, (float)m.adam_t), c2 = 1.0f - std::pow(b2, (float)m.adam_t);
       const float lr_t = (float)(0.5 * (double)lr * (1.0 + std::cos(kPi * (double)(ep * nb + bi) / total)));
@@ -338,7 +283,7 @@ pond_status pond_mlp_train(pond_ctx* ctx, int epochs, int batch, float lr, uint6
       if (st != POND_OK) break;
       if ((bi & 63) == 63 || bi == nb - 1) {
         float l = 0;
-        if (hipMemcpyAsync(&l, m.loss, sizeof(float), hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
+        if (hipMemcpyAsync(&l, m.grad + kMlpParams, sizeof(float), hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
             hipStreamSynchronize(ctx->stream) != hipSuccess) {
           st = POND_ERR_HIP;
           break;
@@ -444,15 +389,12 @@ pond_status pond_mlp_grad(pond_ctx* ctx, const float* X, const float* T, int64_t
   if (s != POND_OK) return s;
   MLP_HIP(ctx, hipMemcpy(m.bx, X, (size_t)B * kMlpIn * 4, hipMemcpyHostToDevice));
   MLP_HIP(ctx, hipMemcpy(m.bt, T, (size_t)B * kMlpOut * 4, hipMemcpyHostToDevice));
-  s = mlp_fwd_bwd(ctx, (int)B, true);
-  if (s != POND_OK) return s;
+  MLP_HIP(ctx, mlp_grad(pond_mlp_weights(ctx), m.bx, m.bt, (int)B, m.part, m.grad, ctx->stream));
   MLP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  MLP_HIP(ctx, hipMemcpy(grad, m.grad, (size_t)kMlpParams * 4, hipMemcpyDeviceToHost));
-  if (loss) {
-    float l = 0;
-    MLP_HIP(ctx, hipMemcpy(&l, m.loss, sizeof(float), hipMemcpyDeviceToHost));
-    *loss = l / (float)B;
-  }
+  std::vector<float> out((size_t)kMlpParams + 1);
+  MLP_HIP(ctx, hipMemcpy(out.data(), m.grad, out.size() * 4, hipMemcpyDeviceToHost));
+  std::memcpy(grad, out.data(), (size_t)kMlpParams * 4);
+  if (loss) *loss = out[kMlpParams] / (float)B;
   return POND_OK;
 }
 

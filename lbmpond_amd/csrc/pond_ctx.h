@@ -34,14 +34,13 @@ struct EventPair {
 struct MlpCtx {
   bool initialized = false, trained = false;
   float* params = nullptr;  // FP32 master parameters (kMlpParams, packed)
-  float* grad = nullptr;
+  float* grad = nullptr;  // kMlpParams gradients and the summed squared error
   float* adam_m = nullptr;
   float* adam_v = nullptr;
   int64_t adam_t = 0;
   unsigned short* W1b = nullptr;  // bf16 copies: W1 144x64, W2 64x64, W3 64x16
   unsigned short* W2b = nullptr;
   unsigned short* W3b = nullptr;
-  float* gw3tmp = nullptr;
   double* mom = nullptr;
   float in_inv[5] = {1, 1, 1, 1, 1};
   float out_scale[4] = {1, 1, 1, 1};
@@ -50,10 +49,7 @@ struct MlpCtx {
   float* Y = nullptr;
   int64_t count = 0, cap = 0;
   int bcap = 0;  // minibatch buffers
-  float *bx = nullptr, *bt = nullptr, *z1acc = nullptr, *z1 = nullptr, *z2acc = nullptr, *z2 = nullptr,
-        *yacc = nullptr, *y = nullptr, *dy = nullptr, *g2 = nullptr, *dz2 = nullptr, *g1 = nullptr, *dz1 = nullptr,
-        *sqerr = nullptr, *loss = nullptr;
-  unsigned short *xb = nullptr, *a1b = nullptr, *a2b = nullptr, *dyb = nullptr, *dz2b = nullptr, *dz1b = nullptr;
+  float *bx = nullptr, *bt = nullptr, *part = nullptr;  // part: the blocks' gradient sums
   int* idx = nullptr;
 };
 
