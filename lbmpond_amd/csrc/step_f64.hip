@@ -161,7 +161,8 @@ __device__ __forceinline__ void basis27(double u0x, double u0y, double u0z, doub
 // The transfer's term loop (structs.cuh:539-548) over the populations f.  The reference drops every
 // NaN or infinite term; a sum that comes out finite has dropped none (one such term leaves the plain
 // sum NaN or infinite), so the plain sum is formed and only a non-finite one is formed again with
-// the test on every term.
+// the test on every term, from the start: kept for that, the 27 products took 54 registers of every
+// node (128^3 vortex 63.7 -> 55.8 ms per step without).
 __device__ __forceinline__ double terms27(double W, const double (&gx)[3], const double (&gy)[3],
                                           const double (&gz)[3], const double (&f)[27]) {
   double p2[3][3];
@@ -177,10 +178,12 @@ __device__ __forceinline__ double terms27(double W, const double (&gx)[3], const
   }
   if (!finite_d(fnew)) {
     fnew = 0;
+    double Wa = W;  // (the compiler would keep the products of the plain sum)
+    asm volatile("" : "+v"(Wa));
 #pragma unroll
     for (int iold = 0; iold < 27; iold++) {
       const int jx = kE27[iold][0] + 1, jy = kE27[iold][1] + 1, jz = kE27[iold][2] + 1;
-      const double fadd = p2[jx][jy] * gz[jz] * f[iold];
+      const double fadd = Wa * gx[jx] * gy[jy] * gz[jz] * f[iold];
       if (finite_d(fadd)) fnew += fadd;
     }
   }
@@ -607,11 +610,11 @@ __device__ __forceinline__ Tgt27 tgt27_of(const Tgt27g3& t, int k) {
 // y from ry and in z from rz.  Calls slice(d) at the start of a slice, row(a) at the start of a row,
 // and node(n, d, a, b) with the node's data.  Row offsets are 32-bit (node_off, mod 2^32).
 //
-// Tried, and slower (128^3 vortex, this walk 65 ms per step): the loads of a node issued a node ahead
-// (74 ms: the populations then live through the weighting and push its values to scratch); each
+// Tried, and no faster (128^3 vortex, this walk 56 ms per step): the loads of a node issued before the
+// weighting of the one before (57 ms: the other wave of the SIMD covers the wait already); each
 // different node of a wave's cells loaded once, 16 bytes per lane, and handed out through LDS (112
-// ms: the loaders' addresses go to scratch, and a scratch access occupies the L1 for as long as a
-// 16-byte load); held to three waves per SIMD (183 ms, scratch again).
+// ms when the walk took 65: the loaders' addresses go to scratch, and a scratch access occupies the
+// L1 for as long as a 16-byte load); held to three waves per SIMD (91 ms, scratch again).
 template <int NR, bool MIR, class SRC, class FS, class FR, class FN>
 __device__ __forceinline__ void walk27(const SRC& src, int x, int ry, int rz, int dlo, int dhi, FS&& slice, FR&& row,
                                        FN&& node) {
@@ -1057,11 +1060,10 @@ __global__ __launch_bounds__(64) void k_step_f64(const NodeSrc gsrc, double* __r
 // converged takes the next one, the iterate stays in LDS and the previous one in registers; the
 // lanes of a cell mostly want the same nodes, so a load touches a few cache lines.  Each value is the
 // same sequence of operations (bit for bit).
-// Per step, before and after: 33x18x14 vortex 10.0 -> 0.85 ms; 128^3 vortex 86 -> 65 ms; 256x128x128
-// shock-bubble 289 -> 181 ms; Lagrange-4 128^3 255 -> 124 ms, 100x52x46 with walls 109 -> 16.5 ms.
-// Bound by the L1: at 128^3 the VALU is busy 60-65 % of the time, the texture-address unit 56 %, with
-// the L1 stalled on pending misses for half of it; the minimum of FP64 operations (no contraction,
-// every rounding of the reference) is half of what the waves issue.
+// Per step, before and after: 33x18x14 vortex 10.0 -> 0.85 ms; 128^3 vortex 86 -> 56 ms; 256x128x128
+// shock-bubble 289 -> 181 ms; Lagrange-4 128^3 255 -> 124 ms, 100x52x46 with walls 109 -> 15.8 ms.
+// Bound by FP64 issue: at 128^3 the VALU is busy 75 % of the time (texture-address unit 54 %), with 330
+// instructions per node where no contraction and every rounding of the reference leave about 290.
 template <int INTERP, class SRC>
 __device__ __forceinline__ void f64_group(const SRC& src, int x, int y, int z, int ey, int ez, const double (&uT)[4],
                                           double s, const StepArgs& a, double (&fn)[3]) {
