@@ -877,13 +877,19 @@ __device__ __forceinline__ void interp_pass_lagr4(const NodeSrcF& src, int x, in
   for (int e = 0; e < 3; e++)
 #pragma unroll
     for (int t = 0; t < 3; t++) acc[e][t] = 0.f;
-  // byte offset of node (xs, yr, lz + b), its mirror image where it lies beyond a mirrored face
-  auto node_off = [&](int xs_, int yr_, int b) -> uint32_t {
+  // cell of node (xs, yr, lz + b) = row_cell(xs, yr) + zo[b], its mirror image where it lies beyond a
+  // mirrored face (wrapped once per step and per pass, not at every node: 150x101x94 8.52 -> 8.10 ms)
+  uint32_t zo[4];
+  bool rz[4] = {false, false, false, false};
+#pragma unroll
+  for (int b = 0; b < 4; b++)
+    zo[b] = (uint32_t)(MIR ? mirror_wrap(lz + b, g.nz, (g.mirror & 4) != 0, rz[b]) : wrapi(lz + b, g.nz)) *
+            ((uint32_t)g.nx * (uint32_t)g.ny);
+  auto row_cell = [&](int xs_, int yr_) -> uint32_t {
     bool rv;
     const int xw = MIR ? mirror_wrap(xs_, g.nx, (g.mirror & 1) != 0, rv) : wrapi(xs_, g.nx);
     const int yw = MIR ? mirror_wrap(yr_, g.ny, (g.mirror & 2) != 0, rv) : wrapi(yr_, g.ny);
-    const int zw = MIR ? mirror_wrap(lz + b, g.nz, (g.mirror & 4) != 0, rv) : wrapi(lz + b, g.nz);
-    return (uint32_t)cell_index(g, xw, yw, zw) * 4u;
+    return (uint32_t)xw + (uint32_t)yw * (uint32_t)g.nx;
   };
   // The (slice, row) steps run as one loop whose node loads are one step ahead, as in
   // interp_pass_weno5c: node b of the next step is loaded into the registers of node b of the
@@ -894,7 +900,7 @@ __device__ __forceinline__ void interp_pass_lagr4(const NodeSrcF& src, int x, in
   Gauge4 nb[4];
 #pragma unroll
   for (int b = 0; b < 4; b++) {
-    const uint32_t boff = node_off(xlo, ylo, b);
+    const uint32_t boff = (row_cell(xlo, ylo) + zo[b]) * 4u;
     load27(src.f, boff, fb[b]);
     nb[b] = ldg4(src, boff);
   }
@@ -921,10 +927,10 @@ __device__ __forceinline__ void interp_pass_lagr4(const NodeSrcF& src, int x, in
     }
     const bool last_row = yr == yhi;
     const int xn = last_row ? xs + 1 : xs, yn = last_row ? ylo : yr + 1;
+    const uint32_t on = row_cell(xn, yn);
 #pragma unroll
     for (int b = 0; b < 4; b++) {
-      bool rzf = false;
-      if (MIR) mirror_wrap(lz + b, g.nz, (g.mirror & 4) != 0, rzf);
+      const bool rzf = rz[b];
       const float fzb = b == 0 ? Fz[0] : b == 1 ? Fz[1] : b == 2 ? Fz[2] : Fz[3];
       Gauge4 n = nb[b];
       // a node beyond a mirrored face is the mirror image of the cell inside
@@ -987,7 +993,7 @@ __device__ __forceinline__ void interp_pass_lagr4(const NodeSrcF& src, int x, in
         for (int t = 0; t < 3; t++) acc[e][t] = __builtin_fmaf(wx[t] * wyz, Tt[t], acc[e][t]);
       }
       // node b of this step is used up: load node b of the next step in its place
-      const uint32_t boff = node_off(xn, yn, b);
+      const uint32_t boff = (on + zo[b]) * 4u;
       load27(src.f, boff, fb[b]);
       nb[b] = ldg4(src, boff);
     }
@@ -1291,7 +1297,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
 // next cell of the wave's run when its own has converged.  Each cell's arithmetic and its order are the
 // same (bit for bit).  Per step, before and after: 256^3 vortex 65.3 -> 39.6 ms, 256^3 shock-bubble
 // 107 -> 69.7 ms, 32^3 shock-bubble 16.9 -> 5.6 ms; Lagrange-4 192^3 Taylor-Green 81 -> 37.5 ms,
-// 150x101x94 22.0 -> 8.5 ms.  256^3 vortex: VALU busy 85 % (57 of 64 lanes), texture-address unit 71 %.
+// 150x101x94 22.0 -> 8.1 ms.  Bound by VALU issue: 256^3 vortex busy 85 % (57 of 64 lanes; texture-address
+// unit 71 %), 150x101x94 86 % (45 lanes: windows and rows that differ between the cells of a wave).
 // Two waves per SIMD (256 registers): with more registers the load latency would be left unhidden.
 template <int INTERP>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_step_split27_cells(
