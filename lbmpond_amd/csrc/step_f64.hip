@@ -1112,9 +1112,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
   const Grid& g = a.g;
   const int64_t P = g.plane;
   const int lane = threadIdx.x;
-  const int slot = lane / 9, gi = lane - 9 * slot;  // lane 63 has no cell
+  // Lanes of a cell (lane 63 has none).  WENO5: side by side, as its groups mostly want the same rows and
+  // neighbouring lanes then the same record.  Lagrange-4: a group's seven cells side by side, as
+  // its groups' rows mostly differ and four neighbouring lanes then read 64 consecutive bytes: 64^3
+  // Taylor-Green 14.0 -> 12.1 ms, 100x52x46 with walls 16.9 -> 16.2 ms per step (WENO5: vortex 1 to 2 %
+  // slower so, shock-bubble 2 % faster).
+  constexpr int CS = WENO ? 9 : 1, GS = WENO ? 1 : 7;  // lane = CS * slot + GS * group
+  const int slot = WENO ? lane / 9 : lane < 63 ? lane % 7 : 7, gi = WENO ? lane % 9 : lane < 63 ? lane / 7 : 0;
   const int ey = gi / 3 - 1, ez = gi % 3 - 1;
-  constexpr uint64_t kHeads = 0x0040201008040201ull;  // lanes 0, 9, .., 54
+  constexpr uint64_t kHeads = WENO ? 0x0040201008040201ull : 0x7full;       // group 0 of every slot
+  constexpr uint64_t kGroups = WENO ? 0x1ffull : 0x0102040810204081ull;     // the groups of slot 0
   if (lane < 28) s_w[lane] = lane < 27 ? a.w[lane] : 0.0;
   const int64_t q0 = xcd_block(blockIdx.x, gridDim.x) * cells;
   const int64_t total = g.ntiles * 64 - q0 < cells ? g.ntiles * 64 - q0 : cells;  // cell slots of the wave
@@ -1129,7 +1136,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
   while (true) {
     const uint64_t want = __ballot(!active) & kHeads;
     if (!active && slot < 7) {
-      const int64_t q = next + __popcll(want & ((1ull << (9 * slot)) - 1ull));
+      const int64_t q = next + __popcll(want & ((1ull << (CS * slot)) - 1ull));
       if (q < total && tile_cell(g, (q0 + q) / 64, (int)((q0 + q) % 64), x, y, z)) {
         cell = cell_index(g, x, y, z);
         F64Iter st;
@@ -1173,23 +1180,24 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
     double acc = 0;
 #pragma unroll
     for (int i = 0; i < 27; i++) acc += s_fn[slot][i] * (wx[kE27[i][0] + 1] + wy[kE27[i][1] + 1] + wz[kE27[i][2] + 1]);
-    const int head = 9 * slot;
+    const int head = CS * slot;
     const double rho = __shfl(acc, head, 64);
     if (rho != 0) acc /= rho;
-    const double m0 = __shfl(acc, head + 1, 64), m1 = __shfl(acc, head + 2, 64), m2 = __shfl(acc, head + 3, 64);
-    double m3 = __shfl(acc, head + 4, 64);
+    const double m0 = __shfl(acc, head + GS, 64), m1 = __shfl(acc, head + 2 * GS, 64),
+                 m2 = __shfl(acc, head + 3 * GS, 64);
+    double m3 = __shfl(acc, head + 4 * GS, 64);
     m3 = (m3 - m0 * m0 - m1 * m1 - m2 * m2) * a.inv_dim;
     if (m3 < 0) m3 = uT[3];  // steps.cu:475-478
     const double mn[4] = {m0, m1, m2, m3};
 #pragma unroll
     for (int k = 0; k < 4; k++)
       if (fabs(mn[k] - uT[k]) >= a.tol_abs + a.tol_rel * fabs(mn[k])) conv = false;
-    const uint64_t bad = __ballot(!conv) >> head;
+    const uint64_t bad = (__ballot(!conv) >> head) & kGroups;
     if (active) {
       niter++;
 #pragma unroll
       for (int k = 0; k < 4; k++) c0[k] = mn[k];
-      const bool done = (bad & 0x1ff) == 0 || niter >= a.max_iter;
+      const bool done = bad == 0 || niter >= a.max_iter;
       if (done || (WENO && niter >= wide_after)) {
         // BGK towards rho*w_i (steps.cu:557-564), two populations per lane and store; a cell left to
         // k_step_f64_27_wide stores its iterate as it is
