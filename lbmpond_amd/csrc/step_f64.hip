@@ -645,6 +645,10 @@ __device__ __forceinline__ void walk27(const SRC& src, int x, int ry, int rz, in
   }
 }
 
+// The WENO5 step's cell slot of a lane: cells in pairs, a group's two lanes side by side (lane 18 p +
+// 2 group + cell of pair p), the seventh cell's groups in lanes 54 .. 62
+__device__ __forceinline__ int weno_slot27(int lane) { return lane < 54 ? lane / 18 * 2 + (lane & 1) : lane < 63 ? 6 : 7; }
+
 // interp_weno5<kD3Q27, VAR> for the three targets of a group (cx[k] of target ex = k - 1; cy, cz
 // shared), on a grid that is not a line, without mirrors.  Window positions are taken relative
 // to the cell's own x, so lanes of a wave whose flow is alike visit the same positions.  Taken
@@ -683,7 +687,7 @@ __device__ __forceinline__ void interp_weno5_g3(const SRC& src, int x, double s,
   // shared by the row's nodes.
   __shared__ double s_ub[3][5][64];
   __shared__ double s_pw[3][3][8];
-  const int lane = threadIdx.x & 63, slot = lane / 9;
+  const int lane = threadIdx.x & 63, slot = weno_slot27(lane);
   double S[3][3];
 #pragma unroll
   for (int k = 0; k < 3; k++) {
@@ -1112,16 +1116,18 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
   const Grid& g = a.g;
   const int64_t P = g.plane;
   const int lane = threadIdx.x;
-  // Lanes of a cell (lane 63 has none).  WENO5: side by side, as its groups mostly want the same rows and
-  // neighbouring lanes then the same record.  Lagrange-4: a group's seven cells side by side, as
-  // its groups' rows mostly differ and four neighbouring lanes then read 64 consecutive bytes: 64^3
-  // Taylor-Green 14.0 -> 12.1 ms, 100x52x46 with walls 16.9 -> 16.2 ms per step (WENO5: vortex 1 to 2 %
-  // slower so, shock-bubble 2 % faster).
-  constexpr int CS = WENO ? 9 : 1, GS = WENO ? 1 : 7;  // lane = CS * slot + GS * group
-  const int slot = WENO ? lane / 9 : lane < 63 ? lane % 7 : 7, gi = WENO ? lane % 9 : lane < 63 ? lane / 7 : 0;
+  // Lanes of a cell (lane 63 has none).  A 16-byte load takes four neighbouring lanes at a time, so
+  // these should want one cache line.  Lagrange-4: a group's seven cells side by side, as its groups'
+  // rows mostly differ (64^3 Taylor-Green 14.0 -> 12.1 ms, 100x52x46 with walls 16.9 -> 16.2 ms per step).
+  // WENO5, whose groups' rows coincide below half a cell of thermal speed: cells in pairs (weno_slot27;
+  // against a cell's nine groups side by side: 128^3 shock-bubble 86.0 -> 82.7 ms, vortex 56.4 ms both).
+  const int slot = WENO ? weno_slot27(lane) : lane < 63 ? lane % 7 : 7;
+  const int gi = WENO ? (lane < 54 ? lane % 18 / 2 : lane < 63 ? lane - 54 : 0) : lane < 63 ? lane / 7 : 0;
+  const int head = WENO ? (slot < 6 ? 18 * (slot / 2) + (slot & 1) : 54) : slot;  // the slot's lane of group 0
+  const int GS = WENO ? (slot < 6 ? 2 : 1) : 7;                                   // and from group to group
   const int ey = gi / 3 - 1, ez = gi % 3 - 1;
-  constexpr uint64_t kHeads = WENO ? 0x0040201008040201ull : 0x7full;       // group 0 of every slot
-  constexpr uint64_t kGroups = WENO ? 0x1ffull : 0x0102040810204081ull;     // the groups of slot 0
+  constexpr uint64_t kHeads = WENO ? 0x400030000c0003ull : 0x7full;  // group 0 of every slot
+  const uint64_t groups = WENO ? (slot < 6 ? 0x15555ull : 0x1ffull) : 0x0102040810204081ull;  // from head on
   if (lane < 28) s_w[lane] = lane < 27 ? a.w[lane] : 0.0;
   const int64_t q0 = xcd_block(blockIdx.x, gridDim.x) * cells;
   const int64_t total = g.ntiles * 64 - q0 < cells ? g.ntiles * 64 - q0 : cells;  // cell slots of the wave
@@ -1136,7 +1142,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
   while (true) {
     const uint64_t want = __ballot(!active) & kHeads;
     if (!active && slot < 7) {
-      const int64_t q = next + __popcll(want & ((1ull << (CS * slot)) - 1ull));
+      const int64_t q = next + __popcll(want & ((1ull << head) - 1ull));
       if (q < total && tile_cell(g, (q0 + q) / 64, (int)((q0 + q) % 64), x, y, z)) {
         cell = cell_index(g, x, y, z);
         F64Iter st;
@@ -1180,7 +1186,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
     double acc = 0;
 #pragma unroll
     for (int i = 0; i < 27; i++) acc += s_fn[slot][i] * (wx[kE27[i][0] + 1] + wy[kE27[i][1] + 1] + wz[kE27[i][2] + 1]);
-    const int head = CS * slot;
     const double rho = __shfl(acc, head, 64);
     if (rho != 0) acc /= rho;
     const double m0 = __shfl(acc, head + GS, 64), m1 = __shfl(acc, head + 2 * GS, 64),
@@ -1192,7 +1197,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
 #pragma unroll
     for (int k = 0; k < 4; k++)
       if (fabs(mn[k] - uT[k]) >= a.tol_abs + a.tol_rel * fabs(mn[k])) conv = false;
-    const uint64_t bad = (__ballot(!conv) >> head) & kGroups;
+    const uint64_t bad = (__ballot(!conv) >> head) & groups;
     if (active) {
       niter++;
 #pragma unroll

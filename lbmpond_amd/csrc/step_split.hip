@@ -1312,15 +1312,21 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
   const Grid& g = a.g;
   const int64_t P = g.plane;
   const int lane = threadIdx.x;
-  // Lanes of a cell (lane 63 has none).  WENO5C: side by side, as its passes mostly want the same z rows
-  // and neighbouring lanes then the same record.  Lagrange-4: a pass's 21 cells side by side, as
-  // its passes' rows mostly differ (floor(z) moves with ez) and four neighbouring lanes then read
-  // 64 consecutive bytes instead of parts of three rows: 192^3 37.3 -> 29.3 ms, 128^3 shock-bubble 15.3 ->
-  // 12.6 ms per step (the WENO5C shock-bubble gains 4 % so, the vortex loses 4 %).
-  constexpr bool BYCELL = INTERP == 2;
-  const int slot = BYCELL ? lane / 3 : lane < 63 ? lane % 21 : 21, pz = BYCELL ? lane % 3 : lane < 63 ? lane / 21 : 0;
-  const int head = BYCELL ? 3 * slot : slot;  // the slot's lane of the first pass
-  constexpr uint64_t kHeads = BYCELL ? 0x1249249249249249ull : 0x1fffffull;
+  // Lanes of a cell (lane 63 has none).  A 16-byte load takes four neighbouring lanes at a time, so
+  // these should want one cache line.  Lagrange-4: a pass's 21 cells side by side, as its passes' rows
+  // mostly differ (floor(z) moves with ez): with a cell's passes side by side, 192^3 took 37.3 instead of
+  // 29.3 ms per step, the 128^3 shock-bubble 15.3 instead of 12.6 ms.  WENO5C: twelve lanes per four cells
+  // (two cells by two passes, the third pass of all four, the other two by two), as its passes' rows
+  // coincide below half a cell of thermal speed and differ above (against a cell's passes side by side:
+  // 256^3 shock-bubble 70.2 -> 67.0 ms, vortex 40.1 -> 40.4 ms; as Lagrange-4: 66.7 and 41.3 ms).
+  constexpr bool BLOCKS = INTERP == 2;
+  const int l12 = lane % 12;
+  const int slot = BLOCKS ? (lane < 60 ? 4 * (lane / 12) + (int)((0xeee444u >> (2 * l12)) & 3) : lane < 63 ? 20 : 21)
+                          : (lane < 63 ? lane % 21 : 21);
+  const int pz = BLOCKS ? (lane < 60 ? (int)((0x50aa50u >> (2 * l12)) & 3) : (lane - 60) % 3) : lane < 63 ? lane / 21 : 0;
+  // the slot's lane of the first pass
+  const int head = BLOCKS ? (slot < 20 ? 12 * (slot / 4) + (slot & 1) + 4 * (slot & 2) : 60) : slot;
+  constexpr uint64_t kHeads = BLOCKS ? 0x1303303303303303ull : 0x1fffffull;
   if (lane < FS) s_w[lane] = lane < 27 ? a.w[lane] : 0.f;
   const int64_t q0 = xcd_block(blockIdx.x, gridDim.x) * cells;
   const int64_t total = g.ntiles * 64 - q0 < cells ? g.ntiles * 64 - q0 : cells;  // cell slots of the wave
