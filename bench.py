@@ -94,13 +94,13 @@ def default_interp(case):
 
 def kernel_name(lattice, prec, interp):
     if lattice == "D3Q125":
-        return "k_step_q125_f64" if prec == "fp64" else "k_step_split125"
-    if lattice == "D1Q5":
-        return "k_step_f64<0,1,false>" if interp == "lagr4" else "k_step_f64<0,0,false>"
+        return "k_step_q125_f64<false>" if prec == "fp64" else "k_step_split125"
     code = {"weno5": 0, "lagr4": 1, "weno5c": 2}[interp]
+    if lattice == "D1Q5":
+        return "k_step_line<1>" if code == 1 else "k_step_line<0>"
     if prec == "fp64":
-        return f"k_step_f64_refill<1,{code},true>"
-    return f"k_step_split27_refill<{code}>" if code != 0 else "k_step_split27<0>"
+        return f"k_step_f64_27<{code},true>"
+    return f"k_step_split27_cells<{code}>" if code != 0 else "k_step_split27_written"
 
 
 class Run:

@@ -91,8 +91,8 @@ typedef struct {
                    FP64 7 or 14 cells; split 21 to 128 cells or whole x rows, by grid size.
      pass1_iters   POND_SPLIT POND_WENO5 / POND_WENO5G: iterations of the first pass of the
                    two-pass step; cells not converged by then are finished by a second kernel
-                   over a compacted list.  -1 (default): one pass.  The other D3Q27 steps take
-                   one pass.
+                   over a compacted list.  -1 (default): one pass.  The other D3Q27 WENO5 steps
+                   leave cells to a second kernel by a rule of their own (grid size).
      global_loads  1: FP64 D3Q27 node loads through 64-bit global addresses, the path of grids
                    whose population planes do not fit 32-bit buffer offsets (above 67,108,800
                    cells).  0 (default): buffer loads where they fit. */

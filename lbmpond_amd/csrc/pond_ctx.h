@@ -86,8 +86,8 @@ struct pond_ctx {
                             // else P, with P = sqrt(|T|)*sign(T)
   float* sq = nullptr;      // split path: node gauge records (ux, uy, uz, sqrt(|T|)*sign(T)) of the load buffer
   float* guess = nullptr;   // split path: learned starting gauge increments (4 planes)
-  // cells left unconverged by the first pass of a two-pass step: count, then per entry the
-  // cell index, 4 gauge doubles, one double and one int (48 B per cell of the grid)
+  // cells left unconverged by a step's first kernel: count, then the D3Q27 WENO5 steps' list of cells,
+  // or per entry of a two-pass step the cell index, 4 gauge doubles, one double and one int (48 B per cell of the grid)
   char* pend = nullptr;
   int64_t pend_cap = 0;
   int* niter = nullptr;     // per-cell gauge iterations of the last step

@@ -12,10 +12,11 @@
 //   * the transfer's NaN/Inf test is made on its sum (terms27);
 //   * the moment sums (structs.cuh:323-327) run over the stored iterate in the same population order.
 //
-// D3Q27 mapping: nine lanes per cell, one (ey, ez) group of three targets each.  D1Q5 lines: 32 lanes
-// per cell; other D1Q5 grids: one lane per cell, 64 consecutive cells (x fastest) per wave.
-// D3Q125 mapping: one 128-lane block per cell, lane = target population (as the reference's
-// 125-thread block), the fixed 3x3x3 neighbourhood staged in LDS.
+// D3Q27 mapping: nine lanes per cell, one (ey, ez) group of three targets each; WENO5 cells that go on
+// iterating, one workgroup each.  D1Q5 lines: 32 lanes per cell; other D1Q5 grids: one lane per
+// cell, 64 consecutive cells (x fastest) per wave.  D3Q125 mapping: one 128-lane block per cell, lane =
+// target population (as the reference's 125-thread block), the nodes of the fixed 3x3x3 neighbourhood
+// through scalar loads.
 #include <type_traits>
 #include "pond_device.h"
 
@@ -1012,16 +1013,11 @@ __device__ __forceinline__ void f64_finish(double* __restrict__ fout, double* __
   niter_out[cell] = st.niter;
 }
 
-// First pass: every cell iterates up to a.pass1_iters times; cells still unconverged are
-// appended to the pending list (one atomic per wave) and finished by a second pass over that
-// list (k_step_f64_rest or k_step_f64_rest_wide).  A wave runs as long as its slowest cell, and
-// a thin layer of cells on shocks and contact discontinuities needs several times the mean
-// count.  Each cell's arithmetic and operation order are those of a single pass.
-// BUF: node loads through buffer resources (planes up to 59,652,323 cells), else global loads.
-// D3Q27: held to two waves per SIMD (256 VGPRs, a few spilled).  Measured on the 384^3
-// shock-bubble FP64 step, A/B on one GPU: the grouped WENO5C kernel 2.70 s at one wave per SIMD
-// (its registers spilled to AGPRs), 2.58 s at two; Lagrange-4 5.34 s -> 4.99 s.  The D1Q5 kernel
-// keeps its registers (held to two waves it would spill 1.7 KB per lane).
+// D1Q5 with one lane per cell (grids that are no line, and long Lagrange-4 lines).  First pass: every cell
+// iterates up to a.pass1_iters times; cells still unconverged are appended to the pending list (one
+// atomic per wave) and finished by a second pass over that list (k_step_f64_rest).  A wave runs as long
+// as its slowest cell, and a thin layer of cells on shocks and contact discontinuities needs several
+// times the mean count.  Each cell's arithmetic and operation order are those of a single pass.
 template <int LAT, int INTERP>
 __global__ __launch_bounds__(64) void k_step_f64(const NodeSrc gsrc, double* __restrict__ fout,
                                                  double* __restrict__ mout, int* __restrict__ niter_out, Pending pend,
