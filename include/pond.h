@@ -85,10 +85,10 @@ typedef struct {
                    tile_patch x tile_patch patches, so the waves resident on one XCD share
                    their stencil halo in its L2; used where nx % 64 == 0 and tile_patch divides
                    ny and nz.  0: plain row order.  -1 (default): 8 for the POND_SPLIT
-                   D3Q27 WENO5C step, 4 otherwise.
+                   D3Q27 WENO5C step where 8 divides ny and nz, 4 otherwise.
      refill_chunk  64-cell tiles owned by one wave, whose lanes take the next unstarted cell
                    of the chunk when theirs converges.  0: one tile per wave.  -1 (default):
-                   FP64 7 or 14 cells; split 21 to 128 cells or whole x rows, by grid size.
+                   FP64 7 or 14 cells; split 21, 42 or 128 cells or whole x rows, by grid size.
      pass1_iters   POND_SPLIT POND_WENO5 / POND_WENO5G: iterations of the first pass of the
                    two-pass step; cells not converged by then are finished by a second kernel
                    over a compacted list.  -1 (default): one pass.  The other D3Q27 WENO5 steps

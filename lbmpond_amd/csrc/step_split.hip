@@ -1996,23 +1996,30 @@ hipError_t launch_step_split(int lattice, int interp, const SplitPtrs& in, const
   if (lattice != kD3Q27) return hipErrorInvalidValue;
   if (interp != 0) {
     const int64_t slots = a.g.ntiles * 64;
-    // Cells per wave.  Where the cells go by x rows (row patches): whole rows, at least 128 cells, so
-    // that the waves resident on an XCD cover a compact patch of rows, but no so many that SIMDs go
-    // without two waves.  In linear order: 128 cells on large grids, one per slot below (the waves in
-    // flight then cover fewer planes, and more of them even out the last round).  ms per step with
-    // 21, 42, 64, 128, 192, 256, 384 cells, WENO5C vortex: 64^3 1.03, 0.98, 0.86, 0.84, 1.10, 1.36,
-    // 1.96; 128^3 6.79, 6.24, 5.95, 5.43, 5.66, 5.36, 5.73; 192^3 22.4, 20.4, 19.2, 17.8, 17.0, 17.5,
-    // 16.9; 250x200x180 28.8, 26.3, 25.6, 23.0, 28.3, 22.1, 27.0; shock-bubble 32^3 5.60, 5.79, 5.86,
-    // 6.34, -, 6.22; Lagrange-4 150x101x94 8.45, 8.84, 9.97, 10.4, -, 11.3.
+    // Cells per wave.  By x rows (row patches, or linear order with WENO5C): whole rows, at least 128
+    // (64) cells, so that the waves resident on an XCD cover a compact patch of rows, but not so many
+    // that SIMDs go without two waves, and on small grids one cell per slot.  Lagrange-4 in linear order: one or two cells per slot (the waves
+    // in flight then cover fewer planes, and more of them even out the last round).  ms per step, with 21,
+    // 42, 64, 128, 192, 256, 384 cells, WENO5C vortex in patches: 64^3 1.03, 0.98, 0.86, 0.84, 1.10, 1.36,
+    // 1.96; 128^3 6.79, 6.24, 5.95, 5.43, 5.66, 5.36, 5.73; 192^3 22.4, 20.4, 19.2, 17.8, 17.0, 17.5, 16.9.
+    // In linear order with 21, 64, 128 cells and one row: 50x40x30 0.40, 0.49, 0.75, -; 100x60x50 1.19, 1.10, 1.28, 1.10; 100x90x80 2.60,
+    // 2.26, 2.27, 2.16; 150x101x94 4.76, 4.35, 4.18, 3.88 (shock-bubble 9.68, 8.36, 8.26, 7.60); 250x200x180
+    // -, 25.9, 23.3, 22.4.  Lagrange-4 with 21, 42, 128 cells: Taylor-Green 150x101x94 7.81, 8.50, 10.4;
+    // 250x200x180 44.5, 46.2, 48.7; shock-bubble 9.94, 9.55, 11.0 and 55.8, 51.1, 53.3.
     int64_t cells;
     if (a.refill_chunk >= 0) {
       cells = a.refill_chunk > 0 ? 64ll * a.refill_chunk : 64;
-    } else if (a.g.rp > 0) {
-      cells = a.g.nx * ((128ll + a.g.nx - 1) / a.g.nx);
+    } else if (interp == 2 && a.g.n < (1 << 17)) {
+      cells = 21;
+    } else if (a.g.rp > 0 || (interp == 2 && a.g.nx <= 512)) {
+      const int64_t least = a.g.rp > 0 ? 128 : 64;
+      cells = a.g.nx * ((least + a.g.nx - 1) / a.g.nx);
       while (cells > 21 && slots / cells < 2048) cells /= 2;
       if (cells < 21) cells = 21;
+    } else if (interp == 2) {
+      cells = 128;
     } else {
-      cells = a.g.n >= (1 << 22) ? 128 : 21;
+      cells = a.g.n >= (1 << 22) ? 42 : 21;
     }
     if (cells > slots) cells = slots;
     const dim3 nb((unsigned)((slots + cells - 1) / cells));
