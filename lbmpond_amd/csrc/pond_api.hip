@@ -399,7 +399,7 @@ pond_status pond_create(const pond_params* p, pond_ctx** out) {
   a.pass1_iters = p->pass1_iters > 0 ? p->pass1_iters : p->precision == POND_SPLIT ? (1 << 30) : 8;
   for (int i = 0; i < ctx->Qn; i++) a.w[i] = ctx->L.w[i];
 
-  if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess)
+  if (hipGetDevice(&ctx->device) != hipSuccess || hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess)
     return bail(POND_ERR_HIP, "pond_create: hipStreamCreate failed");
   ctx->split = p->precision == POND_SPLIT;
   if (!ctx->split) {
@@ -810,14 +810,16 @@ static void widen_floats(double* dst, const float* src, int64_t n) {
 // the planes of one state in order; false: the pinned buffers are not to be had
 static bool read_threaded(pond_ctx* ctx, const std::vector<ReadPlane>& planes, int64_t n, hipError_t* err) {
   if (!ctx->pinned) {
-    if (hipHostMalloc((void**)&ctx->pinned, (size_t)kReadThreads * kReadChunk, hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc((void**)&ctx->pinned, (size_t)kReadThreads * kReadChunk, hipHostMallocPortable) != hipSuccess) {
       (void)hipGetLastError();
       ctx->pinned = nullptr;
       return false;
     }
   }
-  int dev = 0;
-  *err = hipGetDevice(&dev);
+  // An event belongs to the device that is current when it is created, and a stream takes none of
+  // another device: every thread makes the context's device current, the caller's gets its own back.
+  int caller = 0;
+  *err = hipGetDevice(&caller);
   if (*err != hipSuccess) return true;
   std::vector<int64_t> first(planes.size() + 1, 0);  // first chunk of every plane
   for (size_t k = 0; k < planes.size(); k++)
@@ -827,7 +829,7 @@ static bool read_threaded(pond_ctx* ctx, const std::vector<ReadPlane>& planes, i
   auto work = [&](int t) {
     char* buf = ctx->pinned + (int64_t)t * kReadChunk;
     hipEvent_t ev = nullptr;
-    hipError_t e = hipSetDevice(dev);
+    hipError_t e = hipSetDevice(ctx->device);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
     while (e == hipSuccess && bad.load() == (int)hipSuccess) {
       const int64_t q = next.fetch_add(1);
@@ -856,6 +858,10 @@ static bool read_threaded(pond_ctx* ctx, const std::vector<ReadPlane>& planes, i
   work(0);
   for (auto& t : pool) t.join();
   *err = (hipError_t)bad.load();
+  if (caller != ctx->device) {
+    const hipError_t e = hipSetDevice(caller);
+    if (*err == hipSuccess) *err = e;
+  }
   // (a copy left queued by a failed call still writes to the pinned buffers)
   if (*err != hipSuccess) (void)hipStreamSynchronize(ctx->stream);
   return true;

@@ -75,6 +75,7 @@ struct pond_ctx {
   pond::Grid g{};
   pond::StepArgs args{};
   int Qn = 0;
+  int device = 0;           // the device that was current in pond_create: the state's and the stream's
   hipStream_t stream = nullptr;
   int cur = 0;              // index of the buffer holding the current state
   bool has_state = false;
