@@ -89,10 +89,10 @@ typedef struct {
      refill_chunk  64-cell tiles owned by one wave, whose lanes take the next unstarted cell
                    of the chunk when theirs converges.  0: one tile per wave.  -1 (default):
                    FP64 7 or 14 cells; split 21, 42 or 128 cells or whole x rows, by grid size.
-     pass1_iters   POND_SPLIT POND_WENO5 / POND_WENO5G: iterations of the first pass of the
-                   two-pass step; cells not converged by then are finished by a second kernel
-                   over a compacted list.  -1 (default): one pass.  The other D3Q27 WENO5 steps
-                   leave cells to a second kernel by a rule of their own (grid size).
+     pass1_iters   iterations after which an unconverged cell is left to the step's second kernel,
+                   where it has one: D3Q27 POND_WENO5 / POND_WENO5C / POND_WENO5G, and D1Q5 grids
+                   that are no line or POND_LAGR4 lines above 65536 cells.  -1 (default): D3Q27 by
+                   grid size (POND_SPLIT POND_WENO5 / POND_WENO5G: never), D1Q5 8.
      global_loads  1: FP64 D3Q27 node loads through 64-bit global addresses, the path of grids
                    whose population planes do not fit 32-bit buffer offsets (above 67,108,800
                    cells).  0 (default): buffer loads where they fit. */

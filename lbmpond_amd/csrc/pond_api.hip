@@ -392,11 +392,7 @@ pond_status pond_create(const pond_params* p, pond_ctx** out) {
   a.g = g;
   a.global_loads = p->global_loads != 0;
   a.refill_chunk = p->refill_chunk;
-  // Iterations of the first pass of the two-pass steps (D1Q5 with one lane per cell, split WENO5 as
-  // written); cells still unconverged are finished by the second pass.  The latter by default runs in
-  // one pass (192^3 shock-bubble: K=3 7.6, K=8 8.9, single pass 11.5 MLUPS: its second pass, with one
-  // lane per cell too, runs alone after the first and a few slowly converging cells make a tail).
-  a.pass1_iters = p->pass1_iters > 0 ? p->pass1_iters : p->precision == POND_SPLIT ? (1 << 30) : 8;
+  a.pass1_iters = p->pass1_iters;
   for (int i = 0; i < ctx->Qn; i++) a.w[i] = ctx->L.w[i];
 
   if (hipGetDevice(&ctx->device) != hipSuccess || hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess)

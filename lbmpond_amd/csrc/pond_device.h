@@ -32,7 +32,7 @@ struct StepArgs {
   double sqrt_tbase;  // sqrt(TLat), evaluated once on the host (structs.cuh:530)
   double tlat;
   double inv_dim;     // 1./Dim (structs.cuh:330)
-  int pass1_iters;    // D1Q5: iterations of the first pass of the one-lane-per-cell step
+  int pass1_iters;    // iterations after which a cell is left to the step's second kernel (-1: the step's own choice)
   int global_loads;   // 1: global loads even where the buffer-resource loads apply
   int refill_chunk;   // D3Q27: 64-cell tiles per wave (0: one; -1: the step's own choice of cells per wave)
   const int* cell_set;  // Cinfo::set per cell (0: not stepped), or null: every cell is stepped

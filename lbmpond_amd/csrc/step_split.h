@@ -13,7 +13,7 @@ struct SplitArgs {
   double sqrt_tbase;
   double tlat;
   double inv_dim;
-  int pass1_iters;  // D3Q27 WENO5 as written: iterations of the first pass (the rest go to the second)
+  int pass1_iters;      // iterations after which a cell is left to the step's second kernel (-1: the step's own choice)
   float learned_trust;  // largest predicted change (thermal units) taken as a start
   int refill_chunk;     // D3Q27: 64-cell tiles per wave (0: one; -1: the step's own choice of cells per wave)
   float w[kQmax];

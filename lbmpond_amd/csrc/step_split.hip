@@ -2033,7 +2033,8 @@ hipError_t launch_step_split(int lattice, int interp, const SplitPtrs& in, const
     // 1.02, 1.18, 1.36, 5.29; 64^3 2.99, 2.67, 2.54, 2.53, 2.59, 6.70; 128^3 14.2, 12.9, 11.97, 11.61,
     // 11.60, 14.5; 256^3 -, 73.9, 70.7, 69.5, 69.4, 69.8 (vortex, at most 10 iterations: 41.4, 39.82,
     // 39.78, -, -, 39.74).
-    const int wide_after = a.g.n < (1 << 19) ? 8 : 16;
+    // (the list holds the count in 16 bits)
+    const int wide_after = a.pass1_iters > 0 ? min(a.pass1_iters, 0xffff) : a.g.n < (1 << 19) ? 8 : 16;
     if (interp == 2) {
       POND_LAUNCH(2);
       const unsigned nw = (unsigned)(a.g.n < 1024 ? a.g.n : 1024);
@@ -2047,13 +2048,18 @@ hipError_t launch_step_split(int lattice, int interp, const SplitPtrs& in, const
 #undef POND_LAUNCH
     return hipGetLastError();
   }
+  // By default the first pass goes to the end (192^3 shock-bubble: K=3 7.6, K=8 8.9, single pass 11.5
+  // MLUPS: the second, with one lane per cell too, runs alone after the first and a few slowly
+  // converging cells make a tail).
+  SplitArgs b = a;
+  if (b.pass1_iters < 0) b.pass1_iters = 1 << 30;
   // second-pass grid: enough waves to fill the chip several times, never more than the cells
   const int64_t w2 = (a.g.n + 63) / 64;
   const unsigned blocks2 = (unsigned)(w2 < 16384 ? w2 : 16384);
   hipLaunchKernelGGL(k_step_split27_written, dim3((unsigned)a.g.ntiles), dim3(64), 0, st, in.f, in.m, in.T, g4, out.f,
-                     out.m, out.T, niter, guess, pend, a);
+                     out.m, out.T, niter, guess, pend, b);
   hipLaunchKernelGGL(k_step_split27_rest, dim3(blocks2), dim3(64), 0, st, in.f, in.m, in.T, g4, out.f, out.m, out.T,
-                     niter, pend, a);
+                     niter, pend, b);
   return hipGetLastError();
 }
 
