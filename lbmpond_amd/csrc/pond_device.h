@@ -69,6 +69,13 @@ __device__ __forceinline__ int64_t pending_slot(const Pending& p, bool pending, 
 // output buffers: entry 0 is their number, the cells start here
 constexpr int kSlowList = 64;
 
+// a place in that list, taken where the cell's wave would stand idle for it or the list is still short
+// (fewer than `few` cells); -1: the cell stays where it is
+__device__ __forceinline__ int slow_place(int* slow, bool idle, int few) {
+  if (!idle && __hip_atomic_load(slow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= few) return -1;
+  return atomicAdd(slow, 1);
+}
+
 __device__ __forceinline__ int isign_d(double v) { return (0.0 < v) - (v < 0.0); }
 
 // params.h:110-112

@@ -22,6 +22,7 @@
 // fixed-point iteration has the last word: a prediction that is not finite or not positive in T
 // is ignored, and if the residual stops falling before the noise floor, or the cell has not
 // converged after kLearnedBudget iterations, it restarts from its previous gauge.
+#include <climits>
 #include "pond_device.h"
 #include "step_split.h"
 
@@ -1286,6 +1287,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
   }
 }
 
+// A cell late in its iterations goes to k_step_split27_wide where its wave has no cell left to start and no
+// more than this many slots (of 21) with such cells; see launch_step_split.
+constexpr int kWideSlots = 5;
+
 // WENO5C and Lagrange-4 (INTERP 2, 1; 3: Lagrange-4 with mirror walls): three lanes per cell, lane =
 // ez pass of nine targets, 21 cells per wave.
 //
@@ -1305,7 +1310,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
     const float* __restrict__ fin, const float* __restrict__ min, const double* __restrict__ Tin,
     const float* __restrict__ g4in, float* __restrict__ fout, float* __restrict__ mout, double* __restrict__ Tout,
     int* __restrict__ niter_out, const float* __restrict__ guess, int* __restrict__ slow, const SplitArgs a, int cells,
-    int wide_after) {
+    int wide_after, int few) {
   constexpr int FS = 28;
   __shared__ __align__(16) float s_f[22][FS];  // the iterate's populations, [cell][9 (ez+1) + 3 (ey+1) + ex+1]
   __shared__ float s_w[FS];
@@ -1337,16 +1342,25 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
   int x = 0, y = 0, z = 0;
   SplitIter st;
   while (true) {
-    if (INTERP == 2 && active && st.niter >= wide_after) {
-      // left to k_step_split27_wide, its state in three of the cell's output quads (arguments for
-      // separate arrays cost the pass scratch registers: 39.7 -> 49.8 ms on the 256^3 vortex)
-      active = false;
-      const int64_t meta =
-          st.niter | ((int64_t)st.base << 16) | (st.learned ? 1ll << 32 : 0) | (st.contracted ? 1ll << 33 : 0);
-      reinterpret_cast<double2*>(fout)[pz * P + cell] =
-          make_double2(pz == 0 ? st.gc[0] : pz == 1 ? st.gc[2] : st.res_prev,
-                       pz == 0 ? st.gc[1] : pz == 1 ? st.gc[3] : __longlong_as_double(meta));
-      if (pz == 0) slow[kSlowList + atomicAdd(slow, 1)] = (int)cell;
+    if constexpr (INTERP == 2) {
+      const bool late = active && st.niter >= wide_after;
+      const bool idle = next >= total && __popcll(__ballot(late) & kHeads) <= kWideSlots;
+      if (late) {
+        int e = -1;  // the cell's place in the list of k_step_split27_wide
+        if (pz == 0) e = slow_place(slow, idle, few);
+        e = __shfl(e, head, 64);
+        if (e >= 0) {
+          // its state goes with it in three of the cell's output quads (arguments for separate arrays
+          // cost the pass scratch registers: 39.7 -> 49.8 ms on the 256^3 vortex)
+          active = false;
+          const int64_t meta =
+              st.niter | ((int64_t)st.base << 32) | (st.learned ? 1ll << 48 : 0) | (st.contracted ? 1ll << 49 : 0);
+          reinterpret_cast<double2*>(fout)[pz * P + cell] =
+              make_double2(pz == 0 ? st.gc[0] : pz == 1 ? st.gc[2] : st.res_prev,
+                           pz == 0 ? st.gc[1] : pz == 1 ? st.gc[3] : __longlong_as_double(meta));
+          if (pz == 0) slow[kSlowList + e] = (int)cell;
+        }
+      }
     }
     const uint64_t want = __ballot(!active) & kHeads;
     if (!active && slot < 21) {
@@ -1460,10 +1474,10 @@ __global__ __launch_bounds__(kWideThreads) void k_step_split27_wide(
     st.gc[3] = g23.y;
     st.res_prev = rm.x;
     st.rho = 0;
-    st.niter = (int)(meta & 0xffff);
-    st.base = (int)((meta >> 16) & 0xffff);
-    st.learned = (meta >> 32) & 1;
-    st.contracted = (meta >> 33) & 1;
+    st.niter = (int)(meta & 0x7fffffff);
+    st.base = (int)((meta >> 32) & 0xffff);  // (at most kLearnedBudget)
+    st.learned = (meta >> 48) & 1;
+    st.contracted = (meta >> 49) & 1;
     bool conv = false;
     while (!conv && st.niter - st.base < a.max_iter) {
       const double* gc = st.gc;
@@ -2026,15 +2040,23 @@ hipError_t launch_step_split(int lattice, int interp, const SplitPtrs& in, const
     const dim3 nb((unsigned)((slots + cells - 1) / cells));
 #define POND_LAUNCH(I)                                                                                             \
   hipLaunchKernelGGL(k_step_split27_cells<I>, nb, dim3(64), 0, st, in.f, in.m, in.T, g4, out.f, out.m, out.T, niter, \
-                     guess, pend.count, a, (int)cells, wide_after)
+                     guess, pend.count, a, (int)cells, wide_after, few)
     // The iteration after which a cell goes to k_step_split27_wide.  A workgroup there serves a cell's
     // iteration eight times sooner, but the chip gets through far fewer of them: early where the
     // cells kernel leaves it idle.  ms per step for 4, 6, 8, 12, 16 and never, shock-bubble: 32^3 1.03, 0.98,
     // 1.02, 1.18, 1.36, 5.29; 64^3 2.99, 2.67, 2.54, 2.53, 2.59, 6.70; 128^3 14.2, 12.9, 11.97, 11.61,
     // 11.60, 14.5; 256^3 -, 73.9, 70.7, 69.5, 69.4, 69.8 (vortex, at most 10 iterations: 41.4, 39.82,
     // 39.78, -, -, 39.74).
-    // (the list holds the count in 16 bits)
-    const int wide_after = a.pass1_iters > 0 ? min(a.pass1_iters, 0xffff) : a.g.n < (1 << 19) ? 8 : 16;
+    const int wide_after = a.pass1_iters > 0 ? a.pass1_iters : a.g.n < (1 << 19) ? 8 : 16;
+    // From then on a cell goes when its wave stands idle for it: with no cell left to start and at most
+    // kWideSlots slots still at such cells.  The workgroups of the chip do 80 iterations per us, the waves
+    // with all slots in use 900, so a wave whose cells are all late keeps them.  Only the first `few` of a
+    // step go at once: a small grid leaves the chip idle anyway.  Tolerance 0 (every cell to the cap), ms per
+    // step with every late cell handed over and now: 64^3 250, 33, 128^3 1840, 208; tolerance 1.4e-8 (a third
+    // of the cells past 16 iterations): 64^3 53, 15, 128^3 320, 85; T = 0.2 with density jumps 16 cells apart:
+    // 64^3 17.9, 16.7, 128^3 102, 99, 200^3 443, 503 (one lane per cell: 951).  32^3 with few = 4096, 8192 and
+    // 16384: tolerance 0 9.7, 14.9, 21 (all handed over 31.4), 2e-8 2.23, 2.05, 2.04.
+    const int few = a.pass1_iters > 0 ? INT_MAX : a.g.n < (1 << 16) ? 8192 : 4096;
     if (interp == 2) {
       POND_LAUNCH(2);
       const unsigned nw = (unsigned)(a.g.n < 1024 ? a.g.n : 1024);

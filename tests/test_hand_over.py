@@ -97,3 +97,41 @@ def test_split_as_written(gpu, interp, learned):
     niter = same_for_every_hand_over((17, 6, 3), interp, "split", jump_state((17, 6, 3), 0.05), 2 if learned else 1,
                                      (None, 1, 3, 8), learned)
     assert (niter > 8).any()
+
+
+def many_slow(shape, T0):
+    """density jumps 16 cells apart: a quarter of the cells go past 8 iterations"""
+    f = list(smooth_random_state(shape, seed=3, T0=T0))
+    x = np.arange(f[0].size) % shape[0]
+    f[0] = np.where(x % 16 < 8, 3.0 * f[0], f[0])
+    return f
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,tol,least", [((64, 48, 48), None, 8192), ((40, 40, 30), 0.0, 32768)])
+def test_split_more_cells_than_go_at_once(gpu, shape, tol, least):
+    """late cells beyond those that go at once, in waves with and without cells left to start"""
+    niter = same_for_every_hand_over(shape, "weno5c", "split", many_slow(shape, 0.2), 1, (100000, 8, None),
+                                     split_tol_rel=tol, split_tol_abs=tol)
+    assert (niter > 8).sum() > least
+
+
+def step_ms(shape, precision, f, pass1_iters, **kw):
+    with Pond("D3Q27", shape, "weno5c", precision, pass1_iters=pass1_iters, **kw) as p:
+        ms = []
+        for _ in range(3):
+            p.set_state(*f)
+            p.step(1)
+            p.sync()
+            ms.append(p.timing()["last_ms"])
+        print(f"[cap] {precision} {shape} first {pass1_iters}: {min(ms):.2f} ms", flush=True)
+        return min(ms)
+
+
+@pytest.mark.gpu
+def test_split_cells_that_all_go_to_the_cap_keep_their_waves(gpu):
+    """the workgroup kernel takes several times as long for a cell's iteration as full waves"""
+    shape = (80, 80, 80)
+    f = smooth_random_state(shape, seed=3, T0=0.02)
+    tol0 = dict(split_tol_rel=0.0, split_tol_abs=0.0)
+    assert step_ms(shape, "split", f, None, **tol0) < 2 * step_ms(shape, "split", f, 100000, **tol0)
