@@ -17,6 +17,7 @@
 // cell, 64 consecutive cells (x fastest) per wave.  D3Q125 mapping: one 128-lane block per cell, lane =
 // target population (as the reference's 125-thread block), the nodes of the fixed 3x3x3 neighbourhood
 // through scalar loads.
+#include <climits>
 #include <type_traits>
 #include "pond_device.h"
 
@@ -1098,10 +1099,14 @@ __device__ __forceinline__ void f64_group(const SRC& src, int x, int y, int z, i
   }
 }
 
+// A WENO5 cell late in its iterations goes to k_step_f64_27_wide where its wave has no cell left to start and
+// no more than this many slots (of 7) with such cells; see launch_step_f64.
+constexpr int kWideSlots64 = 5;
+
 template <int INTERP, bool BUF>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_step_f64_27(
     const NodeSrc gsrc, double* __restrict__ fout, double* __restrict__ mout, int* __restrict__ niter_out,
-    int* __restrict__ slow, const StepArgs a, int cells, int wide_after) {
+    int* __restrict__ slow, const StepArgs a, int cells, int wide_after, int few) {
   constexpr bool WENO = INTERP != 1 && INTERP != 3;
   using Src = typename std::conditional<BUF, NodeBuf, NodeSrc>::type;
   Src src;
@@ -1199,7 +1204,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
 #pragma unroll
       for (int k = 0; k < 4; k++) c0[k] = mn[k];
       const bool done = bad == 0 || niter >= a.max_iter;
-      if (done || (WENO && niter >= wide_after)) {
+      int e = -1;  // the cell's place in the list of k_step_f64_27_wide
+      if (WENO && !done && niter >= wide_after) {
+        const bool idle = next >= total && __popcll(__ballot(true) & kHeads) <= kWideSlots64;  // (late cells only)
+        if (gi == 0) e = slow_place(slow, idle, few);
+        e = __shfl(e, head, 64);
+      }
+      if (done || e >= 0) {
         // BGK towards rho*w_i (steps.cu:557-564), two populations per lane and store; a cell left to
         // k_step_f64_27_wide stores its iterate as it is
         active = false;
@@ -1221,7 +1232,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
         }
         if (gi < 5) mout[gi * P + cell] = gi == 0 ? rho : gi == 1 ? m0 : gi == 2 ? m1 : gi == 3 ? m2 : m3;
         if (gi == 5) niter_out[cell] = niter;
-        if (WENO && !done && gi == 6) slow[kSlowList + atomicAdd(slow, 1)] = (int)cell;
+        if (WENO && !done && gi == 6) slow[kSlowList + e] = (int)cell;
       }
     }
     wave_lds_order();
@@ -1865,14 +1876,21 @@ hipError_t launch_step_f64(int lattice, int interp, const double* fin, const dou
     const dim3 nb((unsigned)((slots + cells - 1) / cells));
 #define POND_LAUNCH(I)                                                                                           \
   do {                                                                                                           \
-    if (buf) hipLaunchKernelGGL((k_step_f64_27<I, true>), nb, nt, 0, st, src, fout, mout, niter, pend.count, a, (int)cells, wide_after);   \
-    else hipLaunchKernelGGL((k_step_f64_27<I, false>), nb, nt, 0, st, src, fout, mout, niter, pend.count, a, (int)cells, wide_after);      \
+    if (buf) hipLaunchKernelGGL((k_step_f64_27<I, true>), nb, nt, 0, st, src, fout, mout, niter, pend.count, a, (int)cells, wide_after, few);   \
+    else hipLaunchKernelGGL((k_step_f64_27<I, false>), nb, nt, 0, st, src, fout, mout, niter, pend.count, a, (int)cells, wide_after, few);      \
   } while (0)
     // The iteration after which a WENO5 cell goes to k_step_f64_27_wide, early where the grid leaves the
     // chip idle.  ms per step for 5, 6, 8, 12, 16 and never: 33x18x14 vortex 0.64, 0.65, 0.75, 0.84, -,
     // 0.81; shock-bubble 32^3 -, 4.24, 4.10, 4.16, 4.20, 10.4; 64^3 -, 19.5, 17.6, 16.9, 16.9, 20.5;
     // 100^3 -, 55.6, 53.2, 52.1, 52.1, 54.4; 128^3 -, -, 105, 99.7, 99.5, 99.1.
     const int wide_after = a.pass1_iters > 0 ? a.pass1_iters : a.g.n < (1 << 14) ? 6 : a.g.n < (1 << 17) ? 8 : 16;
+    // From then on a cell goes when its wave stands idle for it: with no cell left to start and at most
+    // kWideSlots64 slots still at such cells.  The workgroups of the chip do 28 iterations per us, the waves
+    // with all slots in use 145, so a wave whose cells are all late keeps them; the first 2048 of a step go at
+    // once, as a small grid leaves the chip idle anyway.  Tolerance 0 (every cell to the cap), ms per step with every late cell
+    // handed over and now: 16^3 18.0, 15.2, 32^3 119, 34, 64^3 877, 185 (with 1024: 11.4, 31, 180, but the
+    // 12^3 shock-bubble 1.15 -> 1.29); T = 0.2 with density jumps 16 cells apart 64^3 79.9, 78.3, 96^3 263, 254.
+    const int few = a.pass1_iters > 0 ? INT_MAX : 2048;
     const dim3 nw((unsigned)(a.g.n < 1024 ? a.g.n : 1024)), ntw(kWideThreads64);
 #define POND_WIDE(V) hipLaunchKernelGGL(k_step_f64_27_wide<V>, nw, ntw, 0, st, src, fout, mout, niter, pend.count, a)
     if (code == 1) {

@@ -135,3 +135,19 @@ def test_split_cells_that_all_go_to_the_cap_keep_their_waves(gpu):
     f = smooth_random_state(shape, seed=3, T0=0.02)
     tol0 = dict(split_tol_rel=0.0, split_tol_abs=0.0)
     assert step_ms(shape, "split", f, None, **tol0) < 2 * step_ms(shape, "split", f, 100000, **tol0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,tol,least", [((32, 24, 20), None, 3000), ((12, 20, 14), 0.0, 3000)])
+def test_fp64_more_cells_than_go_at_once(gpu, shape, tol, least):
+    niter = same_for_every_hand_over(shape, "weno5c", "fp64", many_slow(shape, 0.2), 1, (100000, 8, None),
+                                     tol_rel=tol, tol_abs=tol)
+    assert (niter > 8).sum() > least
+
+
+@pytest.mark.gpu
+def test_fp64_cells_that_all_go_to_the_cap_keep_their_waves(gpu):
+    shape = (40, 40, 40)
+    f = smooth_random_state(shape, seed=3, T0=0.02)
+    tol0 = dict(tol_rel=0.0, tol_abs=0.0)
+    assert step_ms(shape, "fp64", f, None, **tol0) < 2 * step_ms(shape, "fp64", f, 100000, **tol0)
