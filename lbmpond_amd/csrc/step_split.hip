@@ -2074,7 +2074,7 @@ hipError_t launch_step_split(int lattice, int interp, const SplitPtrs& in, const
   // MLUPS: the second, with one lane per cell too, runs alone after the first and a few slowly
   // converging cells make a tail).
   SplitArgs b = a;
-  if (b.pass1_iters < 0) b.pass1_iters = 1 << 30;
+  b.pass1_iters = a.pass1_iters < 0 ? 1 << 30 : a.pass1_iters < 255 ? a.pass1_iters : 255;  // (8 bits in the list)
   // second-pass grid: enough waves to fill the chip several times, never more than the cells
   const int64_t w2 = (a.g.n + 63) / 64;
   const unsigned blocks2 = (unsigned)(w2 < 16384 ? w2 : 16384);

@@ -151,3 +151,11 @@ def test_fp64_cells_that_all_go_to_the_cap_keep_their_waves(gpu):
     f = smooth_random_state(shape, seed=3, T0=0.02)
     tol0 = dict(tol_rel=0.0, tol_abs=0.0)
     assert step_ms(shape, "fp64", f, None, **tol0) < 2 * step_ms(shape, "fp64", f, 100000, **tol0)
+
+
+@pytest.mark.gpu
+def test_split_as_written_after_hundreds_of_iterations(gpu):
+    """the second kernel of the WENO5 as written takes a cell's count over whatever the first pass's length"""
+    niter = same_for_every_hand_over((6, 4, 3), "weno5", "split", jump_state((6, 4, 3), 0.05), 1, (None, 200, 255, 300),
+                                     max_iter=400, split_tol_rel=0.0, split_tol_abs=0.0)
+    assert (niter == 400).any()
