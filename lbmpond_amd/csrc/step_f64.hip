@@ -17,7 +17,6 @@
 // cell, 64 consecutive cells (x fastest) per wave.  D3Q125 mapping: one 128-lane block per cell, lane =
 // target population (as the reference's 125-thread block), the nodes of the fixed 3x3x3 neighbourhood
 // through scalar loads.
-#include <climits>
 #include <type_traits>
 #include "pond_device.h"
 
@@ -1890,7 +1889,7 @@ hipError_t launch_step_f64(int lattice, int interp, const double* fin, const dou
     // once, as a small grid leaves the chip idle anyway.  Tolerance 0 (every cell to the cap), ms per step with every late cell
     // handed over and now: 16^3 18.0, 15.2, 32^3 119, 34, 64^3 877, 185 (with 1024: 11.4, 31, 180, but the
     // 12^3 shock-bubble 1.15 -> 1.29); T = 0.2 with density jumps 16 cells apart 64^3 79.9, 78.3, 96^3 263, 254.
-    const int few = a.pass1_iters > 0 ? INT_MAX : 2048;
+    constexpr int few = 2048;
     const dim3 nw((unsigned)(a.g.n < 1024 ? a.g.n : 1024)), ntw(kWideThreads64);
 #define POND_WIDE(V) hipLaunchKernelGGL(k_step_f64_27_wide<V>, nw, ntw, 0, st, src, fout, mout, niter, pend.count, a)
     if (code == 1) {

@@ -22,7 +22,6 @@
 // fixed-point iteration has the last word: a prediction that is not finite or not positive in T
 // is ignored, and if the residual stops falling before the noise floor, or the cell has not
 // converged after kLearnedBudget iterations, it restarts from its previous gauge.
-#include <climits>
 #include "pond_device.h"
 #include "step_split.h"
 
@@ -2069,7 +2068,7 @@ hipError_t launch_step_split(int lattice, int interp, const SplitPtrs& in, const
     // of the cells past 16 iterations): 64^3 53, 15, 128^3 320, 85; T = 0.2 with density jumps 16 cells apart:
     // 64^3 17.9, 16.7, 128^3 102, 99, 200^3 443, 503 (one lane per cell: 951).  32^3 with few = 4096, 8192 and
     // 16384: tolerance 0 9.7, 14.9, 21 (all handed over 31.4), 2e-8 2.23, 2.05, 2.04.
-    const int few = a.pass1_iters > 0 ? INT_MAX : a.g.n < (1 << 16) ? 8192 : 4096;
+    const int few = a.g.n < (1 << 16) ? 8192 : 4096;
     if (interp == 2) {
       POND_LAUNCH(2);
       const unsigned nw = (unsigned)(a.g.n < 1024 ? a.g.n : 1024);

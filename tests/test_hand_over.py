@@ -33,6 +33,20 @@ for k in (1, 3, 50):
     assert out.split() == ["1", "3", "50"]
 
 
+@pytest.mark.parametrize("precision,kernel,arg", [("split", "k_step_split27_cells", 13), ("fp64", "k_step_f64_27ILi", 8)])
+def test_given_hand_over_keeps_the_bound_on_the_list(stub, precision, kernel, arg):
+    """the number of cells that go at once, whatever their wave does, with pass1_iters given and not"""
+    out = hip_stub.run(stub, f"""
+stub.stub_watch({kernel!r}.encode(), {arg})
+for k in (3, None):
+    with Pond("D3Q27", (64, 64, 32), "weno5c", {precision!r}, pass1_iters=k) as p:
+        p.set_state(*[np.ones(p.n)] * 5)
+        p.step(1)
+    print(*last({kernel!r})[0])
+""").split()
+    assert out[0] == out[1] and 0 < int(out[0]) < 64 * 64 * 32
+
+
 def jump_state(shape, T0, bad=False):
     f = list(smooth_random_state(shape, seed=3, T0=T0))
     x = np.arange(f[0].size) % shape[0]
