@@ -1833,8 +1833,10 @@ hipError_t launch_node_prep(int lattice, const double* m, double* P, int64_t n, 
 // The line kernel does 3-4 times the work per cell and iteration of the one-lane kernel (lanes of a
 // target repeat its tail), and pays where the chip is not full or the iteration counts are uneven.
 // WENO5: every line (2^20 cells, the longest: 5.3 -> 1.0 ms on the Sod tube, 3.6 -> 2.9 ms on a
-// smooth wave with 3.65 iterations everywhere).  Lagrange-4 on that wave: 32768 cells 0.120 -> 0.090
-// ms, 131072 cells 0.24 -> 0.35 ms.
+// smooth wave with 3.65 iterations everywhere).  Lagrange-4, one lane per cell and here, on a smooth wave
+// with 3 iterations everywhere and on the Sod tube: 32768 cells 0.099 -> 0.070 and 0.26 -> 0.044 ms, 49152
+// 0.101 -> 0.101 and 0.27 -> 0.057, 65536 0.102 -> 0.131 and 0.26 -> 0.069; the wave with mirror walls 65536
+// 1.61 -> 0.135.  The limit gives the wave's third away for the tube's factor of four.
 bool f64_line_step(int lattice, int interp, const Grid& g) {
   return lattice == kD1Q5 && g.ny == 1 && g.nz == 1 && (interp != 1 || g.n <= kLineCellsLagr4);
 }
