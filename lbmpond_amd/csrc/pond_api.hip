@@ -398,6 +398,7 @@ pond_status pond_create(const pond_params* p, pond_ctx** out) {
   if (hipGetDevice(&ctx->device) != hipSuccess || hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess)
     return bail(POND_ERR_HIP, "pond_create: hipStreamCreate failed");
   ctx->split = p->precision == POND_SPLIT;
+  const bool line = f64_line_step(p->lattice, p->interp, g);
   if (!ctx->split) {
     const size_t fbytes = (size_t)f64_fcount(p->lattice, ctx->Qn, g.plane) * sizeof(double);
     const size_t mbytes = (size_t)5 * g.plane * sizeof(double);
@@ -406,10 +407,11 @@ pond_status pond_create(const pond_params* p, pond_ctx** out) {
         return bail(POND_ERR_NOMEM, "pond_create: hipMalloc of the state buffers failed");
       ctx->bytes += (int64_t)(fbytes + mbytes);
     }
-    // D3Q27: 32-byte gauge records (ux, uy, uz, P); otherwise one P plane
-    if (hipMalloc(&ctx->nodeP, (size_t)(p->lattice == POND_D3Q27 ? 4 : 1) * g.plane * sizeof(double)) != hipSuccess)
+    // D3Q27: 32-byte gauge records (ux, uy, uz, P); D1Q5 off a line: one P plane
+    const size_t pbytes = (size_t)g.plane * (p->lattice == POND_D3Q27 ? 32 : p->lattice == POND_D1Q5 && !line ? 8 : 0);
+    if (pbytes && hipMalloc(&ctx->nodeP, pbytes) != hipSuccess)
       return bail(POND_ERR_NOMEM, "pond_create: hipMalloc of the node planes failed");
-    ctx->bytes += (int64_t)g.plane * (p->lattice == POND_D3Q27 ? 32 : 8);
+    ctx->bytes += (int64_t)pbytes;
   } else {
     const size_t fbytes = (size_t)split_fcount(p->lattice, ctx->Qn, g.plane) * sizeof(float);
     const size_t mbytes = (size_t)4 * g.plane * sizeof(float);
@@ -420,9 +422,11 @@ pond_status pond_create(const pond_params* p, pond_ctx** out) {
         return bail(POND_ERR_NOMEM, "pond_create: hipMalloc of the split state buffers failed");
       ctx->bytes += (int64_t)(fbytes + mbytes + tbytes);
     }
-    if (hipMalloc(&ctx->sq, (size_t)g.plane * 4 * sizeof(float)) != hipSuccess)
-      return bail(POND_ERR_NOMEM, "pond_create: hipMalloc of the node gauge records failed");
-    ctx->bytes += (int64_t)g.plane * 4 * sizeof(float);
+    if (p->lattice == POND_D3Q27) {
+      if (hipMalloc(&ctx->sq, (size_t)g.plane * 4 * sizeof(float)) != hipSuccess)
+        return bail(POND_ERR_NOMEM, "pond_create: hipMalloc of the node gauge records failed");
+      ctx->bytes += (int64_t)g.plane * 4 * sizeof(float);
+    }
     if (p->use_mlp) {
       if (hipMalloc(&ctx->guess, (size_t)4 * g.plane * sizeof(float)) != hipSuccess)
         return bail(POND_ERR_NOMEM, "pond_create: hipMalloc of the predicted-gauge planes failed");
@@ -446,8 +450,12 @@ pond_status pond_create(const pond_params* p, pond_ctx** out) {
   }
   if (hipMalloc(&ctx->niter, (size_t)g.plane * sizeof(int)) != hipSuccess)
     return bail(POND_ERR_NOMEM, "pond_create: hipMalloc of niter failed");
-  ctx->pend_cap = g.plane;
-  const size_t pend_bytes = 256 + (size_t)g.plane * (4 + 4 * 8 + 8 + 4);
+  // The header with the count; behind it the two-pass steps' entries or the slow cells of the D3Q27
+  // steps that have a workgroup kernel for them (the other steps leave no cell to a second kernel).
+  const bool slow_list = p->lattice == POND_D3Q27 && (ctx->split ? p->interp == POND_WENO5C : p->interp != POND_LAGR4);
+  const bool two_pass = p->lattice == POND_D1Q5 ? !line : p->lattice == POND_D3Q27 && p->interp != POND_LAGR4 && !slow_list;
+  ctx->pend_cap = two_pass ? g.plane : 0;
+  const size_t pend_bytes = (size_t)kSlowList * sizeof(int) + (size_t)g.plane * (two_pass ? 4 + 4 * 8 + 8 + 4 : slow_list ? 4 : 0);
   if (hipMalloc(&ctx->pend, pend_bytes) != hipSuccess)
     return bail(POND_ERR_NOMEM, "pond_create: hipMalloc of the pending-cell list failed");
   ctx->bytes += (int64_t)pend_bytes;
@@ -692,7 +700,7 @@ static SplitPending pending_view(pond_ctx* ctx) {
   char* b = ctx->pend;
   SplitPending v;
   v.count = (int*)b;
-  v.g = (double*)(b + 256);
+  v.g = (double*)(b + kSlowList * sizeof(int));
   v.res = v.g + 4 * cap;
   v.cell = (int*)(v.res + cap);
   v.meta = v.cell + cap;

@@ -83,12 +83,13 @@ struct pond_ctx {
   pond::F64Buf f64[2];
   pond::SplitBuf sp[2];
   pond::SplitArgs sargs{};
-  double* nodeP = nullptr;  // plain path: per cell of the load buffer, D3Q27 the record (ux, uy, uz, P),
-                            // else P, with P = sqrt(|T|)*sign(T)
-  float* sq = nullptr;      // split path: node gauge records (ux, uy, uz, sqrt(|T|)*sign(T)) of the load buffer
+  double* nodeP = nullptr;  // plain path: per cell of the load buffer, D3Q27 the record (ux, uy, uz, P), D1Q5
+                            // off a line P, with P = sqrt(|T|)*sign(T)
+  float* sq = nullptr;      // split D3Q27: node gauge records (ux, uy, uz, sqrt(|T|)*sign(T)) of the load buffer
   float* guess = nullptr;   // split path: learned starting gauge increments (4 planes)
-  // cells left unconverged by a step's first kernel: count, then the D3Q27 WENO5 steps' list of cells,
-  // or per entry of a two-pass step the cell index, 4 gauge doubles, one double and one int (48 B per cell of the grid)
+  // cells left unconverged by a step's first kernel: the count, then the D3Q27 WENO5 steps' list of cells (4 B
+  // per cell of the grid), or per entry of a two-pass step the cell index, 4 gauge doubles, one double
+  // and one int (48 B per cell)
   char* pend = nullptr;
   int64_t pend_cap = 0;
   int* niter = nullptr;     // per-cell gauge iterations of the last step
