@@ -326,17 +326,15 @@ __device__ __forceinline__ double transfer5(const SRC& s, uint32_t boff, const T
 }
 
 // ---------------------------------------------------------------------------------------------
-// Lattice traits for the one-lane-per-cell kernel
+// Lattice traits: the transfer to one target (interp_weno5, interp_lagr4), and for D1Q5 what the
+// one-lane-per-cell kernel needs besides
 
 template <int LAT>
 struct Lat;
 
 template <>
 struct Lat<kD3Q27> {
-  static constexpr int Q = 27;
   using Tgt = Tgt27;
-  __device__ static double efc(int i, int d) { return (double)kE27[i][d]; }
-  __device__ static Tgt tgt(int i, const double* g) { return make_tgt27e(kE27[i][0], kE27[i][1], kE27[i][2], g[0], g[1], g[2], g[3]); }
   template <class SRC>
   __device__ static double xfer(const SRC& s, uint32_t boff, const Tgt& t, double sqTb) {
     return transfer27(s, boff, t, sqTb);
@@ -993,13 +991,12 @@ __device__ __forceinline__ bool f64_start(const NodeSrc& gsrc, int64_t cell, con
 }
 
 // BGK towards rho*w_i in the converged gauge (steps.cu:557-564) and the cell's outputs
-template <int Q>
 __device__ __forceinline__ void f64_finish(double* __restrict__ fout, double* __restrict__ mout,
                                            int* __restrict__ niter_out, int64_t cell, const F64Iter& st,
                                            const StepArgs& a) {
   const int64_t P = a.g.plane;
-  for (int i = 0; i < Q; i++) {
-    const int64_t o = f64_fidx(Q == 27 ? kD3Q27 : kD1Q5, i, cell, P);
+  for (int i = 0; i < 5; i++) {
+    const int64_t o = f64_fidx(kD1Q5, i, cell, P);
     double f = fout[o];
     const double feq = st.rho0 * a.w[i];
     f += a.dtau * (feq - f);
@@ -1037,7 +1034,7 @@ __global__ __launch_bounds__(64) void k_step_f64(const NodeSrc gsrc, double* __r
     const int stop = a.pass1_iters < a.max_iter ? a.pass1_iters : a.max_iter;
     const bool conv = f64_iterate<LAT, INTERP>(src, gsrc, fout, cell, x, y, z, zero, st, stop, a);
     pending = !conv && st.niter < a.max_iter;
-    if (!pending) f64_finish<Lat<LAT>::Q>(fout, mout, niter_out, cell, st, a);
+    if (!pending) f64_finish(fout, mout, niter_out, cell, st, a);
   }
   bool any;
   const int64_t e = pending_slot(pend, pending, any);
@@ -1401,7 +1398,7 @@ __global__ __launch_bounds__(64) void k_step_f64_rest(const NodeSrc gsrc, double
     st.niter = pend.meta[e];
     // the zero-cell start only matters for the first iteration, which the first pass ran
     f64_iterate<LAT, INTERP>(src, gsrc, fout, cell, x, y, z, false, st, a.max_iter, a);
-    f64_finish<Lat<LAT>::Q>(fout, mout, niter_out, cell, st, a);
+    f64_finish(fout, mout, niter_out, cell, st, a);
   }
 }
 

@@ -599,8 +599,7 @@ __device__ __forceinline__ void node_group(const NodePass& p, int ey, float sq1,
 // contracts over y with its own basis and adds to its three targets as interp_group_weno5c
 // does.  The three sub-stencil sums of each target are accumulated slice by slice (a slice's
 // y/z sum enters every sub-stencil whose window holds it), so only the five smoothness samples
-// of a window are kept.  Each target's value is stored to fout (its population slot of this
-// cell).  Windows or rows far apart (absurd gauges) fall back to
+// of a window are kept.  The values go to o[3 (ey+1) + ex+1] (LDS).  Windows or rows far apart (absurd gauges) fall back to
 // interp_group_weno5c per group, which bounds the loops whatever the gauge.
 __device__ __forceinline__ void interp_pass_weno5c(const NodeSrcF& src, int x, int y, int z, double s,
                                                    const double gc[4], int ez, float sqTb, float* o) {
@@ -845,7 +844,7 @@ constexpr int kLearnedBudget = 12;
 // value with its tensor Lagrange weight.  The per-axis basis factors w (1/(2T1) or -1/T1) are
 // applied to the finished sums.  MIR: mirror boundaries on the axes of g.mirror (a node beyond
 // a mirrored face is the mirror image of the cell inside).  Windows or rows far apart (absurd
-// gauges) fall back to interp_lagr4f per target.  Each target's value is stored to fout.
+// gauges) fall back to interp_lagr4f per target.  The values go to o[3 (ey+1) + ex+1] (LDS).
 template <bool MIR>
 __device__ __forceinline__ void interp_pass_lagr4(const NodeSrcF& src, int x, int y, int z, double s,
                                                   const double gc[4], int ez, float sqTb, float* o) {
