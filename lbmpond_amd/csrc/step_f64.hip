@@ -613,7 +613,7 @@ __device__ __forceinline__ Tgt27 tgt27_of(const Tgt27g3& t, int k) {
 // weighting of the one before (57 ms: the other wave of the SIMD covers the wait already); each
 // different node of a wave's cells loaded once, 16 bytes per lane, and handed out through LDS (112
 // ms when the walk took 65: the loaders' addresses go to scratch, and a scratch access occupies the
-// L1 for as long as a 16-byte load); held to three waves per SIMD (91 ms, scratch again).
+// L1 for as long as a 16-byte load); held to three waves per SIMD (91 ms, scratch in the walk itself).
 template <int NR, bool MIR, class SRC, class FS, class FR, class FN>
 __device__ __forceinline__ void walk27(const SRC& src, int x, int ry, int rz, int dlo, int dhi, FS&& slice, FR&& row,
                                        FN&& node) {
@@ -1059,8 +1059,11 @@ __global__ __launch_bounds__(64) void k_step_f64(const NodeSrc gsrc, double* __r
 // same sequence of operations (bit for bit).
 // Per step, before and after: 33x18x14 vortex 10.0 -> 0.85 ms; 128^3 vortex 86 -> 56 ms; 256x128x128
 // shock-bubble 289 -> 181 ms; Lagrange-4 128^3 255 -> 124 ms, 100x52x46 with walls 109 -> 15.8 ms.
-// Bound by FP64 issue: at 128^3 the VALU is busy 75 % of the time (texture-address unit 54 %), with 330
-// instructions per node where no contraction and every rounding of the reference leave about 290.
+// Bound by FP64 issue where the flow is smooth: 128^3 vortex VALU busy 75 % (texture-address unit 53 %), 332
+// instructions per node where no contraction and every rounding of the reference leave about 290.  On the 384^3
+// shock-bubble 59 and 62 %, with 53 lanes in use: neither is full, and two waves per SIMD do not hide the loads.
+// The kernel spills 113 registers (364 bytes per lane; WENO5 as written 128 and 424, Lagrange-4 69 and 280),
+// all of them outside the loop over the nodes: 13 GB written per step at 128^3 against 0.56 GB of output, 192 GB at 384^3.
 template <int INTERP, class SRC>
 __device__ __forceinline__ void f64_group(const SRC& src, int x, int y, int z, int ey, int ez, const double (&uT)[4],
                                           double s, const StepArgs& a, double (&fn)[3]) {
@@ -1414,7 +1417,7 @@ __global__ __launch_bounds__(64) void k_step_f64_rest(const NodeSrc gsrc, double
 //     multiplications read directly (from LDS, 125 broadcast reads per node and wave took as long as
 //     the arithmetic).  A node beyond a mirror wall (MIR) is read permuted, through LDS;
 //   * lane q of a wave sums moment q % 5 over the populations in order (every lane used to sum all five).
-// 40^3 turbulence 20.1 -> 12.4 ms per step, 64^3 82 -> 51 ms; the VALU is busy 94 % of the time, 83 % of
+// 40^3 turbulence 20.1 -> 12.4 ms per step, 64^3 82 -> 51 ms; the VALU is busy 93 % of the time, 80 % of
 // its instructions being the terms.
 template <bool MIR>
 __global__ __launch_bounds__(128) void k_step_q125_f64(const double* __restrict__ fin, const double* __restrict__ min,

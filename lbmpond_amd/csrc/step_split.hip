@@ -1313,8 +1313,8 @@ constexpr int kWideSlots = 5;
 // next cell of the wave's run when its own has converged.  Each cell's arithmetic and its order are the
 // same (bit for bit).  Per step, before and after: 256^3 vortex 65.3 -> 39.6 ms, 256^3 shock-bubble
 // 107 -> 69.7 ms, 32^3 shock-bubble 16.9 -> 5.6 ms; Lagrange-4 192^3 Taylor-Green 81 -> 37.5 ms,
-// 150x101x94 22.0 -> 8.1 ms.  Bound by VALU issue: 256^3 vortex busy 85 % (57 of 64 lanes; texture-address
-// unit 71 %), 150x101x94 86 % (45 lanes: windows and rows that differ between the cells of a wave).
+// 150x101x94 22.0 -> 8.1 ms.  Bound by VALU issue: 256^3 vortex busy 86 % (57 of 64 lanes; texture-address
+// unit 73 %), 150x101x94 90 % (44 lanes: windows and rows that differ between the cells of a wave).
 // Two waves per SIMD (256 registers): with more registers the load latency would be left unhidden.
 template <int INTERP>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_step_split27_cells(
@@ -1632,8 +1632,8 @@ __global__ __launch_bounds__(kWideThreads) void k_step_split27_wide(
 // the 27 nodes with the interpolation weights of their target.  With a lane per target instead
 // (128 lanes per cell, the contractions through LDS, two barriers per node) the step was bound by
 // its 30 LDS reads for every 15 FMAs: 96^3 turbulence 26.0 -> 7.7 ms per step, 160^3 122 -> 36 ms.
-// Bound now by VALU issue (72 % of the cycles, 3350 instructions per iteration of a wave, 1875 of
-// them the contractions); the texture-address unit is 46 % busy.
+// Bound now by VALU issue (75 % of the cycles, 3400 instructions per iteration of a wave, 1875 of
+// them the contractions); the texture-address unit is 50 % busy.
 //
 // A wave owns `chunk` consecutive cells; a half whose cell is done takes the next one, so cells
 // that need more iterations hold up nobody but themselves.
